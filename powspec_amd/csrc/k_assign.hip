@@ -36,7 +36,7 @@ static_assert(sizeof(Rec) == 24, "record layout");
 
 using DevPart = PshDevPart;
 
-__device__ __forceinline__ int window_width(int scheme) { return scheme + 1; }
+constexpr int kFewParts = 8;   // part tables passed as kernel arguments
 
 // Periodic wrap into [0, Ng).  Bases and window ends are at most a window
 // (or a grid) away from [0, Ng), so one compare settles nearly every call;
@@ -47,89 +47,85 @@ __device__ __forceinline__ int wrap(int c, int Ng) {
   return r < 0 ? r + Ng : r;
 }
 
+// a / L correctly rounded, rL being 1 / L rounded: one Newton step brings
+// a rL within an ulp, and the step after that rounds correctly (Markstein's
+// theorem on quotients from a correctly rounded reciprocal).  Five FP64
+// operations where the compiler's division takes about a dozen, several of
+// them at a quarter of the rate.  Finite a and L away from overflow, as grid
+// coordinates are; an infinite a gives NaN, and such a particle fails the box
+// check (boxes) or leaves no valid box (surveys).
+__host__ __device__ __forceinline__ double div_rn(double a, double L, double rL) {
+  double q = a * rL;
+  q = __builtin_fma(__builtin_fma(-q, L, a), rL, q);
+  return __builtin_fma(__builtin_fma(-q, L, a), rL, q);
+}
+
 // Base cell (leftmost window cell, unwrapped) and window fraction of a grid
 // coordinate x >= 0, following src/genr_mesh.c:57-66 (NGP), 94-104 (CIC),
 // 152-172 (TSC), 256-263 (PCS).  The fraction is d = x - (int)x for CIC/PCS
 // and the signed offset from the middle node for TSC.
-__device__ __forceinline__ void axis_base(double x, int scheme, int &b,
-                                          double &f) {
-  int x0 = (int)x;
-  double d = x - x0;
-  switch (scheme) {
-    case 0:
-      b = (d >= 0.5) ? x0 + 1 : x0;
-      f = 0;
-      break;
-    case 1:
-      b = x0;
-      f = d;
-      break;
-    case 2:
-      if (d < 0.5) {
-        b = x0 - 1;
-        f = d;
-      } else {
-        b = x0;
-        f = d - 1;
-      }
-      break;
-    default:
-      b = x0 - 1;
-      f = d;
-      break;
+template <int SCHEME>
+__device__ __forceinline__ void axis_base(double x, int &b, double &d) {
+  const int x0 = (int)x;
+  d = x - x0;
+  if (SCHEME == 0) {
+    b = (d >= 0.5) ? x0 + 1 : x0;
+  } else if (SCHEME == 1) {
+    b = x0;
+  } else if (SCHEME == 2) {
+    b = (d < 0.5) ? x0 - 1 : x0;
+    if (!(d < 0.5)) d -= 1;
+  } else {
+    b = x0 - 1;
   }
 }
 
-// Per-particle plain/shifted bases.  The shifted grid uses the reference's
-// periodic shift (src/genr_mesh.c:595-600: x >= smin + L -> x - L) before
-// the coordinate (x - smin) * Ng / L.
-struct PartCells {
-  int b[3];        // plain-grid base, wrapped into [0, Ng)
-  int delta[3];    // shifted base - plain base (mod Ng), 0 or 1
-  float f[3];
-  bool ok;
-};
+// Cells of a particle along one axis: plain-grid base wrapped into [0, Ng),
+// window fraction, and the shifted grid's base minus the plain one (mod Ng),
+// 0 or 1.  The shifted grid uses the reference's periodic shift
+// (src/genr_mesh.c:595-600: x >= smin + L -> x - L) before the coordinate
+// (x - smin) * Ng / L, which is the plain one plus 1/2 up to rounding: the
+// offset follows from the plain fraction unless that lies within kShiftEps
+// of a value where the offset changes; then (and where g.shift_exact says
+// that the box corner's rounding may exceed kShiftEps cells) the shifted
+// coordinate is formed as the reference forms it.
+constexpr float kShiftEps = 1e-6f;
 
-__device__ PartCells part_cells(const double *r, const PshAssignGeom &g) {
+template <int SCHEME, bool IL>
+__device__ __forceinline__ void axis_cells(double r, const PshAssignGeom &g, int a, int &b,
+                                           float &f, int &delta) {
 #pragma clang fp contract(off)
-  PartCells pc;
-  pc.ok = true;
   const double Ngd = (double)g.Ng;
-  for (int a = 0; a < 3; a++) {
-    double x = (r[a] - g.bmin[a]) * Ngd / g.L[a];
-    int b;
-    double f;
-    axis_base(x, g.scheme, b, f);
-    pc.b[a] = wrap(b, g.Ng);
-    pc.f[a] = (float)f;
-    pc.delta[a] = 0;
-    if (g.intlace) {
-      double p = r[a];
+  int bu;
+  double d;
+  axis_base<SCHEME>(div_rn((r - g.bmin[a]) * Ngd, g.L[a], g.rL[a]), bu, d);
+  b = wrap(bu, g.Ng);
+  const float ff = (float)d;
+  f = SCHEME == 0 ? 0.f : ff;
+  delta = 0;
+  if (IL) {
+    // NGP: 1 below the half cell; CIC, PCS: 1 from the half cell on; TSC
+    // (signed fraction): 1 for the fractions below the half cell, d >= 0
+    bool sure;
+    if (SCHEME == 0) {
+      delta = ff < 0.5f;
+      sure = fabsf(ff - 0.5f) > kShiftEps && ff > kShiftEps && ff < 1.f - kShiftEps;
+    } else if (SCHEME == 2) {
+      delta = ff >= 0.f;
+      sure = fabsf(ff) > kShiftEps && fabsf(ff) < 0.5f - kShiftEps;
+    } else {
+      delta = ff >= 0.5f;
+      sure = fabsf(ff - 0.5f) > kShiftEps;
+    }
+    if (g.shift_exact || !sure) {
+      double p = r;
       if (p >= g.smin[a] + g.L[a]) p -= g.L[a];
-      double xs = (p - g.smin[a]) * Ngd / g.L[a];
       int bs;
-      double fs;
-      axis_base(xs, g.scheme, bs, fs);
-      int dlt = wrap(bs - b, g.Ng);
-      if (dlt > 1) pc.ok = false;
-      pc.delta[a] = dlt;
+      double ds;
+      axis_base<SCHEME>(div_rn((p - g.smin[a]) * Ngd, g.L[a], g.rL[a]), bs, ds);
+      delta = wrap(bs - bu, g.Ng);
     }
   }
-  return pc;
-}
-
-// Tiles touched along one axis by the union window [b, b + W - 1 + delta]
-// (b in [0, Ng), tiles of 2^TS cells).
-__device__ __forceinline__ int axis_tiles(int b, int W, int delta, int Ng,
-                                          int TS, int t[2]) {
-  int e = b + W - 1 + delta;
-  t[0] = b >> TS;
-  int te = wrap(e, Ng) >> TS;
-  if (te != t[0]) {
-    t[1] = te;
-    return 2;
-  }
-  return 1;
 }
 
 __device__ __forceinline__ int find_part(const DevPart *parts, int nparts,
@@ -212,61 +208,80 @@ __device__ __forceinline__ Loaded load_particle(const DevPart *parts, int nparts
   return L;
 }
 
-// Tiles (mock-local indices) touched by a particle rr = (x, y, z, w) and,
-// with FILL, its record.  Returns the number of tiles (0 and flag bit 2 when the
-// shifted grid's base is inconsistent).  With CHECK and g.check_box, a
-// coordinate outside [bmin, bmin + L) (bmin = 0 for simulation boxes) sets
-// flag bit 4: the box check of
-// simulation catalogues (src/genr_mesh.c:517-533) folded into the count
-// pass, which reads every particle anyway (NaN passes, as it passes the
-// reference's min/max comparisons).
-template <bool FILL, bool CHECK = false>
-__device__ __forceinline__ int particle_tiles(const PshAssignGeom &g, const double *rr,
-                                              float wscale, int W, uint32_t *tiles, Rec &rec,
-                                              int *flags) {
+// The tiles a particle's windows meet: the tile of its plain base, and per
+// axis the offset of the tile of the union window's last cell (0: the same
+// tile).  A window plus the shifted grid's cell meets at most two tiles per
+// axis, so combination k (bit 0: z, 1: y, 2: x) is a tile of its own when
+// its axes all have a second tile.
+struct PartTiles {
+  int t0;
+  int off[3];   // x, y, z
+  __device__ __forceinline__ bool has(int k) const {
+    return (!(k & 4) || off[0]) && (!(k & 2) || off[1]) && (!(k & 1) || off[2]);
+  }
+  __device__ __forceinline__ uint32_t tile(int k) const {
+    return (uint32_t)(t0 + ((k & 4) ? off[0] : 0) + ((k & 2) ? off[1] : 0) +
+                      ((k & 1) ? off[2] : 0));
+  }
+};
+
+// Tiles (mock-local indices) touched by a particle rr = (x, y, z, w) and its
+// record.  Returns false (and sets flag bit 2) when the shifted grid's base
+// is inconsistent.  With CHECK and g.check_box, a coordinate outside
+// [bmin, bmin + L) (bmin = 0 for simulation boxes) sets flag bit 4: the box
+// check of simulation catalogues (src/genr_mesh.c:517-533) folded into the
+// count pass, which reads every particle anyway (NaN passes, as it passes
+// the reference's min/max comparisons).
+template <int SCHEME, bool IL, bool CHECK>
+__device__ __forceinline__ bool particle_tiles(const PshAssignGeom &g, const double *rr,
+                                               float wscale, PartTiles &pt, Rec &rec,
+                                               int *flags) {
+  constexpr int W = SCHEME + 1;
   if (CHECK && g.check_box) {
     bool bad = false;
 #pragma unroll
     for (int a = 0; a < 3; a++) bad |= (rr[a] < g.bmin[a]) || (rr[a] >= g.bmin[a] + g.L[a]);
     if (bad) atomicOr(flags, 4);
   }
-  PartCells pc = part_cells(rr, g);
-  if (!pc.ok) {
+  int b[3], dl[3];
+#pragma unroll
+  for (int a = 0; a < 3; a++) axis_cells<SCHEME, IL>(rr[a], g, a, b[a], rec.f[a], dl[a]);
+  if (IL && (dl[0] | dl[1] | dl[2]) > 1) {
     atomicOr(flags, 2);
-    return 0;
+    return false;
   }
-  int tx[2], ty[2], tz[2];
-  int nx = axis_tiles(pc.b[0], W, pc.delta[0], g.Ng, g.tile_shift[0], tx);
-  int ny = axis_tiles(pc.b[1], W, pc.delta[1], g.Ng, g.tile_shift[1], ty);
-  int nz = axis_tiles(pc.b[2], W, pc.delta[2], g.Ng, g.tile_shift[2], tz);
-  int nt = 0;
-  for (int a = 0; a < nx; a++)
-    for (int b = 0; b < ny; b++)
-      for (int c = 0; c < nz; c++)
-        tiles[nt++] = ((uint32_t)tx[a] * g.ntile[1] + ty[b]) * g.ntile[2] + tz[c];
-  if (FILL) {
-    rec.f[0] = pc.f[0];
-    rec.f[1] = pc.f[1];
-    rec.f[2] = pc.f[2];
-    rec.w = (float)rr[3] * wscale;
-    rec.bxy = (uint32_t)pc.b[0] | ((uint32_t)pc.b[1] << 16);
-    rec.bz = (uint32_t)pc.b[2] |
-             ((uint32_t)(pc.delta[0] | (pc.delta[1] << 1) | (pc.delta[2] << 2)) << 16);
+  int t[3], o[3];
+#pragma unroll
+  for (int a = 0; a < 3; a++) {
+    t[a] = b[a] >> g.tile_shift[a];
+    o[a] = (wrap(b[a] + W - 1 + dl[a], g.Ng) >> g.tile_shift[a]) - t[a];
   }
-  return nt;
+  pt.t0 = (t[0] * g.ntile[1] + t[1]) * g.ntile[2] + t[2];
+  pt.off[0] = o[0] * g.ntile[1] * g.ntile[2];
+  pt.off[1] = o[1] * g.ntile[2];
+  pt.off[2] = o[2];
+  rec.w = (float)rr[3] * wscale;
+  rec.bxy = (uint32_t)b[0] | ((uint32_t)b[1] << 16);
+  rec.bz = (uint32_t)b[2] | ((uint32_t)(dl[0] | (dl[1] << 1) | (dl[2] << 2)) << 16);
+  return true;
 }
 
 // Largest |weight| of a launch, for the fixed-point scale of the deposit
-// (flags[1] holds the bits of a non-negative float).
+// (flags[1] holds the bits of a non-negative float).  The plain read skips
+// the atomic where the maximum is already known: one address takes every
+// wave's, and waves of equal weights would queue there.
 __device__ __forceinline__ void publish_wmax(float wmax, int *flags) {
   for (int o = 32; o > 0; o >>= 1) wmax = fmaxf(wmax, __shfl_xor(wmax, o));
-  if (__lane_id() == 0) atomicMax(reinterpret_cast<unsigned *>(flags) + 1, __float_as_uint(wmax));
+  unsigned *p = reinterpret_cast<unsigned *>(flags) + 1;
+  const unsigned w = __float_as_uint(wmax);
+  if (__lane_id() == 0 && w > __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+    atomicMax(p, w);
 }
 
-// Run-aggregated increment of LDS or global counters: lanes with `act` whose counter index `t`
+// Run-aggregated increment of global counters: lanes with `act` whose counter index `t`
 // equals the previous lane's form a run (space-ordered catalogues put
 // neighbouring particles into one tile, so a wave holds a few long runs);
-// the run's first lane adds the run length with one LDS atomic and every
+// the run's first lane adds the run length with one atomic and every
 // lane gets old + its rank in the run (RET), or nothing (count only).
 // Shuffled catalogues make every lane its own run: one atomic per lane, as
 // without aggregation.
@@ -294,196 +309,198 @@ __device__ __forceinline__ uint32_t run_increment(uint32_t *hist, uint32_t t, bo
   return base + (uint32_t)(lane - hl);
 }
 
-template <bool FILL>
-__global__ void __launch_bounds__(256)
-assign_bucket(PshAssignGeom g, const DevPart *__restrict__ parts, int nparts,
-              size_t ntotal, uint32_t *__restrict__ counts,
-              uint32_t *__restrict__ cursors, Rec *__restrict__ recs,
-              size_t rec_cap, int *__restrict__ flags) {
-  const int W = window_width(g.scheme);
-  const uint32_t tiles_per_mock = (uint32_t)g.ntile[0] * g.ntile[1] * g.ntile[2];
-  const size_t stride = (size_t)gridDim.x * blockDim.x;
-  // every lane of a wave runs the same number of iterations so that the
-  // wave-level aggregation below sees converged waves
-  const size_t iters = (ntotal + stride - 1) / stride;
-  const UPart P0 = uniform_part(parts, nparts, blockIdx.x * (size_t)blockDim.x);
-  size_t gi = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
-  float wmax = 0.f;
-  // software pipeline: the next particle's loads are in flight while the
-  // current one is processed
-  bool cur_live = gi < ntotal;
-  Loaded cur = load_particle(parts, nparts, P0, gi, cur_live);
-#pragma unroll 1
-  for (size_t it = 0; it < iters; it++, gi += stride) {
-    const size_t gn = gi + stride;
-    const bool nxt_live = it + 1 < iters && gn < ntotal;
-    const Loaded nxt = load_particle(parts, nparts, P0, gn, nxt_live);
-    uint32_t tiles[8];
-    int nt = 0;
-    Rec rec;
-    if (cur_live) {
-      nt = particle_tiles<FILL, !FILL>(g, cur.r, cur.wscale, W, tiles, rec, flags);
-      const uint32_t mbase = (uint32_t)cur.mock * tiles_per_mock;
-      for (int k = 0; k < nt; k++) tiles[k] += mbase;
-      if (FILL && nt) wmax = fmaxf(wmax, fabsf(rec.w));
-    }
-#pragma unroll
-    for (int k = 0; k < 8; k++) {
-      const bool act = k < nt;
-      if (!__ballot(act)) break;
-      const uint32_t t = act ? tiles[k] : 0u;
-      if (FILL) {
-        const uint32_t slot = run_increment<true>(cursors, t, act);
-        if (act) {
-          if (slot < rec_cap) recs[slot] = rec;
-          else atomicOr(flags, 1);
-        }
-      } else {
-        run_increment<false>(counts, t, act);
-      }
-    }
-    cur = nxt;
-    cur_live = nxt_live;
-  }
-  if (FILL) publish_wmax(wmax, flags);
-}
-
-// Bucketing with an LDS histogram of one mock's tiles (meshes of at most
-// kLdsTiles tiles per mock).  Workgroup b takes particles [b kChunk,
-// (b+1) kChunk) -- a split that depends on the total only, so captured
-// graphs stay valid for any mock sizes -- and histograms the (particle,
-// tile) pairs of the mock of its first particle in LDS; particles of another
-// mock (at a part boundary) use global atomics directly.
-//  count: the histogram is added to the global counters, one atomic per
-//         nonzero tile;
-//  fill:  one atomic per nonzero tile reserves the workgroup's range of each
-//         bucket, then a second sweep over the chunk (L2-resident) hands out
-//         slots with LDS atomics.
+// Bucketing.  Workgroup b takes particles [b chunk, (b+1) chunk) -- a split
+// that depends on the total only, so captured graphs stay valid for any mock
+// sizes -- and counts their (particle, tile) pairs in LDS, in a window of
+// the tiles of its first particle's mock: all of them up to kWinTiles, else
+// kWinTilesBig around the first particle's tile (a catalogue ordered by x
+// stays inside; the x tile index is the slowest).  Pairs outside the window
+// or of another mock are singles, counted and placed with global atomics.
+//  count: each nonzero window counter is added to the tile's count with one
+//         atomic, whose return value -- the place of the workgroup's range in
+//         the bucket -- goes to whist;
+//  scan:  starts = exclusive sums of counts + singles; the singles of a
+//         bucket follow the ranges of the workgroups (cursors);
+//  fill:  starts + whist is where the workgroup's range begins: slots are
+//         handed out with LDS atomics.
+// Without whist (no memory for it) every pair counts as a single in the
+// count pass, and the fill pass counts its chunk again to reserve ranges.
 // The deposit accumulates in integers, so the order of records within a
 // bucket does not matter.
-constexpr int kChunk = 16384;
-constexpr int kLdsTiles = 32768;
-constexpr int kLdsThreads = 1024;
+// Bound: the catalogue's bytes where its order keeps a tile's records
+// together, the 128-byte lines of isolated 24-byte records where it does not.
+// Measured on MI355X, count + fill: 2e7 space-ordered particles at N = 1024
+// (PCS, interlaced, 131072 tiles) 1.86 -> 0.73 ms with the cells from
+// multiplications and one coordinate per axis (the FP64 divisions and the
+// second coordinate were most of 450 instructions per particle) and the
+// window in place of a global atomic per run; 2e4 particles at N = 64
+// 75 -> 12 us and 1e6 at N = 256 86 -> 41 us with chunks that fill the chip.
+constexpr int kChunkMax = 16384;
+constexpr int kWinTiles = 32768;      // 128 KB of LDS, one workgroup per CU
+constexpr int kWinTilesBig = 16384;   // 64 KB, two
+constexpr int kBucketThreads = 1024;
 
-template <bool FILL>
-__global__ void __launch_bounds__(kLdsThreads, 8)   // 8 waves per SIMD: two workgroups per CU
-assign_bucket_lds(PshAssignGeom g, const DevPart *__restrict__ parts, int nparts,
-                  size_t ntotal, uint32_t *__restrict__ counts,
-                  uint32_t *__restrict__ cursors, Rec *__restrict__ recs, size_t rec_cap,
-                  int *__restrict__ flags, uint32_t *__restrict__ whist) {
+__host__ __device__ inline uint32_t window_tiles(uint32_t tpm) {
+  return tpm <= (uint32_t)kWinTiles ? tpm : (uint32_t)kWinTilesBig;
+}
+
+// Particles per workgroup: as many as leave two workgroups for each of the
+// 256 CUs, between 256 and kChunkMax, and at least half of the window
+// (whose clearing and flushing a chunk pays for).
+inline size_t bucket_chunk(const PshAssignGeom &g, size_t ntotal) {
+  if (g.lean) return kChunkMax;
+  const uint32_t win = window_tiles((uint32_t)g.ntile[0] * g.ntile[1] * g.ntile[2]);
+  size_t c = 256;
+  while (c < (size_t)kChunkMax && (2 * c * 512 <= ntotal || c * 2 < win)) c *= 2;
+  return c;
+}
+
+template <int SCHEME, bool IL, bool FILL>
+__global__ void __launch_bounds__(kBucketThreads, 8)   // 8 waves per SIMD: two workgroups per CU
+assign_bucket(PshAssignGeom g, const DevPart *__restrict__ parts, int nparts, size_t ntotal,
+              uint32_t chunk, uint32_t *__restrict__ counts, uint32_t *__restrict__ cursors,
+              const uint32_t *__restrict__ starts, Rec *__restrict__ recs, size_t rec_cap,
+              int *__restrict__ flags, uint32_t *__restrict__ whist) {
   extern __shared__ uint32_t hist[];
-  const int W = window_width(g.scheme);
   const uint32_t tpm = (uint32_t)g.ntile[0] * g.ntile[1] * g.ntile[2];
-  const size_t c0 = (size_t)blockIdx.x * kChunk;
-  const size_t c1 = min(ntotal, c0 + (size_t)kChunk);
+  const uint32_t win = window_tiles(tpm);
+  const uint32_t T = blockDim.x;
+  const size_t c0 = (size_t)blockIdx.x * chunk;
+  const size_t c1 = min(ntotal, c0 + (size_t)chunk);
   const UPart P0 = uniform_part(parts, nparts, c0);
   const int mock0 = P0.mock;
-  const uint32_t mbase0 = (uint32_t)mock0 * tpm;
-  uint32_t *wh = whist ? whist + (size_t)blockIdx.x * tpm : nullptr;
-  uint32_t tiles[8];
-  Rec rec;
-  if (FILL && wh) {
-    // the count pass left this workgroup's histogram in HBM: reserve the
-    // workgroup's range of each bucket without another pass over the chunk
-    for (uint32_t i = threadIdx.x; i < tpm; i += blockDim.x) {
-      const uint32_t v = wh[i];
-      hist[i] = v ? atomicAdd(&cursors[mbase0 + i], v) : 0u;
-    }
-    __syncthreads();
-  } else {
-    for (uint32_t i = threadIdx.x; i < tpm; i += blockDim.x) hist[i] = 0;
-    __syncthreads();
-    // every lane of a wave runs the same number of iterations (the chunk is a
-    // multiple of the workgroup size), so the run aggregation sees whole waves
-    static_assert(kChunk % kLdsThreads == 0, "chunk of whole workgroup sweeps");
-    // pass A: histogram of this mock's pairs (count: others go to global)
-    {
-      // software pipeline: the next particle's loads are in flight while the
-      // current one is processed
-      size_t gi = c0 + threadIdx.x;
-      bool cur_live = gi < c1;
-      Loaded cur = load_particle(parts, nparts, P0, gi, cur_live);
-#pragma unroll 1
-      for (int it = 0; it < kChunk / kLdsThreads; it++) {
-        const size_t gn = gi + kLdsThreads;
-        const bool nxt_live = it + 1 < kChunk / kLdsThreads && gn < c1;
-        const Loaded nxt = load_particle(parts, nparts, P0, gn, nxt_live);
-        int nt = 0;
-        int mock = mock0;
-        if (cur_live) {
-          nt = particle_tiles<false, !FILL>(g, cur.r, cur.wscale, W, tiles, rec, flags);
-          mock = cur.mock;
-        }
-#pragma unroll
-        for (int k = 0; k < 8; k++) {
-          const bool act = k < nt;
-          if (!__ballot(act)) break;
-          const bool here = act && mock == mock0;
-          run_increment<false>(hist, here ? tiles[k] : 0u, here);
-          if (!FILL && act && !here) atomicAdd(&counts[(uint32_t)mock * tpm + tiles[k]], 1u);
-        }
-        cur = nxt;
-        cur_live = nxt_live;
-        gi = gn;
-      }
-    }
-    __syncthreads();
-    if (!FILL) {
-      for (uint32_t i = threadIdx.x; i < tpm; i += blockDim.x) {
-        const uint32_t v = hist[i];
-        if (wh) wh[i] = v;
-        if (v) atomicAdd(&counts[mbase0 + i], v);
-      }
-      return;
-    }
-    for (uint32_t i = threadIdx.x; i < tpm; i += blockDim.x)
-      if (hist[i]) hist[i] = atomicAdd(&cursors[mbase0 + i], hist[i]);
-    __syncthreads();
-  }   // without a stored histogram
-  // pass B: records
-  float wmax = 0.f;
-  {
-    // software pipeline: the next particle's loads are in flight while the
-    // current one is processed
+  uint32_t wbase = 0;
+  if (win < tpm) {
+    // a quarter of the window below the first particle's tile
+    const Loaded L0 = load_particle(parts, nparts, P0, c0, true);
+    PartTiles pt;
+    Rec rec;
+    int ign = 0;
+    pt.t0 = 0;
+    particle_tiles<SCHEME, false, false>(g, L0.r, 0.f, pt, rec, &ign);
+    const uint32_t t = (uint32_t)__builtin_amdgcn_readfirstlane(pt.t0);
+    wbase = min(t > win / 4 ? t - win / 4 : 0u, tpm - win);
+  }
+  const uint32_t mbase0 = (uint32_t)mock0 * tpm + wbase;
+  uint32_t *wh = whist ? whist + (size_t)blockIdx.x * win : nullptr;
+  const int iters = (int)((chunk + T - 1) / T);
+
+  // one sweep over the chunk; the next particle's loads are in flight while
+  // the current one is processed, and every lane of a wave runs the same
+  // number of iterations (the run aggregation sees whole waves)
+  auto sweep = [&](auto check, auto use) {
     size_t gi = c0 + threadIdx.x;
     bool cur_live = gi < c1;
     Loaded cur = load_particle(parts, nparts, P0, gi, cur_live);
 #pragma unroll 1
-    for (int it = 0; it < kChunk / kLdsThreads; it++) {
-      const size_t gn = gi + kLdsThreads;
-      const bool nxt_live = it + 1 < kChunk / kLdsThreads && gn < c1;
+    for (int it = 0; it < iters; it++) {
+      const size_t gn = gi + T;
+      const bool nxt_live = it + 1 < iters && gn < c1;
       const Loaded nxt = load_particle(parts, nparts, P0, gn, nxt_live);
-      int nt = 0;
-      int mock = mock0;
-      if (cur_live) {
-        nt = particle_tiles<true>(g, cur.r, cur.wscale, W, tiles, rec, flags);
-        mock = cur.mock;
-        if (nt) wmax = fmaxf(wmax, fabsf(rec.w));
-      }
-#pragma unroll
-      for (int k = 0; k < 8; k++) {
-        const bool act = k < nt;
-        if (!__ballot(act)) break;
-        const bool here = act && mock == mock0;
-        uint32_t slot = run_increment<true>(hist, here ? tiles[k] : 0u, here);
-        if (act && !here) slot = atomicAdd(&cursors[(uint32_t)mock * tpm + tiles[k]], 1u);
-        if (act) {
-          if (slot < rec_cap) recs[slot] = rec;
-          else atomicOr(flags, 1);
-        }
-      }
+      PartTiles pt;
+      Rec rec;
+      bool live = cur_live;
+      pt.t0 = pt.off[0] = pt.off[1] = pt.off[2] = 0;
+      if (live)
+        live = particle_tiles<SCHEME, IL, decltype(check)::value>(g, cur.r, cur.wscale, pt, rec,
+                                                                  flags);
+      use(pt, rec, live, cur.mock);
       cur = nxt;
       cur_live = nxt_live;
       gi = gn;
     }
+  };
+  auto clear = [&]() {
+    for (uint32_t i = threadIdx.x; i < win; i += T) hist[i] = 0;
+    __syncthreads();
+  };
+  // counts the pairs inside the window; `single` takes the others (k-th
+  // tile of the lanes of a wave together)
+  auto count_pairs = [&](auto check, bool singles) {
+    sweep(check, [&](const PartTiles &pt, const Rec &, bool live, int mock) {
+      const bool mine = live && mock == mock0;
+      bool out = false;
+#pragma unroll
+      for (int k = 0; k < 8; k++) {
+        if (!live || !pt.has(k)) continue;
+        const uint32_t w = pt.tile(k) - wbase;
+        if (mine && w < win) atomicAdd(&hist[w], 1u);
+        else out = true;
+      }
+      if (!singles || !__ballot(out)) return;
+#pragma unroll
+      for (int k = 0; k < 8; k++) {
+        const bool act = out && pt.has(k) && !(mine && pt.tile(k) - wbase < win);
+        if (!__ballot(act)) continue;
+        run_increment<false>(cursors, act ? (uint32_t)mock * tpm + pt.tile(k) : 0u, act);
+      }
+    });
+    __syncthreads();
+  };
+
+  if (!FILL) {
+    clear();
+    count_pairs(std::true_type{}, true);
+    for (uint32_t i = threadIdx.x; i < win; i += T) {
+      const uint32_t v = hist[i];
+      if (wh) wh[i] = v ? atomicAdd(&counts[mbase0 + i], v) : 0u;
+      else if (v) atomicAdd(&cursors[mbase0 + i], v);
+    }
+    return;
   }
+  if (wh) {
+    for (uint32_t i = threadIdx.x; i < win; i += T) hist[i] = starts[mbase0 + i] + wh[i];
+  } else {
+    clear();
+    count_pairs(std::false_type{}, false);
+    for (uint32_t i = threadIdx.x; i < win; i += T)
+      if (hist[i]) hist[i] = atomicAdd(&cursors[mbase0 + i], hist[i]);
+  }
+  __syncthreads();
+  float wmax = 0.f;
+  sweep(std::false_type{}, [&](const PartTiles &pt, const Rec &rec, bool live, int mock) {
+    const bool mine = live && mock == mock0;
+    if (live) wmax = fmaxf(wmax, fabsf(rec.w));
+    uint32_t slot[8];
+    bool out = false;
+    // every slot is asked for before the first record is written
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+      slot[k] = 0xffffffffu;
+      if (!live || !pt.has(k)) continue;
+      const uint32_t w = pt.tile(k) - wbase;
+      if (mine && w < win) slot[k] = atomicAdd(&hist[w], 1u);
+      else out = true;
+    }
+    if (__ballot(out)) {
+#pragma unroll
+      for (int k = 0; k < 8; k++) {
+        const bool act = out && pt.has(k) && !(mine && pt.tile(k) - wbase < win);
+        if (!__ballot(act)) continue;
+        const uint32_t q =
+            run_increment<true>(cursors, act ? (uint32_t)mock * tpm + pt.tile(k) : 0u, act);
+        if (act) slot[k] = q;
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+      if (!live || !pt.has(k)) continue;
+      if (slot[k] < rec_cap) recs[slot[k]] = rec;
+      else atomicOr(flags, 1);
+    }
+  });
   publish_wmax(wmax, flags);
 }
 
-// ---- exclusive scan of uint32 counters (3 kernels) -------------------------
+// ---- exclusive scan of uint32 counters -------------------------------------
+// One workgroup up to kScanOne counters (a launch costs more than the scan),
+// else three kernels.  TWO: the counters are in[i] + cursors[i], and cursors
+// becomes out[i] + in[i].
 constexpr int kScanThreads = 256;
 constexpr int kScanItems = 16;
 constexpr int kScanBlock = kScanThreads * kScanItems;
+constexpr int kScanOneThreads = 1024;
+constexpr size_t kScanOne = 32768;
 
 __device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t v,
                                                          uint32_t *sh,
@@ -512,16 +529,80 @@ __device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t v,
   return res;
 }
 
+template <bool TWO>
+__global__ void __launch_bounds__(kScanOneThreads)
+scan_one(const uint32_t *__restrict__ in, uint32_t *__restrict__ out,
+         uint32_t *__restrict__ cursors, int n) {
+  __shared__ uint32_t sh[17];
+  uint32_t carry = 0;
+  // a thread takes 16 consecutive counters with 16-byte accesses (word by
+  // word, a wave's accesses touch 64 lines each: 31 us for 16384 counters)
+  constexpr int K = 16;
+  for (int base = 0; base < n; base += K * kScanOneThreads) {
+    const int i0 = base + K * threadIdx.x;
+    const bool whole = i0 + K <= n;
+    uint32_t v[K], c[K], s = 0;
+#pragma unroll
+    for (int k = 0; k < K; k += 4) {
+      uint4 a = make_uint4(0u, 0u, 0u, 0u), b = a;
+      if (whole) {
+        a = *reinterpret_cast<const uint4 *>(in + i0 + k);
+        if (TWO) b = *reinterpret_cast<const uint4 *>(cursors + i0 + k);
+      }
+      v[k] = a.x, v[k + 1] = a.y, v[k + 2] = a.z, v[k + 3] = a.w;
+      c[k] = b.x, c[k + 1] = b.y, c[k + 2] = b.z, c[k + 3] = b.w;
+    }
+    if (!whole) {
+#pragma unroll
+      for (int k = 0; k < K; k++) {
+        if (i0 + k >= n) break;
+        v[k] = in[i0 + k];
+        if (TWO) c[k] = cursors[i0 + k];
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < K; k++) s += v[k] + c[k];
+    uint32_t tot;
+    uint32_t ex = block_exclusive_scan(s, sh, tot) + carry;
+#pragma unroll
+    for (int k = 0; k < K; k++) {   // c: the exclusive sum; v: c + v
+      const uint32_t t = v[k] + c[k];
+      v[k] += ex;
+      c[k] = ex;
+      ex += t;
+    }
+#pragma unroll
+    for (int k = 0; k < K; k += 4) {
+      if (whole) {
+        *reinterpret_cast<uint4 *>(out + i0 + k) = make_uint4(c[k], c[k + 1], c[k + 2], c[k + 3]);
+        if (TWO)
+          *reinterpret_cast<uint4 *>(cursors + i0 + k) =
+              make_uint4(v[k], v[k + 1], v[k + 2], v[k + 3]);
+      } else {
+#pragma unroll
+        for (int q = k; q < k + 4; q++) {
+          if (i0 + q >= n) break;
+          out[i0 + q] = c[q];
+          if (TWO) cursors[i0 + q] = v[q];
+        }
+      }
+    }
+    carry += tot;
+  }
+  if (threadIdx.x == 0) out[n] = carry;
+}
+
+template <bool TWO>
 __global__ void __launch_bounds__(kScanThreads)
-scan_local(const uint32_t *__restrict__ in, uint32_t *__restrict__ out,
-           uint32_t *__restrict__ bsum, size_t n) {
+scan_local(const uint32_t *__restrict__ in, const uint32_t *__restrict__ in2,
+           uint32_t *__restrict__ out, uint32_t *__restrict__ bsum, size_t n) {
   __shared__ uint32_t sh[17];
   size_t base = (size_t)blockIdx.x * kScanBlock + (size_t)threadIdx.x * kScanItems;
   uint32_t v[kScanItems];
   uint32_t s = 0;
 #pragma unroll
   for (int i = 0; i < kScanItems; i++) {
-    v[i] = (base + i < n) ? in[base + i] : 0u;
+    v[i] = (base + i < n) ? in[base + i] + (TWO ? in2[base + i] : 0u) : 0u;
     s += v[i];
   }
   uint32_t tot;
@@ -549,10 +630,10 @@ scan_sums(uint32_t *__restrict__ bsum, int nb) {
   if (threadIdx.x == 0) bsum[nb] = carry;
 }
 
-template <bool CURSORS>
+template <bool TWO>
 __global__ void __launch_bounds__(kScanThreads)
-scan_add(uint32_t *__restrict__ out, uint32_t *__restrict__ cursors,
-         const uint32_t *__restrict__ bsum, size_t n, int nb) {
+scan_add(const uint32_t *__restrict__ in, uint32_t *__restrict__ out,
+         uint32_t *__restrict__ cursors, const uint32_t *__restrict__ bsum, size_t n, int nb) {
   size_t base = (size_t)blockIdx.x * kScanBlock;
   uint32_t off = bsum[blockIdx.x];
   for (int i = threadIdx.x; i < kScanBlock; i += kScanThreads) {
@@ -560,16 +641,57 @@ scan_add(uint32_t *__restrict__ out, uint32_t *__restrict__ cursors,
     if (k < n) {
       uint32_t v = out[k] + off;
       out[k] = v;
-      if (CURSORS) cursors[k] = v;
+      if (TWO) cursors[k] = v + in[k];
     }
   }
   if (blockIdx.x == 0 && threadIdx.x == 0) out[n] = bsum[nb];
+}
+
+template <bool TWO>
+hipError_t launch_scan(const uint32_t *in, uint32_t *out, uint32_t *cursors, uint32_t *tmp,
+                       size_t n, hipStream_t s) {
+  const bool aligned = ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out) |
+                         reinterpret_cast<uintptr_t>(cursors)) & 15) == 0;
+  if (n <= kScanOne && aligned) {
+    hipLaunchKernelGGL((scan_one<TWO>), dim3(1), dim3(kScanOneThreads), 0, s, in, out, cursors,
+                       (int)n);
+  } else {
+    const int nsb = (int)((n + kScanBlock - 1) / kScanBlock);
+    hipLaunchKernelGGL((scan_local<TWO>), dim3(nsb), dim3(kScanThreads), 0, s, in, cursors, out,
+                       tmp, n);
+    hipLaunchKernelGGL(scan_sums, dim3(1), dim3(kScanThreads), 0, s, tmp, nsb);
+    hipLaunchKernelGGL((scan_add<TWO>), dim3(nsb), dim3(kScanThreads), 0, s, in, out, cursors,
+                       tmp, n, nsb);
+  }
+  return hipGetLastError();
 }
 
 __global__ void fill_zero_u32(uint32_t *p, size_t n) {
   for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n;
        i += (size_t)gridDim.x * blockDim.x)
     p[i] = 0u;
+}
+
+// Start of an assignment in one launch: the tile counters and the flags
+// cleared and, when they are few, the part table written from the arguments
+// (a copy from host memory costs the caller a staging copy and another
+// launch).
+struct FewParts {
+  int n;
+  DevPart p[kFewParts];
+};
+
+__global__ void __launch_bounds__(256)
+assign_begin(uint32_t *__restrict__ counts, uint32_t *__restrict__ cursors, size_t n,
+             int *__restrict__ flags, DevPart *__restrict__ parts, FewParts few) {
+  for (size_t i = blockIdx.x * (size_t)256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) {
+    counts[i] = 0u;
+    cursors[i] = 0u;
+  }
+  if (blockIdx.x == 0) {
+    if (threadIdx.x < 4) flags[threadIdx.x] = 0;
+    if ((int)threadIdx.x < few.n) parts[threadIdx.x] = few.p[threadIdx.x];
+  }
 }
 
 // ---- deposit: one workgroup per tile ------------------------------------------
@@ -1060,11 +1182,11 @@ bool psh_zfuse_tile(int Ng, int intlace, int tile[3]) {
 }
 
 size_t psh_assign_whist_words(const PshAssignGeom &g, size_t ntotal) {
-  const size_t tpm = (size_t)g.ntile[0] * g.ntile[1] * g.ntile[2];
-  if (tpm > (size_t)kLdsTiles || ntotal == 0) return 0;
-  const size_t blocks = (ntotal + kChunk - 1) / kChunk;
-  const size_t words = blocks * tpm;
-  return words <= ((size_t)1 << 30) ? words : 0;   // at most 4 GB of histograms
+  const uint32_t tpm = (uint32_t)g.ntile[0] * g.ntile[1] * g.ntile[2];
+  if (ntotal == 0 || (g.lean && tpm > (uint32_t)kWinTiles)) return 0;
+  const size_t chunk = bucket_chunk(g, ntotal);
+  const size_t words = (ntotal + chunk - 1) / chunk * window_tiles(tpm);
+  return words <= ((size_t)1 << 30) ? words : 0;   // at most 4 GB
 }
 
 hipError_t psh_fill_zero_u32(uint32_t *p, size_t n, hipStream_t s) {
@@ -1078,12 +1200,7 @@ hipError_t psh_fill_zero_u32(uint32_t *p, size_t n, hipStream_t s) {
 hipError_t psh_exclusive_scan_u32(const uint32_t *in, uint32_t *out, uint32_t *tmp, size_t n,
                                   hipStream_t s) {
   if (n == 0) return hipErrorInvalidValue;
-  const int nsb = (int)((n + kScanBlock - 1) / kScanBlock);
-  hipLaunchKernelGGL(scan_local, dim3(nsb), dim3(kScanThreads), 0, s, in, out, tmp, n);
-  hipLaunchKernelGGL(scan_sums, dim3(1), dim3(kScanThreads), 0, s, tmp, nsb);
-  hipLaunchKernelGGL(scan_add<false>, dim3(nsb), dim3(kScanThreads), 0, s, out,
-                     (uint32_t *)nullptr, tmp, n, nsb);
-  return hipGetLastError();
+  return launch_scan<false>(in, out, nullptr, tmp, n, s);
 }
 
 size_t psh_assign_scan_bytes(size_t ntiles) {
@@ -1091,60 +1208,72 @@ size_t psh_assign_scan_bytes(size_t ntiles) {
   return (nsb + 1) * sizeof(uint32_t);
 }
 
-hipError_t psh_assign_run(const PshAssignGeom &g, const PshDevPart *d_parts,
-                          int nparts, size_t ntotal, int nmock,
-                          uint32_t *counts, uint32_t *starts, uint32_t *cursors,
-                          void *records, size_t rec_cap, float *meshA,
-                          float *meshB, size_t mstride, uint32_t *d_scan_tmp,
-                          int *d_flags, hipStream_t s, hipEvent_t ev_deposit,
-                          uint32_t *whist) {
+namespace {
+template <int SCHEME, bool IL>
+hipError_t launch_bucket(bool fill, const PshAssignGeom &g, const PshDevPart *parts, int nparts,
+                         size_t ntotal, uint32_t *counts, uint32_t *cursors,
+                         const uint32_t *starts, Rec *recs, size_t rec_cap, int *flags,
+                         uint32_t *whist, hipStream_t s) {
+  const uint32_t tpm = (uint32_t)g.ntile[0] * g.ntile[1] * g.ntile[2];
+  const size_t lds = sizeof(uint32_t) * window_tiles(tpm);
+  const uint32_t chunk = (uint32_t)bucket_chunk(g, ntotal);
+  // two particles per thread at least, for the loads in flight
+  unsigned threads = kBucketThreads;
+  while (threads > 256 && threads * 2 > chunk) threads /= 2;
+  auto k = fill ? assign_bucket<SCHEME, IL, true> : assign_bucket<SCHEME, IL, false>;
+  if (lds > 64 * 1024)
+    (void)hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize,
+                              (int)lds);
+  hipLaunchKernelGGL(k, dim3((unsigned)((ntotal + chunk - 1) / chunk)), dim3(threads), lds, s, g,
+                     parts, nparts, ntotal, chunk, counts, cursors, starts, recs, rec_cap, flags,
+                     whist);
+  return hipGetLastError();
+}
+}  // namespace
+
+hipError_t psh_assign_run(const PshAssignGeom &g, PshDevPart *d_parts, const PshDevPart *h_parts,
+                          int nparts, size_t ntotal, int nmock, uint32_t *counts,
+                          uint32_t *starts, uint32_t *cursors, void *records, size_t rec_cap,
+                          float *meshA, float *meshB, size_t mstride, uint32_t *d_scan_tmp,
+                          int *d_flags, hipStream_t s, hipEvent_t ev_deposit, uint32_t *whist) {
   if (nparts < 1) return hipErrorInvalidValue;
   const size_t ntiles = (size_t)g.ntile[0] * g.ntile[1] * g.ntile[2] * nmock;
-  const int nsb = (int)((ntiles + kScanBlock - 1) / kScanBlock);
   hipError_t e;
-  if ((e = psh_fill_zero_u32(counts, ntiles, s)) != hipSuccess) return e;
-  unsigned pblocks = (unsigned)((ntotal + 255) / 256);
-  if (pblocks > 16384) pblocks = 16384;
-  if (pblocks == 0) pblocks = 1;
-  Rec *recs = reinterpret_cast<Rec *>(records);
-  const size_t tpm = (size_t)g.ntile[0] * g.ntile[1] * g.ntile[2];
-  const bool lds = tpm <= (size_t)kLdsTiles;
-  const unsigned cblocks = (unsigned)((ntotal + kChunk - 1) / kChunk);
-  const size_t lds_bytes = sizeof(uint32_t) * tpm;
-  if (lds && lds_bytes > 64 * 1024) {
-    (void)hipFuncSetAttribute((const void *)assign_bucket_lds<false>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);
-    (void)hipFuncSetAttribute((const void *)assign_bucket_lds<true>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);
+  FewParts few{};
+  if (h_parts && nparts <= kFewParts) {
+    few.n = nparts;
+    for (int i = 0; i < nparts; i++) few.p[i] = h_parts[i];
+  } else if (h_parts) {
+    if ((e = hipMemcpyAsync(d_parts, h_parts, sizeof(PshDevPart) * nparts,
+                            hipMemcpyHostToDevice, s)) != hipSuccess)
+      return e;
   }
-  if (ntotal > 0) {
-    if (lds)
-      hipLaunchKernelGGL((assign_bucket_lds<false>), dim3(cblocks), dim3(kLdsThreads),
-                         lds_bytes, s, g, d_parts, nparts, ntotal, counts, cursors, recs,
-                         rec_cap, d_flags, whist);
-    else
-      hipLaunchKernelGGL((assign_bucket<false>), dim3(pblocks), dim3(256), 0, s, g,
-                         d_parts, nparts, ntotal, counts, cursors, recs, rec_cap,
-                         d_flags);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-  }
-  hipLaunchKernelGGL(scan_local, dim3(nsb), dim3(kScanThreads), 0, s, counts,
-                     starts, d_scan_tmp, ntiles);
-  hipLaunchKernelGGL(scan_sums, dim3(1), dim3(kScanThreads), 0, s, d_scan_tmp, nsb);
-  hipLaunchKernelGGL(scan_add<true>, dim3(nsb), dim3(kScanThreads), 0, s, starts,
-                     cursors, d_scan_tmp, ntiles, nsb);
+  const size_t zb = (ntiles + 255) / 256;
+  hipLaunchKernelGGL(assign_begin, dim3((unsigned)(zb < 1024 ? zb : 1024)), dim3(256), 0, s,
+                     counts, cursors, ntiles, d_flags, d_parts, few);
   if ((e = hipGetLastError()) != hipSuccess) return e;
-  if (ntotal > 0) {
-    if (lds)
-      hipLaunchKernelGGL((assign_bucket_lds<true>), dim3(cblocks), dim3(kLdsThreads),
-                         lds_bytes, s, g, d_parts, nparts, ntotal, counts, cursors, recs,
-                         rec_cap, d_flags, whist);
-    else
-      hipLaunchKernelGGL((assign_bucket<true>), dim3(pblocks), dim3(256), 0, s, g,
-                         d_parts, nparts, ntotal, counts, cursors, recs, rec_cap,
-                         d_flags);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-  }
+  Rec *recs = reinterpret_cast<Rec *>(records);
+  auto bucket = [&](bool fill) -> hipError_t {
+    if (ntotal == 0) return hipSuccess;
+    auto go = [&](auto scheme) {
+      constexpr int S = decltype(scheme)::value;
+      return g.intlace ? launch_bucket<S, true>(fill, g, d_parts, nparts, ntotal, counts, cursors,
+                                                starts, recs, rec_cap, d_flags, whist, s)
+                       : launch_bucket<S, false>(fill, g, d_parts, nparts, ntotal, counts,
+                                                 cursors, starts, recs, rec_cap, d_flags, whist,
+                                                 s);
+    };
+    switch (g.scheme) {
+      case 0: return go(std::integral_constant<int, 0>{});
+      case 1: return go(std::integral_constant<int, 1>{});
+      case 2: return go(std::integral_constant<int, 2>{});
+      default: return go(std::integral_constant<int, 3>{});
+    }
+  };
+  if ((e = bucket(false)) != hipSuccess) return e;
+  if ((e = launch_scan<true>(counts, starts, cursors, d_scan_tmp, ntiles, s)) != hipSuccess)
+    return e;
+  if ((e = bucket(true)) != hipSuccess) return e;
   if (ev_deposit) (void)hipEventRecord(ev_deposit, s);
   switch (g.scheme) {
     case 0: return launch_deposit<0>(g, ntiles, starts, recs, rec_cap, meshA, meshB, mstride, d_flags, ntotal, s);

@@ -592,7 +592,15 @@ void set_assign_geom(psh_ctx *ctx) {
     g.bmin[a] = ctx->bmin[a];
     g.smin[a] = ctx->bmin[a] - 0.5 * ctx->L[a] / ctx->Ng;   // src/genr_mesh.c:817-818
     g.L[a] = ctx->L[a];
+    g.rL[a] = 1.0 / ctx->L[a];
   }
+  // a corner's rounding in cells, against the margin of 1e-6 cells that the
+  // bucketing allows the shifted coordinate
+  g.shift_exact = 0;
+  for (int a = 0; a < 3; a++)
+    if (!((fabs(ctx->bmin[a]) + ctx->L[a]) / ctx->L[a] * ctx->Ng < 1e-7 / DBL_EPSILON))
+      g.shift_exact = 1;
+  g.lean = ctx->arena != nullptr;
   // tiles of whole z rows in the fused shape: the deposit transforms its rows
   // (boxes; surveys keep the real mesh for their Y_lm-weighted passes)
   int zt[3];
@@ -836,11 +844,8 @@ int run_assign(psh_ctx *ctx, const std::vector<PshDevPart> &hp, int nmock,
   int rc;
   if ((rc = ensure_assign_scratch(ctx, nmock, (int)hp.size(), ntotal))) return rc;
   for (int attempt = 0; attempt < 4; attempt++) {
-    HIPCHK(ctx, hipMemcpyAsync(ctx->d_parts, hp.data(), sizeof(PshDevPart) * hp.size(),
-                               hipMemcpyHostToDevice, ctx->stream));
-    HIPCHK(ctx, psh_fill_zero_u32((uint32_t *)ctx->d_flags, 4, ctx->stream));
     ev_record(ctx, E_ASSIGN);
-    HIPCHK(ctx, psh_assign_run(ctx->ag, ctx->d_parts, (int)hp.size(), ntotal, nmock,
+    HIPCHK(ctx, psh_assign_run(ctx->ag, ctx->d_parts, hp.data(), (int)hp.size(), ntotal, nmock,
                                ctx->counts, ctx->starts, ctx->cursors, ctx->records,
                                ctx->rec_cap, meshA, meshB, ctx->mstride, ctx->scan_tmp,
                                ctx->d_flags, ctx->stream,
@@ -1868,13 +1873,13 @@ extern "C" int psh_ctx_run_batch(psh_ctx *ctx, const psh_data *d_data,
         HIPCHK(ctx, hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
         bool prof = ctx->profiling;
         ctx->profiling = false;
-        hipError_t e1 = psh_fill_zero_u32((uint32_t *)ctx->d_flags, 4, ctx->stream);
-        hipError_t e2 = psh_assign_run(ctx->ag, ctx->d_parts, nmock, ntotal, nmock, ctx->counts,
+        hipError_t e2 = psh_assign_run(ctx->ag, ctx->d_parts, nullptr, nmock, ntotal, nmock,
+                                       ctx->counts,
                                        ctx->starts, ctx->cursors, ctx->records, ctx->rec_cap,
                                        ctx->meshA, mB, ctx->mstride, ctx->scan_tmp,
                                        ctx->d_flags, ctx->stream, nullptr,
                                        ctx->whist_words ? ctx->whist : nullptr);
-        int rc2 = (e1 == hipSuccess && e2 == hipSuccess)
+        int rc2 = e2 == hipSuccess
                       ? run_sim_fft_bin(ctx, nmock, ctx->d_bins)
                       : PSH_ERR_DEVICE;
         ctx->profiling = prof;

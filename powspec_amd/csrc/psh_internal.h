@@ -80,6 +80,11 @@ struct PshAssignGeom {
   double bmin[3];       // box corner of the plain grid
   double smin[3];       // box corner of the shifted grid
   double L[3];          // box size
+  double rL[3];         // 1 / L, correctly rounded
+  // the corners' rounding may exceed the margin within which the shifted
+  // grid's cells follow from the plain grid's (a box far from the origin)
+  int shift_exact;
+  int lean;             // bucketing with the least scratch (static-scratch runs)
   // z transform fused into the deposit (tiles of whole z rows, boxes): the
   // deposit writes half-complex rows (k_z <= kzlim) instead of real ones
   int zfuse;
@@ -120,16 +125,18 @@ size_t psh_assign_scan_bytes(size_t ntiles);
 // (meshA) and shifted (meshB, interlacing only) meshes of nmock mocks; mock
 // m's meshes start at meshA + m*mstride, meshB + m*mstride.
 // counts, starts (ntiles+1), cursors: uint32 scratch; records: rec_cap
-// records; flags: bit 0 record overflow, bit 1 inconsistent shifted base.
-hipError_t psh_assign_run(const PshAssignGeom &g, const PshDevPart *d_parts,
-    int nparts, size_t ntotal, int nmock, uint32_t *counts, uint32_t *starts,
-    uint32_t *cursors, void *records, size_t rec_cap, float *meshA,
+// records; flags (4 words, cleared first): bit 0 record overflow, bit 1
+// inconsistent shifted base, bit 2 coordinate outside the box.  The part
+// table is written to d_parts from h_parts (nullptr: it is there already, as
+// a captured run needs it).
+hipError_t psh_assign_run(const PshAssignGeom &g, PshDevPart *d_parts,
+    const PshDevPart *h_parts, int nparts, size_t ntotal, int nmock,
+    uint32_t *counts, uint32_t *starts, uint32_t *cursors, void *records, size_t rec_cap, float *meshA,
     float *meshB, size_t mstride, uint32_t *d_scan_tmp, int *d_flags,
     hipStream_t s, hipEvent_t ev_deposit = nullptr, uint32_t *whist = nullptr);
 
-// uint32 words of the per-workgroup tile histograms that let the fill pass
-// skip its recount (0 when the LDS bucketing does not apply or they would
-// exceed 4 GB); whist passed to psh_assign_run must hold that many.
+// uint32 words of the per-workgroup bucket ranges that let the fill pass
+// skip its recount (0 when they would exceed 4 GB); whist passed to psh_assign_run must hold that many.
 size_t psh_assign_whist_words(const PshAssignGeom &g, size_t ntotal);
 
 // ---------------------------------------------------------------------------
