@@ -371,32 +371,39 @@ class DeviceArray:
 
 
 class _PkArrays:
+    """psh_pk and the arrays it points to, views of one buffer that only this
+    call's result refers to."""
+
     def __init__(self, nbin, nl):
-        self.k = np.zeros(nbin)
-        self.kedge = np.zeros(nbin + 1)
-        self.km = np.zeros(nbin)
-        self.cnt = np.zeros(nbin, np.uint64)
-        self.lcnt = np.zeros(nl * nbin)
-        self.pl = [np.zeros(nl * nbin), np.zeros(nl * nbin)]
-        self.xpl = np.zeros(nl * nbin)
+        nb, n = nbin, nl * nbin
+        buf = np.zeros(4 * nb + 1 + 4 * n)
+        base = buf.ctypes.data
         self.pk = Pk()
-        self.pk.k = self.k.ctypes.data
-        self.pk.kedge = self.kedge.ctypes.data
-        self.pk.km = self.km.ctypes.data
-        self.pk.cnt = self.cnt.ctypes.data
-        self.pk.lcnt = self.lcnt.ctypes.data
-        self.pk.pl[0] = self.pl[0].ctypes.data
-        self.pk.pl[1] = self.pl[1].ctypes.data
-        self.pk.xpl = self.xpl.ctypes.data
+        off = 0
+
+        def take(count):
+            nonlocal off
+            off += count
+            return buf[off - count:off], base + 8 * (off - count)
+
+        self.k, self.pk.k = take(nb)
+        self.kedge, self.pk.kedge = take(nb + 1)
+        self.km, self.pk.km = take(nb)
+        cnt, self.pk.cnt = take(nb)
+        self.cnt = cnt.view(np.uint64)
+        self.lcnt, self.pk.lcnt = take(n)
+        p0, self.pk.pl[0] = take(n)
+        p1, self.pk.pl[1] = take(n)
+        self.pl = [p0, p1]
+        self.xpl, self.pk.xpl = take(n)
         self.nbin, self.nl = nbin, nl
 
     def result(self):
         nb, nl = self.nbin, self.nl
-        return {"nbin": nb, "k": self.k.copy(), "kedge": self.kedge.copy(),
-                "km": self.km.copy(), "cnt": self.cnt.copy(),
-                "lcnt": self.lcnt.reshape(nl, nb).copy(),
-                "pl": [p.reshape(nl, nb).copy() for p in self.pl],
-                "xpl": self.xpl.reshape(nl, nb).copy()}
+        return {"nbin": nb, "k": self.k, "kedge": self.kedge, "km": self.km,
+                "cnt": self.cnt, "lcnt": self.lcnt.reshape(nl, nb),
+                "pl": [p.reshape(nl, nb) for p in self.pl],
+                "xpl": self.xpl.reshape(nl, nb)}
 
 
 class Context:
@@ -503,22 +510,19 @@ class Context:
 
     def run_survey_device(self, d_data: DeviceArray, nd: int, d_rand: DeviceArray, nr: int,
                           alpha: float, shot: float, norm: float):
-        nb = None
-        arr = None
         # the box (and so nbin) is known only after the bounds pass: size the
-        # output generously, then trim
+        # output generously, then keep the part that was written
         cap = 1 << 14
         arr = _PkArrays(cap, self.conf.npole)
         self._check(self.L.psh_ctx_run_survey_device(
             self.h, d_data.ptr, C.c_size_t(nd), d_rand.ptr, C.c_size_t(nr), C.c_double(alpha),
             C.c_double(shot), C.c_double(norm), C.byref(arr.pk)))
-        nb = self.nbin()
-        res = arr.result()
-        out = {"nbin": nb, "k": res["k"][:nb], "kedge": res["kedge"][:nb + 1],
-               "km": res["km"][:nb], "cnt": res["cnt"][:nb]}
-        flat = lambda a: a.ravel()[: self.conf.npole * nb].reshape(self.conf.npole, nb)
-        out["pl"] = [flat(p) for p in res["pl"]]
-        out["xpl"] = flat(res["xpl"])
+        nb, nl = self.nbin(), self.conf.npole
+        out = {"nbin": nb, "k": arr.k[:nb].copy(), "kedge": arr.kedge[:nb + 1].copy(),
+               "km": arr.km[:nb].copy(), "cnt": arr.cnt[:nb].copy()}
+        flat = lambda a: a[: nl * nb].reshape(nl, nb).copy()
+        out["pl"] = [flat(p) for p in arr.pl]
+        out["xpl"] = flat(arr.xpl)
         return out
 
     def run_batch(self, d_data: DeviceArray, offsets, weight_sums, graph=False):

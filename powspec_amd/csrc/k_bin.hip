@@ -181,7 +181,8 @@ constexpr int kRedAcc = 16, kRedSlices = 16;
 
 template <class T>
 __global__ void __launch_bounds__(kRedAcc * kRedSlices)
-reduce_kernel(const T *__restrict__ part, int grid, int nacc, T *__restrict__ out) {
+reduce_kernel(const T *__restrict__ part, int grid, int nacc, T *__restrict__ out,
+              T *__restrict__ hout, const int *__restrict__ flags, T *__restrict__ hflags) {
   __shared__ T sh[kRedSlices][kRedAcc];
   const int l = threadIdx.x % kRedAcc, slice = threadIdx.x / kRedAcc;
   const int a = blockIdx.x * kRedAcc + l;
@@ -200,15 +201,18 @@ reduce_kernel(const T *__restrict__ part, int grid, int nacc, T *__restrict__ ou
     T t = sh[0][l];
     for (int q = 1; q < kRedSlices; q++) t += sh[q][l];
     out[(size_t)m * nacc + a] = t;
+    if (hout) hout[(size_t)m * nacc + a] = t;
   }
+  if (hflags && blockIdx.x == 0 && m == 0 && threadIdx.x == 0) *hflags = (T)flags[0];
 }
 
 template <class T>
 hipError_t launch_reduce(const T *part, int nmock, int grid, int nacc, T *out,
-                         hipStream_t s) {
+                         hipStream_t s, T *hout = nullptr, const int *flags = nullptr,
+                         T *hflags = nullptr) {
   const dim3 blocks((unsigned)((nacc + kRedAcc - 1) / kRedAcc), (unsigned)nmock);
   hipLaunchKernelGGL(reduce_kernel<T>, blocks, dim3(kRedAcc * kRedSlices), 0, s, part,
-                     grid, nacc, out);
+                     grid, nacc, out, hout, flags, hflags);
   return hipGetLastError();
 }
 
@@ -311,8 +315,9 @@ hipError_t psh_geometry(int Ng, const PshAxisTables &ax, const PshBins &b,
 }
 
 hipError_t psh_reduce_partials(const double *partials, int nmock, int grid, int nacc,
-                               double *out, hipStream_t s) {
-  return launch_reduce<double>(partials, nmock, grid, nacc, out, s);
+                               double *out, hipStream_t s, double *hout, const int *flags,
+                               double *hflags) {
+  return launch_reduce<double>(partials, nmock, grid, nacc, out, s, hout, flags, hflags);
 }
 
 hipError_t psh_coord_bounds(const double *xyzw, size_t n, double *partial,

@@ -162,6 +162,11 @@ struct psh_ctx {
   double *d_bins = nullptr;
   size_t bins_cap = 0;
   double *d_bounds = nullptr;
+  // pinned host memory that the last kernels write their results to: the
+  // assignment's flags, then the bin sums (nullptr: not available, the
+  // results are copied from device memory)
+  double *h_res = nullptr;
+  size_t h_res_cap = 0;
 
   // device particle staging (host-catalogue runs)
   double *d_cat = nullptr;
@@ -772,6 +777,59 @@ int ensure_partials(psh_ctx *ctx, int nmock, int grid, int nacc, int slots) {
   return PSH_OK;
 }
 
+// Pinned host memory for `sums` results behind the assignment's flags
+// (h_res[0]).  Kernels that write their few results there spare the caller
+// the copies after them: each is a launch and, from pageable memory, a wait
+// of its own (measured: 2 waits and 2 copies, about 35 us per call).
+void ensure_results(psh_ctx *ctx, size_t sums) {
+  if (ctx->arena || sums + 1 <= ctx->h_res_cap) return;
+  drop_graph(ctx);   // a captured graph holds the old buffer
+  if (ctx->h_res) (void)hipHostFree(ctx->h_res);
+  ctx->h_res = nullptr;
+  ctx->h_res_cap = 0;
+  void *p = nullptr;
+  if (hipHostMalloc(&p, sizeof(double) * (sums + 1), hipHostMallocCoherent) != hipSuccess) {
+    (void)hipGetLastError();
+    return;
+  }
+  ctx->h_res = static_cast<double *>(p);
+  ctx->h_res_cap = sums + 1;
+}
+
+// The sums of n doubles written to h_res + 1 (or, without it, left at
+// d_sums) and the flags, once everything enqueued has run.
+int fetch_results(psh_ctx *ctx, const double *d_sums, size_t n, double *sums, int *flags) {
+  if (!ctx->h_res) {
+    HIPCHK(ctx, hipMemcpyAsync(sums, d_sums, sizeof(double) * n, hipMemcpyDeviceToHost,
+                               ctx->stream));
+    HIPCHK(ctx, hipMemcpyAsync(flags, ctx->d_flags, sizeof(int), hipMemcpyDeviceToHost,
+                               ctx->stream));
+  }
+  HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+  if (ctx->h_res) {
+    *flags = (int)ctx->h_res[0];
+    memcpy(sums, ctx->h_res + 1, sizeof(double) * n);
+  }
+  return PSH_OK;
+}
+
+// What a run's flags say: PSH_OK, an error, or kRerun after an overflow of
+// the record buffer (grown here) on any but the last of kAttempts runs.
+constexpr int kRerun = 1;
+constexpr int kAttempts = 4;
+
+int flags_error(psh_ctx *ctx, int flags, int attempt) {
+  if (flags & 4)
+    return set_err(ctx, PSH_ERR_CATA, "particle coordinate outside the box [0, BOX_SIZE)");
+  if (flags & 2)
+    return set_err(ctx, PSH_ERR_MESH, "inconsistent interlaced cell of a particle");
+  if (!(flags & 1)) return PSH_OK;
+  if (attempt + 1 == kAttempts)
+    return set_err(ctx, PSH_ERR_MESH, "assignment record buffer overflow");
+  const int rc = grow_records(ctx);
+  return rc ? rc : kRerun;
+}
+
 // Persistent workgroups per mock of the fused x pass: as many as the device
 // holds at once (CUs x per_cu, the kernel's workgroups per CU), shared among
 // the mocks, a multiple of 8 (one share per XCD), at most one per tile.
@@ -827,7 +885,8 @@ void ev_collect(psh_ctx *ctx) {
   ctx->ms[7] = ev_ms(ctx, E_ASSIGN, E_DEPOSIT);
 }
 
-// Assign parts (device table already built on host) into meshes.
+// Enqueue the assignment of parts into meshes; the run's results carry its
+// flags (flags_error).
 int run_assign(psh_ctx *ctx, const std::vector<PshDevPart> &hp, int nmock,
                float *meshA, float *meshB) {
   const Mark mark("psh:assign");
@@ -843,53 +902,48 @@ int run_assign(psh_ctx *ctx, const std::vector<PshDevPart> &hp, int nmock,
                    ctx->ag.tile[0], ctx->ag.tile[1], ctx->ag.tile[2]);
   int rc;
   if ((rc = ensure_assign_scratch(ctx, nmock, (int)hp.size(), ntotal))) return rc;
-  for (int attempt = 0; attempt < 4; attempt++) {
-    ev_record(ctx, E_ASSIGN);
-    HIPCHK(ctx, psh_assign_run(ctx->ag, ctx->d_parts, hp.data(), (int)hp.size(), ntotal, nmock,
-                               ctx->counts, ctx->starts, ctx->cursors, ctx->records,
-                               ctx->rec_cap, meshA, meshB, ctx->mstride, ctx->scan_tmp,
-                               ctx->d_flags, ctx->stream,
-                               ctx->profiling ? ctx->tm.ev[E_DEPOSIT] : nullptr,
-                               ctx->whist_words ? ctx->whist : nullptr));
-    ev_record(ctx, E_ASSIGNED);
-    int flags = 0;
-    HIPCHK(ctx, hipMemcpyAsync(&flags, ctx->d_flags, sizeof(int), hipMemcpyDeviceToHost,
-                               ctx->stream));
-    HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
-    if (flags & 4)
-      return set_err(ctx, PSH_ERR_CATA, "particle coordinate outside the box [0, BOX_SIZE)");
-    if (flags & 2)
-      return set_err(ctx, PSH_ERR_MESH, "inconsistent interlaced cell of a particle");
-    if (!(flags & 1)) return PSH_OK;
-    if ((rc = grow_records(ctx))) return rc;
-  }
-  return set_err(ctx, PSH_ERR_MESH, "assignment record buffer overflow");
+  ev_record(ctx, E_ASSIGN);
+  HIPCHK(ctx, psh_assign_run(ctx->ag, ctx->d_parts, hp.data(), (int)hp.size(), ntotal, nmock,
+                             ctx->counts, ctx->starts, ctx->cursors, ctx->records,
+                             ctx->rec_cap, meshA, meshB, ctx->mstride, ctx->scan_tmp,
+                             ctx->d_flags, ctx->stream,
+                             ctx->profiling ? ctx->tm.ev[E_DEPOSIT] : nullptr,
+                             ctx->whist_words ? ctx->whist : nullptr));
+  ev_record(ctx, E_ASSIGNED);
+  return PSH_OK;
+}
+
+// Forward z and y passes of the nmesh consecutive meshes from A on (real
+// fields `in`, which may be A itself).
+int fft_zy(psh_ctx *ctx, const float *in, float2 *A, int nmesh, const int *ylive, int kzlim) {
+  const PshYlmR noy{};
+  if (in)
+    HIPCHK(ctx, psh_fft_z_r2c(ctx->Ng, in, A, nmesh, ctx->mstride, ctx->tw, noy, ctx->stream,
+                              kzlim));
+  ev_record(ctx, E_ZDONE);
+  HIPCHK(ctx, psh_fft_y(ctx->Ng, A, nmesh, ctx->mstride, ctx->tw, 0, ctx->stream, ylive,
+                        ctx->ysched));
+  ev_record(ctx, E_YDONE);
+  return PSH_OK;
 }
 
 // FFTs of the plain (and shifted) meshes of nmock mocks, fused binning.
 int run_sim_fft_bin(psh_ctx *ctx, int nmock, double *out_bins /*[nmock][nacc]*/) {
   const Mark mark("psh:fft_bin");
   const int N = ctx->Ng;
-  PshYlmR noy{};
   float2 *A = reinterpret_cast<float2 *>(ctx->meshA);
   float2 *B = ctx->conf.intlace ? reinterpret_cast<float2 *>(ctx->meshB) : nullptr;
-  if (!ctx->ag.zfuse) {   // else the deposit wrote half-complex rows already
-    HIPCHK(ctx, psh_fft_z_r2c(N, ctx->meshA, A, nmock, ctx->mstride, ctx->tw, noy,
-                              ctx->stream, ctx->kzlim));
-    if (B)
-      HIPCHK(ctx, psh_fft_z_r2c(N, ctx->meshB, B, nmock, ctx->mstride, ctx->tw, noy,
-                                ctx->stream, ctx->kzlim));
-  }
-  ev_record(ctx, E_ZDONE);
-  HIPCHK(ctx, psh_fft_y(N, A, nmock, ctx->mstride, ctx->tw, 0, ctx->stream, ctx->d_ylive,
-                        ctx->ysched));
-  if (B)
-    HIPCHK(ctx, psh_fft_y(N, B, nmock, ctx->mstride, ctx->tw, 0, ctx->stream, ctx->d_ylive,
-                          ctx->ysched));
-  ev_record(ctx, E_YDONE);
+  int rc;
+  // with the fused deposit the meshes hold half-complex rows already; the
+  // shifted grid's meshes follow the plain ones when every mock is in use
+  const float *real = ctx->ag.zfuse ? nullptr : ctx->meshA;
+  const bool joined = B && nmock == ctx->nmock_max;
+  if ((rc = fft_zy(ctx, real, A, nmock * (joined ? 2 : 1), ctx->d_ylive, ctx->kzlim))) return rc;
+  if (B && !joined &&
+      (rc = fft_zy(ctx, real ? ctx->meshB : nullptr, B, nmock, ctx->d_ylive, ctx->kzlim)))
+    return rc;
   const int grid = xgrid_for(ctx, nmock, ctx->xres_sim);
   const int nacc = psh_xbin_nacc(ctx->bins, PSH_EPI_SIM);
-  int rc;
   if ((rc = ensure_partials(ctx, nmock, grid, nacc, 1))) return rc;
   PshXBinArgs a{};
   a.epi = PSH_EPI_SIM;
@@ -910,7 +964,9 @@ int run_sim_fft_bin(psh_ctx *ctx, int nmock, double *out_bins /*[nmock][nacc]*/)
     HIPCHK(ctx, psh_fft_x_bin(N, a, ctx->tw, ctx->stream));
   }
   ev_record(ctx, E_XDONE);
-  HIPCHK(ctx, psh_reduce_partials(ctx->partials, nmock, grid, nacc, out_bins, ctx->stream));
+  HIPCHK(ctx, psh_reduce_partials(ctx->partials, nmock, grid, nacc, out_bins, ctx->stream,
+                                  ctx->h_res ? ctx->h_res + 1 : nullptr, ctx->d_flags,
+                                  ctx->h_res));
   return PSH_OK;
 }
 
@@ -966,14 +1022,25 @@ int survey_slots(const psh_ctx *ctx) {
 // raw[0..nb) = sum |F0|^2 alias mult (src/multipole.c:579-660), then per pole
 // n >= 1 and m = -l..l: sum Re(F0 conj(Y_lm(k) S_lm)) with S_lm the transform
 // of Y_lm(r) times the field (src/mp_template.c:48-149).
-int survey_raw(psh_ctx *ctx, const std::vector<PshDevPart> &hp, std::vector<double> &raw,
-               double dc) {
+// One run; *flags receives the assignment's.
+int survey_run(psh_ctx *ctx, const std::vector<PshDevPart> &hp, std::vector<double> &raw,
+               double dc, int *flags) {
   const Mark mark("psh:survey");
   const int N = ctx->Ng;
   const bool il = ctx->conf.intlace;
   const int nb = ctx->nbin, nl = ctx->conf.npole;
   ev_record(ctx, E_START);
   int rc;
+  // the l = 0 and l > 0 passes each at their own grid, over one partials buffer
+  const int grid = xgrid_for(ctx, 1, ctx->xres_s0);
+  const int gridl = xgrid_for(ctx, 1, ctx->xres_sl);
+  const int nslots = survey_slots(ctx);
+  if ((rc = ensure_partials(ctx, 1, std::max(grid, gridl), nb, nslots))) return rc;
+  ensure_results(ctx, (size_t)nslots * nb);
+  // a group of (l, m) fields leaves its sums in the slot of its first m; the
+  // others stay zero
+  double *hsum = ctx->h_res ? ctx->h_res + 1 : nullptr;
+  if (hsum) memset(hsum, 0, sizeof(double) * (size_t)nslots * nb);
   // plain grid -> A when interlaced (combined into A), else -> B (real field
   // kept for the multipole weights) and transformed out of place into A
   float *plain = il ? ctx->meshA : ctx->meshB;
@@ -981,25 +1048,8 @@ int survey_raw(psh_ctx *ctx, const std::vector<PshDevPart> &hp, std::vector<doub
 
   float2 *A = reinterpret_cast<float2 *>(ctx->meshA);
   float2 *B = reinterpret_cast<float2 *>(ctx->meshB);
-  PshYlmR noy{};
-  if (il) {
-    HIPCHK(ctx, psh_fft_z_r2c(N, ctx->meshA, A, 1, ctx->mstride, ctx->tw, noy, ctx->stream));
-    HIPCHK(ctx, psh_fft_z_r2c(N, ctx->meshB, B, 1, ctx->mstride, ctx->tw, noy, ctx->stream));
-    HIPCHK(ctx, psh_fft_y(N, A, 1, ctx->mstride, ctx->tw, 0, ctx->stream, nullptr,
-                          ctx->ysched));
-    HIPCHK(ctx, psh_fft_y(N, B, 1, ctx->mstride, ctx->tw, 0, ctx->stream, nullptr,
-                          ctx->ysched));
-  } else {
-    HIPCHK(ctx, psh_fft_z_r2c(N, ctx->meshB, A, 1, ctx->mstride, ctx->tw, noy, ctx->stream));
-    HIPCHK(ctx, psh_fft_y(N, A, 1, ctx->mstride, ctx->tw, 0, ctx->stream, nullptr,
-                          ctx->ysched));
-  }
-  ev_record(ctx, E_YDONE);
-  // the l = 0 and l > 0 passes each at their own grid, over one partials buffer
-  const int grid = xgrid_for(ctx, 1, ctx->xres_s0);
-  const int gridl = xgrid_for(ctx, 1, ctx->xres_sl);
-  const int nslots = survey_slots(ctx);
-  if ((rc = ensure_partials(ctx, 1, std::max(grid, gridl), nb, nslots))) return rc;
+  // interlaced: A and B (adjacent) in place, else B out of place into A
+  if ((rc = fft_zy(ctx, plain, A, il ? 2 : 1, nullptr, 1 << 30))) return rc;
   PshXBinArgs a{};
   a.epi = PSH_EPI_SURVEY0;
   a.A = A;
@@ -1027,7 +1077,8 @@ int survey_raw(psh_ctx *ctx, const std::vector<PshDevPart> &hp, std::vector<doub
     HIPCHK(ctx, psh_fft_x_bin(N, w, ctx->tw, ctx->stream));
   }
   ev_record(ctx, E_XDONE);
-  HIPCHK(ctx, psh_reduce_partials(ctx->partials, 1, grid, nb, ctx->d_bins, ctx->stream));
+  HIPCHK(ctx, psh_reduce_partials(ctx->partials, 1, grid, nb, ctx->d_bins, ctx->stream, hsum,
+                                  ctx->d_flags, ctx->h_res));
   if (il) {
     // back to configuration space: B = c2r(F0) / Ntot (src/multipole.c:489-500)
     HIPCHK(ctx, psh_fft_x(N, A, B, 1, ctx->mstride, ctx->tw, 1, ctx->stream));
@@ -1056,9 +1107,9 @@ int survey_raw(psh_ctx *ctx, const std::vector<PshDevPart> &hp, std::vector<doub
   // transforms every field of the group and bins Re(F0 conj(sum_m Y_lm(k)
   // F_lm)) once.  A group's sums go to the slot of its first m; the other
   // slots of the pole stay zero (the host adds a pole's slots).
-  if (nslots > 1)
-    HIPCHK(ctx, hipMemsetAsync(ctx->d_bins + nb, 0, sizeof(double) * (size_t)(nslots - 1) * nb,
-                               ctx->stream));
+  if (nslots > 1 && !hsum)
+    HIPCHK(ctx, psh_fill_zero_u32(reinterpret_cast<uint32_t *>(ctx->d_bins + nb),
+                                  2 * (size_t)(nslots - 1) * nb, ctx->stream));
   int ngrp = 0;
   const size_t fstride_c = ctx->mstride / 2;
   for (int n = 1; n < nl; n++) {
@@ -1108,14 +1159,13 @@ int survey_raw(psh_ctx *ctx, const std::vector<PshDevPart> &hp, std::vector<doub
       lrec(3 * ngrp + 2);
       ngrp++;
       HIPCHK(ctx, psh_reduce_partials(ctx->partials, 1, gridl, nb,
-                                      ctx->d_bins + (size_t)gslot * nb, ctx->stream));
+                                      ctx->d_bins + (size_t)gslot * nb, ctx->stream,
+                                      hsum ? hsum + (size_t)gslot * nb : nullptr));
     }
   }
   ev_record(ctx, E_END);
   raw.assign((size_t)nslots * nb, 0.0);
-  HIPCHK(ctx, hipMemcpyAsync(raw.data(), ctx->d_bins, sizeof(double) * raw.size(),
-                             hipMemcpyDeviceToHost, ctx->stream));
-  HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+  if ((rc = fetch_results(ctx, ctx->d_bins, raw.size(), raw.data(), flags))) return rc;
   ev_collect(ctx);
   if (ctx->profiling) {
     // surveys: [5] the l > 0 fields' fused x passes, [6] their z and y passes
@@ -1137,6 +1187,17 @@ int survey_raw(psh_ctx *ctx, const std::vector<PshDevPart> &hp, std::vector<doub
     ctx->ms[6] = ok ? tzy : -1.0;
   }
   return PSH_OK;
+}
+
+int survey_raw(psh_ctx *ctx, const std::vector<PshDevPart> &hp, std::vector<double> &raw,
+               double dc) {
+  int rc = kRerun;
+  for (int attempt = 0; rc == kRerun; attempt++) {
+    int flags = 0;
+    if ((rc = survey_run(ctx, hp, raw, dc, &flags))) return rc;
+    rc = flags_error(ctx, flags, attempt);
+  }
+  return rc;
 }
 
 // Survey normalisation (src/multipole.c:1096-1153): l = 0 as (S/cnt - shot)
@@ -1178,32 +1239,45 @@ void normalise_survey(const psh_ctx *ctx, const double *raw, double shot, double
   }
 }
 
-// Coordinate bounds of n device records folded into mn/mx; *wsum (may be
-// NULL) receives the sum of their weights (block sums added in block order).
-int bounds_device(psh_ctx *ctx, const double *d, size_t n, double mn[3], double mx[3],
-                  double *wsum = nullptr) {
-  if (wsum) *wsum = 0.0;
-  if (n == 0) return PSH_OK;
-  int blocks = (int)((n + 255) / 256);
-  if (blocks > 1024) blocks = 1024;
+// Coordinate bounds of narr arrays of device records folded into mn/mx;
+// wsum[i] (wsum may be NULL) receives the sum of array i's weights (block
+// sums added in block order).  The arrays' launches are waited for together.
+int bounds_device(psh_ctx *ctx, const double *const *d, const size_t *n, int narr, double mn[3],
+                  double mx[3], double *wsum = nullptr) {
+  constexpr int kBlocks = 1024;
   int rc;
   if (!ctx->d_bounds &&
-      (rc = dev_alloc(ctx, &ctx->d_bounds, (size_t)1024 * PSH_BOUNDS_STRIDE)))
+      (rc = dev_alloc(ctx, &ctx->d_bounds, (size_t)2 * kBlocks * PSH_BOUNDS_STRIDE)))
     return rc;
-  HIPCHK(ctx, psh_coord_bounds(d, n, ctx->d_bounds, blocks, ctx->stream));
-  std::vector<double> h((size_t)blocks * PSH_BOUNDS_STRIDE);
-  HIPCHK(ctx, hipMemcpyAsync(h.data(), ctx->d_bounds, sizeof(double) * h.size(),
-                             hipMemcpyDeviceToHost, ctx->stream));
-  HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
-  double ws = 0.0;
-  for (int b = 0; b < blocks; b++) {
-    for (int a = 0; a < 3; a++) {
-      if (mn[a] > h[b * PSH_BOUNDS_STRIDE + a]) mn[a] = h[b * PSH_BOUNDS_STRIDE + a];
-      if (mx[a] < h[b * PSH_BOUNDS_STRIDE + 3 + a]) mx[a] = h[b * PSH_BOUNDS_STRIDE + 3 + a];
+  for (int i0 = 0; i0 < narr; i0 += 2) {   // the buffer holds two arrays' partials
+    const int na = std::min(2, narr - i0);
+    int blocks[2] = {0, 0};
+    for (int i = 0; i < na; i++) {
+      blocks[i] = (int)std::min<size_t>((n[i0 + i] + 255) / 256, kBlocks);
+      if (blocks[i])
+        HIPCHK(ctx, psh_coord_bounds(d[i0 + i], n[i0 + i],
+                                     ctx->d_bounds + (size_t)i * blocks[0] * PSH_BOUNDS_STRIDE,
+                                     blocks[i], ctx->stream));
     }
-    ws += h[b * PSH_BOUNDS_STRIDE + 6];
+    std::vector<double> h((size_t)(blocks[0] + blocks[1]) * PSH_BOUNDS_STRIDE);
+    if (!h.empty()) {
+      HIPCHK(ctx, hipMemcpyAsync(h.data(), ctx->d_bounds, sizeof(double) * h.size(),
+                                 hipMemcpyDeviceToHost, ctx->stream));
+      HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+    }
+    for (int i = 0; i < na; i++) {
+      double ws = 0.0;
+      for (int b = 0; b < blocks[i]; b++) {
+        const double *p = h.data() + ((size_t)i * blocks[0] + b) * PSH_BOUNDS_STRIDE;
+        for (int a = 0; a < 3; a++) {
+          if (mn[a] > p[a]) mn[a] = p[a];
+          if (mx[a] < p[3 + a]) mx[a] = p[3 + a];
+        }
+        ws += p[6];
+      }
+      if (wsum) wsum[i0 + i] = ws;
+    }
   }
-  if (wsum) *wsum = ws;
   return PSH_OK;
 }
 
@@ -1393,9 +1467,12 @@ int ctx_init(psh_ctx *ctx, const psh_conf *conf, int nmock_max) {
     return set_err(ctx, PSH_ERR_DEVICE, "no usable HIP device");
   }
   const size_t nm = (size_t)ctx->nmock_max;
-  if ((rc = dev_alloc(ctx, &ctx->meshA, ctx->mstride * nm)) ||
-      ((conf->intlace || ctx->survey) && (rc = dev_alloc(ctx, &ctx->meshB, ctx->mstride * nm))) ||
-      (ctx->survey && ctx->ellmax > 0 && (rc = alloc_survey_fields(ctx))))
+  // the shifted grid's (surveys: the second) meshes follow the plain ones, so
+  // that one launch of a pass takes both
+  const bool two = conf->intlace || ctx->survey;
+  if ((rc = dev_alloc(ctx, &ctx->meshA, ctx->mstride * nm * (two ? 2 : 1)))) return rc;
+  if (two) ctx->meshB = ctx->meshA + ctx->mstride * nm;
+  if ((ctx->survey && ctx->ellmax > 0 && (rc = alloc_survey_fields(ctx))))
     return rc;
   if ((rc = dev_alloc(ctx, &ctx->tw, (size_t)ctx->Ng))) return rc;
   if (psh_fft_twiddles_fill(ctx->Ng, ctx->tw) != hipSuccess)
@@ -1443,12 +1520,13 @@ extern "C" int psh_ctx_destroy(psh_ctx *ctx) {
   if (ctx->stream || ctx->arena) (void)hipStreamSynchronize(ctx->stream);
   if (ctx->gexec) (void)hipGraphExecDestroy(ctx->gexec);
   if (ctx->graph) (void)hipGraphDestroy(ctx->graph);
-  void *bufs[] = {ctx->meshA, ctx->meshB, ctx->meshS, ctx->counts, ctx->starts, ctx->cursors,
+  void *bufs[] = {ctx->meshA, ctx->meshS, ctx->counts, ctx->starts, ctx->cursors,
                   ctx->scan_tmp, ctx->d_parts, ctx->records, ctx->d_flags, ctx->tw,
                   ctx->phase, ctx->d_tab, ctx->d_ylive, ctx->d_gcnt, ctx->d_gkm,
                   ctx->d_glcnt, ctx->partials, ctx->d_bins, ctx->d_bounds, ctx->d_cat,
                   ctx->whist, ctx->d_mlp, ctx->d_ax, ctx->d_ay, ctx->d_acorr, ctx->d_afeat};
   for (void *p : bufs) ctx_free(ctx, p);
+  if (ctx->h_res) (void)hipHostFree(ctx->h_res);
   for (int i = 0; i < E_COUNT; i++)
     if (ctx->tm.ev[i]) (void)hipEventDestroy(ctx->tm.ev[i]);
   for (hipEvent_t e : ctx->tm.lev) (void)hipEventDestroy(e);
@@ -1598,8 +1676,13 @@ extern "C" int psh_fault_inject(int what, long value) {
 int sim_box_error(psh_ctx *ctx, const std::vector<PshDevPart> &hp) {
   double mn[3] = {DBL_MAX, DBL_MAX, DBL_MAX}, mx[3] = {-DBL_MAX, -DBL_MAX, -DBL_MAX};
   int rc;
-  for (auto &p : hp)
-    if ((rc = bounds_device(ctx, p.xyzw, p.n, mn, mx))) return rc;
+  std::vector<const double *> d;
+  std::vector<size_t> n;
+  for (auto &p : hp) {
+    d.push_back(p.xyzw);
+    n.push_back(p.n);
+  }
+  if ((rc = bounds_device(ctx, d.data(), n.data(), (int)hp.size(), mn, mx))) return rc;
   if ((rc = def_box(ctx, mn, mx))) return rc;
   return set_err(ctx, PSH_ERR_CATA, "particle coordinate outside the box [0, BOX_SIZE)");
 }
@@ -1619,41 +1702,53 @@ int sim_raw(psh_ctx *ctx, const std::vector<PshDevPart> &hp, std::vector<double>
   const double zero[3] = {0, 0, 0};
   if ((rc = def_box(ctx, zero, zero))) return rc;
   if ((rc = ensure_geometry(ctx))) return rc;
-  rc = run_assign(ctx, hp, 1, ctx->meshA, ctx->conf.intlace ? ctx->meshB : nullptr);
-  if (rc == PSH_ERR_CATA) return sim_box_error(ctx, hp);
-  if (rc) return rc;
-  const int nacc = psh_xbin_nacc(ctx->bins, PSH_EPI_SIM);
-  if ((rc = ensure_partials(ctx, 1, xgrid_for(ctx, 1, ctx->xres_sim), nacc, 1))) return rc;
-  if ((rc = run_sim_fft_bin(ctx, 1, ctx->d_bins))) return rc;
   const int nb = ctx->nbin, nl = ctx->conf.npole, nmu = ctx->bins.nmu;
+  const int nacc = psh_xbin_nacc(ctx->bins, PSH_EPI_SIM);
   const bool mlp = correct && ctx->mlp_nnet > 0 && !ctx->conf.intlace && nmu > 1;
+  if ((rc = ensure_partials(ctx, 1, xgrid_for(ctx, 1, ctx->xres_sim), nacc, 1))) return rc;
+  if (mlp && (rc = ensure_alias_rows(ctx))) return rc;
+  ensure_results(ctx, (size_t)nacc + (size_t)nl * nb);
   ctx->last_norm = norm;
   ctx->last_shot = shot;
-  if (mlp && (rc = ensure_alias_rows(ctx))) return rc;
-  if (mlp) {
-    const int rows = nb * nmu;
-    HIPCHK(ctx, psh_alias_features(ctx->d_bins, ctx->d_gcnt, nb, nmu, norm, shot,
-                                   M_PI * ctx->Ng / std::max(ctx->L[0], std::max(ctx->L[1], ctx->L[2])),
-                                   ctx->bins.kedge0, ctx->bins.dk, ctx->bins.logscale,
-                                   ctx->conf.assign, ctx->d_ax, ctx->d_afeat, ctx->stream));
-    // the ensemble in one launch (the networks' rows side by side in d_ay)
-    HIPCHK(ctx, psh_mlp_forward_async(ctx->d_mlp, ctx->d_ax, rows, ctx->d_ay, ctx->stream,
-                                      ctx->mlp_nnet));
-    HIPCHK(ctx, psh_alias_apply(ctx->d_ay, ctx->mlp_nnet, ctx->d_ax, ctx->d_bins, nl, nb, nmu,
-                                ctx->d_acorr, ctx->stream));
+  std::vector<double> sums((size_t)nacc + (mlp ? (size_t)nl * nb : 0));
+  rc = kRerun;
+  for (int attempt = 0; rc == kRerun; attempt++) {
+    if ((rc = run_assign(ctx, hp, 1, ctx->meshA, ctx->conf.intlace ? ctx->meshB : nullptr)))
+      return rc;
+    if ((rc = run_sim_fft_bin(ctx, 1, ctx->d_bins))) return rc;
+    if (mlp) {
+      const int rows = nb * nmu;
+      HIPCHK(ctx, psh_alias_features(ctx->d_bins, ctx->d_gcnt, nb, nmu, norm, shot,
+                                     M_PI * ctx->Ng / std::max(ctx->L[0], std::max(ctx->L[1], ctx->L[2])),
+                                     ctx->bins.kedge0, ctx->bins.dk, ctx->bins.logscale,
+                                     ctx->conf.assign, ctx->d_ax, ctx->d_afeat, ctx->stream));
+      // the ensemble in one launch (the networks' rows side by side in d_ay)
+      HIPCHK(ctx, psh_mlp_forward_async(ctx->d_mlp, ctx->d_ax, rows, ctx->d_ay, ctx->stream,
+                                        ctx->mlp_nnet));
+      HIPCHK(ctx, psh_alias_apply(ctx->d_ay, ctx->mlp_nnet, ctx->d_ax, ctx->d_bins, nl, nb, nmu,
+                                  ctx->h_res ? ctx->h_res + 1 + nacc : ctx->d_acorr,
+                                  ctx->stream));
+      if (!ctx->h_res)
+        HIPCHK(ctx, hipMemcpyAsync(sums.data() + nacc, ctx->d_acorr, sizeof(double) * nl * nb,
+                                   hipMemcpyDeviceToHost, ctx->stream));
+    }
+    ev_record(ctx, E_END);
+    int flags = 0;
+    if ((rc = fetch_results(ctx, ctx->d_bins, ctx->h_res ? sums.size() : (size_t)nacc,
+                            sums.data(), &flags)))
+      return rc;
+    rc = flags_error(ctx, flags, attempt);
   }
-  ev_record(ctx, E_END);
-  ctx->cells.assign(nacc, 0.0);
-  HIPCHK(ctx, hipMemcpyAsync(ctx->cells.data(), ctx->d_bins, sizeof(double) * nacc,
-                             hipMemcpyDeviceToHost, ctx->stream));
-  raw.assign((size_t)nl * nb, 0.0);
-  if (mlp)
-    HIPCHK(ctx, hipMemcpyAsync(raw.data(), ctx->d_acorr, sizeof(double) * nl * nb,
-                               hipMemcpyDeviceToHost, ctx->stream));
-  HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
-  if (!mlp)
+  if (rc == PSH_ERR_CATA) return sim_box_error(ctx, hp);
+  if (rc) return rc;
+  ctx->cells.assign(sums.begin(), sums.begin() + nacc);
+  if (mlp) {
+    raw.assign(sums.begin() + nacc, sums.end());
+  } else {
+    raw.assign((size_t)nl * nb, 0.0);
     for (size_t q = 0; q < raw.size(); q++)
       for (int c = 0; c < nmu; c++) raw[q] += ctx->cells[q * nmu + c];
+  }
   ev_collect(ctx);
   return PSH_OK;
 }
@@ -1847,15 +1942,15 @@ extern "C" int psh_ctx_run_batch(psh_ctx *ctx, const psh_data *d_data,
   const int nacc = psh_xbin_nacc(ctx->bins, PSH_EPI_SIM);
   if ((rc = ensure_partials(ctx, nmock, grid, nacc, 1))) return rc;
   if ((rc = ensure_assign_scratch(ctx, nmock, nmock, ntotal))) return rc;
+  ensure_results(ctx, (size_t)nmock * nacc);
   // boxes: weights of one sign, 64-bit cells only for the fused shape's
   // small grids (run_assign sets the same for the eager path)
   ctx->ag.wide = ctx->ag.zfuse && psh_zfuse_wide(ctx->Ng);
   float *mB = ctx->conf.intlace ? ctx->meshB : nullptr;
   std::vector<double> raw((size_t)nmock * nacc);
   int flags = 0;
-  // a replay whose records overflow the buffer is rerun after the buffer
-  // grows (the graph, which holds the old buffer, is captured again), as the
-  // eager path's run_assign does
+  // a run whose records overflow the buffer is repeated after the buffer
+  // grows (a graph, which holds the old buffer, is captured again)
   for (int attempt = 0;; attempt++) {
     ev_record(ctx, E_START);
     if (!graph) {
@@ -1904,14 +1999,9 @@ extern "C" int psh_ctx_run_batch(psh_ctx *ctx, const psh_data *d_data,
       HIPCHK(ctx, hipGraphLaunch(ctx->gexec, ctx->stream));
     }
     ev_record(ctx, E_END);
-    HIPCHK(ctx, hipMemcpyAsync(raw.data(), ctx->d_bins, sizeof(double) * raw.size(),
-                               hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(ctx, hipMemcpyAsync(&flags, ctx->d_flags, sizeof(int), hipMemcpyDeviceToHost,
-                               ctx->stream));
-    HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
-    if (!(flags & 1)) break;
-    if (attempt == 3) return set_err(ctx, PSH_ERR_MESH, "assignment record buffer overflow");
-    if ((rc = grow_records(ctx))) return rc;
+    if ((rc = fetch_results(ctx, ctx->d_bins, raw.size(), raw.data(), &flags))) return rc;
+    rc = flags_error(ctx, flags, attempt);
+    if (rc != kRerun) break;
   }
   if (graph) {
     if (ctx->profiling) {
@@ -1921,9 +2011,7 @@ extern "C" int psh_ctx_run_batch(psh_ctx *ctx, const psh_data *d_data,
   } else {
     ev_collect(ctx);
   }
-  if (flags & 4)
-    return set_err(ctx, PSH_ERR_CATA, "particle coordinate outside the box [0, BOX_SIZE)");
-  if (flags & 2) return set_err(ctx, PSH_ERR_MESH, "inconsistent interlaced cell of a particle");
+  if (rc) return rc;
   const double vol = ctx->L[0] * ctx->L[1] * ctx->L[2];
   const int nmu = ctx->bins.nmu;
   std::vector<double> sums((size_t)ctx->conf.npole * ctx->nbin);
@@ -2254,10 +2342,10 @@ extern "C" int psh_ctx_run_survey_device(psh_ctx *ctx, const psh_data *d_data, s
   int rc;
   // box from the coordinate range of data and randoms (src/genr_mesh.c:427-578)
   double mn[3] = {DBL_MAX, DBL_MAX, DBL_MAX}, mx[3] = {-DBL_MAX, -DBL_MAX, -DBL_MAX};
-  double swd = 0, swr = 0;
-  if ((rc = bounds_device(ctx, (const double *)d_data, nd, mn, mx, &swd)) ||
-      (rc = bounds_device(ctx, (const double *)d_rand, nr, mn, mx, &swr)) ||
-      (rc = def_box(ctx, mn, mx)) || (rc = ensure_geometry(ctx)))
+  const double *arr[2] = {(const double *)d_data, (const double *)d_rand};
+  const size_t num[2] = {nd, nr};
+  double sw[2] = {0, 0};
+  if ((rc = bounds_device(ctx, arr, num, 2, mn, mx, sw)) || (rc = def_box(ctx, mn, mx)) || (rc = ensure_geometry(ctx)))
     return rc;
   CatDev cd[2] = {};
   cd[0].data = (const double *)d_data;
@@ -2267,8 +2355,8 @@ extern "C" int psh_ctx_run_survey_device(psh_ctx *ctx, const psh_data *d_data, s
   cd[0].alpha = alpha;
   cd[0].shot = shot;
   cd[0].norm = norm;
-  cd[0].sw_d = swd;
-  cd[0].sw_r = swr;
+  cd[0].sw_d = sw[0];
+  cd[0].sw_r = sw[1];
   return run_catalogues(ctx, cd, 1, out);
 }
 

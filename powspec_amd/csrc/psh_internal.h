@@ -247,9 +247,11 @@ hipError_t psh_geometry(int Ng, const PshAxisTables &ax, const PshBins &b,
     hipStream_t s);
 
 // Sum partials[nmock][grid][nacc] over grid in a fixed order into
-// out[nmock][nacc].
+// out[nmock][nacc]; hout and hflags (pinned host memory, may be nullptr)
+// receive the sums and flags[0] as well.
 hipError_t psh_reduce_partials(const double *partials, int nmock, int grid,
-    int nacc, double *out, hipStream_t s);
+    int nacc, double *out, hipStream_t s, double *hout = nullptr,
+    const int *flags = nullptr, double *hflags = nullptr);
 
 // Exclusive scan of n uint32 counts into out[0..n] (out[n] = total); tmp
 // holds psh_assign_scan_bytes(n) bytes.  in and out must not overlap.

@@ -72,3 +72,24 @@ def test_batch_parts(psh, nmock):
             # integers may sit at another power of two than alone
             s = np.abs(one["pl"][0][0]) + L ** 3 / w
             assert np.all(np.abs(g["pl"][0] - one["pl"][0]) <= 1e-5 * s)
+
+
+def test_record_overflow_reruns(psh, oracle):
+    """Every particle at a corner of eight tiles: more records than the buffer
+    expects, found when the run's results arrive; the run is repeated with a
+    larger buffer, and the next one fits at once."""
+    Ng, n = 64, 30000
+    rng = np.random.default_rng(3)
+    d = np.empty((n, 4))
+    d[:, :3] = (8 * rng.integers(0, Ng // 8, (n, 3)) + 7.6) * (L / Ng)
+    d[:, 3] = 1.0
+    kw = dict(gsize=Ng, assign=psh.PCS, intlace=True, bsize=L, kbin=0.02, poles=[0, 2, 4])
+    ref = oracle.run(oracle.make_conf(**kw), [d])
+    dev = psh.DeviceArray.from_numpy(d)
+    for graph in (None, False, True):
+        ctx = psh.Context(psh.make_conf(**kw))
+        ctx.set_tiles((8, 8, 8))
+        for _ in range(2):
+            got = (ctx.run_device(dev, n, float(n)) if graph is None else
+                   ctx.run_batch(dev, [0, n], [float(n)], graph=graph)[0])
+            _check(got, ref, [0, 2, 4], ref["shot"][0])
