@@ -26,11 +26,15 @@
 
 namespace {
 
+// A particle as one of its tiles sees it: cells relative to the tile's first
+// (a window that begins in the neighbouring tile before it has negative
+// ones), so the deposit needs neither the tile's place nor the periodic wrap.
+constexpr int kRecBias = 8;   // added to the local cells, which start at -W
 struct __align__(8) Rec {
   float f[3];      // window fraction on the plain grid, per axis
   float w;         // particle weight times the catalogue scale
-  uint32_t bxy;    // base cell x | y << 16 (plain grid)
-  uint32_t bz;     // base cell z | delta bits (shifted grid) << 16
+  uint32_t bxy;    // biased local base cell x | y << 16 (plain grid)
+  uint32_t bz;     // biased local base cell z | delta bits (shifted grid) << 16
 };
 static_assert(sizeof(Rec) == 24, "record layout");
 
@@ -216,6 +220,14 @@ __device__ __forceinline__ Loaded load_particle(const DevPart *parts, int nparts
 struct PartTiles {
   int t0;
   int off[3];   // x, y, z
+  // the record as tile k sees it: a second tile along an axis lies the
+  // tile's extent after the first
+  __device__ __forceinline__ Rec record(Rec r, const PshAssignGeom &g, int k) const {
+    if (k & 4) r.bxy -= (uint32_t)g.tile[0];
+    if (k & 2) r.bxy -= (uint32_t)g.tile[1] << 16;
+    if (k & 1) r.bz -= (uint32_t)g.tile[2];
+    return r;
+  }
   __device__ __forceinline__ bool has(int k) const {
     return (!(k & 4) || off[0]) && (!(k & 2) || off[1]) && (!(k & 1) || off[2]);
   }
@@ -226,7 +238,7 @@ struct PartTiles {
 };
 
 // Tiles (mock-local indices) touched by a particle rr = (x, y, z, w) and its
-// record.  Returns false (and sets flag bit 2) when the shifted grid's base
+// record as the first of them sees it.  Returns false (and sets flag bit 2) when the shifted grid's base
 // is inconsistent.  With CHECK and g.check_box, a coordinate outside
 // [bmin, bmin + L) (bmin = 0 for simulation boxes) sets flag bit 4: the box
 // check of simulation catalogues (src/genr_mesh.c:517-533) folded into the
@@ -261,6 +273,8 @@ __device__ __forceinline__ bool particle_tiles(const PshAssignGeom &g, const dou
   pt.off[1] = o[1] * g.ntile[2];
   pt.off[2] = o[2];
   rec.w = (float)rr[3] * wscale;
+#pragma unroll
+  for (int a = 0; a < 3; a++) b[a] = (b[a] & (g.tile[a] - 1)) + kRecBias;
   rec.bxy = (uint32_t)b[0] | ((uint32_t)b[1] << 16);
   rec.bz = (uint32_t)b[2] | ((uint32_t)(dl[0] | (dl[1] << 1) | (dl[2] << 2)) << 16);
   return true;
@@ -414,8 +428,9 @@ assign_bucket(PshAssignGeom g, const DevPart *__restrict__ parts, int nparts, si
     for (uint32_t i = threadIdx.x; i < win; i += T) hist[i] = 0;
     __syncthreads();
   };
-  // counts the pairs inside the window; `single` takes the others (k-th
-  // tile of the lanes of a wave together)
+  uint32_t ranges = 0;   // nonzero counters and singles
+  // counts the pairs inside the window and, with `singles`, the others (the
+  // k-th tiles of a wave's lanes together)
   auto count_pairs = [&](auto check, bool singles) {
     sweep(check, [&](const PartTiles &pt, const Rec &, bool live, int mock) {
       const bool mine = live && mock == mock0;
@@ -433,19 +448,28 @@ assign_bucket(PshAssignGeom g, const DevPart *__restrict__ parts, int nparts, si
         const bool act = out && pt.has(k) && !(mine && pt.tile(k) - wbase < win);
         if (!__ballot(act)) continue;
         run_increment<false>(cursors, act ? (uint32_t)mock * tpm + pt.tile(k) : 0u, act);
+        ranges += act;
       }
     });
     __syncthreads();
   };
 
   if (!FILL) {
+    __shared__ uint32_t nrange;
+    if (threadIdx.x == 0) nrange = 0;
     clear();
     count_pairs(std::true_type{}, true);
     for (uint32_t i = threadIdx.x; i < win; i += T) {
       const uint32_t v = hist[i];
+      ranges += v != 0;
       if (wh) wh[i] = v ? atomicAdd(&counts[mbase0 + i], v) : 0u;
       else if (v) atomicAdd(&cursors[mbase0 + i], v);
     }
+    // ranges of records that fill the buckets (record_group)
+    for (int o = 32; o > 0; o >>= 1) ranges += __shfl_xor(ranges, o);
+    if (__lane_id() == 0) atomicAdd(&nrange, ranges);
+    __syncthreads();
+    if (threadIdx.x == 0) atomicAdd(reinterpret_cast<uint32_t *>(flags) + 2, nrange);
     return;
   }
   if (wh) {
@@ -485,7 +509,7 @@ assign_bucket(PshAssignGeom g, const DevPart *__restrict__ parts, int nparts, si
 #pragma unroll
     for (int k = 0; k < 8; k++) {
       if (!live || !pt.has(k)) continue;
-      if (slot[k] < rec_cap) recs[slot[k]] = rec;
+      if (slot[k] < rec_cap) recs[slot[k]] = pt.record(rec, g, k);
       else atomicOr(flags, 1);
     }
   });
@@ -696,7 +720,11 @@ assign_begin(uint32_t *__restrict__ counts, uint32_t *__restrict__ cursors, size
 
 // ---- deposit: one workgroup per tile ------------------------------------------
 
+// The products that are added to something are fused into the addition
+// explicitly: left to the compiler, which fusions it makes depends on the code
+// around the call, and so would the last bits of the weights.
 __device__ __forceinline__ void window_weights(int scheme, float f, float *w) {
+#pragma clang fp contract(off)
   switch (scheme) {
     case 0:
       w[0] = 1.f;
@@ -706,21 +734,18 @@ __device__ __forceinline__ void window_weights(int scheme, float f, float *w) {
       w[1] = f;
       break;
     case 2: {
-      float a = 0.5f - f;
-      w[0] = 0.5f * a * a;
-      w[1] = 0.75f - f * f;
-      w[2] = 1.f - w[0] - w[1];
+      const float a = 0.5f - f, h = 0.5f * a;
+      w[0] = a * h;
+      w[1] = __builtin_fmaf(-f, f, 0.75f);
+      w[2] = __builtin_fmaf(-a, h, 1.f) - w[1];
       break;
     }
     default: {
-      float d2 = f * f;
-      float w3 = d2 * f;
-      float w2 = 1.f + 3.f * (f + d2 - w3);
-      float w1 = 4.f - 6.f * d2 + 3.f * w3;
-      w[3] = w3;
-      w[2] = w2;
-      w[1] = w1;
-      w[0] = 6.f - w1 - w2 - w3;
+      const float d2 = f * f;
+      w[3] = f * d2;
+      w[2] = __builtin_fmaf(__builtin_fmaf(-f, d2, __builtin_fmaf(f, f, f)), 3.f, 1.f);
+      w[1] = __builtin_fmaf(3.f, w[3], __builtin_fmaf(-6.f, d2, 4.f));
+      w[0] = __builtin_fmaf(-f, d2, (6.f - w[1]) - w[2]);
       break;
     }
   }
@@ -762,7 +787,7 @@ struct Acc<true> {
 
 // Window axes x and y: an axis a >= branch_axes is deposited without
 // branches (a window cell outside the tile gets weight 0 and the address of
-// cell 0 along that axis; adding the integer 0 there is exact), an axis
+// a cell inside; adding the integer 0 there is exact), an axis
 // below keeps a branch per plane or row, which skips whole planes or rows
 // outside the tile.  Measured on MI355X: y without branches for CIC and TSC,
 // with them for PCS (whose 4-cell rows make a skipped row worth more).
@@ -770,79 +795,71 @@ struct Acc<true> {
 // row is W consecutive cells from one base address (constant LDS offsets,
 // no per-cell mask or address arithmetic); cells in the padding are
 // dropped, their tile deposits them from its own record.  A record's tile
-// meets the union of the plain and the shifted window, so the plain
-// window's first cell b lies in [T0 - W, T0 + T[2]) and the shifted one's
-// in [T0 - W + 1, T0 + T[2]] (up to a wrap by Ng): W cells of padding on
-// each side hold every window cell outside the tile.  When T[2] + W >= Ng
-// (one tile, or two tiles on a tiny grid) a window offset is ambiguous
-// modulo Ng, and z goes the branch-free way of x and y instead (ZPAD false).
+// meets the union of the plain and the shifted window, so the window's first
+// cell lies in [-W, T[2]] and W cells of padding on each side hold every
+// cell outside the tile.
+// WRAP: some axis of the tile spans the grid, so that windows wrap around
+// inside the tile; z then goes the branch-free way of x and y.
 template <int SCHEME>
 constexpr int branch_axes() { return SCHEME == 3 ? 2 : 1; }
 
-// Accumulate one particle's window into an LDS tile of fixed-point cells
-// (rows of P2 = T[2] + 2 W cells, the tile's first z cell at W).
-template <int SCHEME, bool WIDE, bool ZPAD>
-__device__ __forceinline__ void deposit_one(typename Acc<WIDE>::T *lds, const int *T,
-                                            const int *T0, int Ng, int P2, const int *b,
-                                            const float *f, float w) {
+// Accumulate one particle's window, whose first cell is l (local), into an
+// LDS tile of fixed-point cells (rows of P2 >= T[2] + 2 W cells, the tile's
+// first z cell at W).
+template <int SCHEME, bool WIDE, bool WRAP>
+__device__ __forceinline__ void deposit_one(typename Acc<WIDE>::T *lds, const int *T, int Ng,
+                                            int P2, const int *l, const float *f, float w) {
   constexpr int W = SCHEME + 1;
   constexpr int kBranchAxes = branch_axes<SCHEME>();
   float wt[3][4];
-  int l[3][4];
-  unsigned m[3];
 #pragma unroll
-  for (int a = 0; a < 3; a++) {
-    window_weights(SCHEME, f[a], wt[a]);
-    m[a] = 0;
-    if (ZPAD && a == 2) break;
+  for (int a = 0; a < 3; a++) window_weights(SCHEME, f[a], wt[a]);
+  // cell n of axis a, and whether it lies in the tile
+  auto cell = [&](int a, int n, bool &in) -> int {
+    int c = l[a] + n;
+    if (WRAP && c >= Ng) c -= Ng;
+    in = (unsigned)c < (unsigned)T[a];
+    return c;
+  };
+  int zc[4];   // WRAP: the row's cells
+  if (WRAP) {
 #pragma unroll
     for (int n = 0; n < W; n++) {
-      int c = b[a] + n;
-      if (c >= Ng) c -= Ng;
-      const int lc = c - T0[a];
-      const bool in = lc >= 0 && lc < T[a];
-      if (a < kBranchAxes) {
-        l[a][n] = lc;
-        if (in) m[a] |= 1u << n;
-      } else {
-        l[a][n] = in ? lc : 0;
-        if (!in) wt[a][n] = 0.f;
-      }
+      bool in;
+      const int c = cell(2, n, in);
+      zc[n] = in ? c : 0;
+      if (!in) wt[2][n] = 0.f;
     }
-  }
-  // ZPAD: offset in a padded row of the window's first z cell, b - T0 + W
-  // modulo Ng, in [0, T[2] + W] (cells up to T[2] + 2W - 1 < P2).  The
-  // difference itself lies in [W + T[2] - Ng, Ng + W): windows wrapped by Ng
-  // at the tile at z = 0 (b in [Ng - W, Ng)) give b + W in [Ng, Ng + W),
-  // and the shifted window of the last tile whose base wrapped to 0 gives
-  // T[2] + W - Ng < 0; with T[2] + W < Ng one addition or subtraction of Ng
-  // maps both into range and moves nothing else.
-  int zoff = W;
-  if (ZPAD) {
-    zoff = b[2] - T0[2] + W;
-    if (zoff >= Ng) zoff -= Ng;
-    else if (zoff < 0) zoff += Ng;
   }
   if (SCHEME == 3) w *= (1.0f / 216.0f);
   const float half = __builtin_copysignf(0.5f, w);   // window weights are >= 0
-  // row offsets: one integer multiply per window cell of x and of y
+  // row offsets: the products stay below 2^24 (a tile has at most 40960
+  // cells), where the integer multiply-add runs at full rate
+  const int z0 = WRAP ? W : l[2] + W;
   int ry[4];
+  bool iny[4];
 #pragma unroll
-  for (int j = 0; j < W; j++) ry[j] = l[1][j] * P2 + zoff;
+  for (int j = 0; j < W; j++) {
+    const int c = cell(1, j, iny[j]);
+    if (kBranchAxes <= 1 && !iny[j]) wt[1][j] = 0.f;
+    ry[j] = __mul24(min(max(c, 0), T[1] - 1), P2) + z0;
+  }
   const int PP = T[1] * P2;
 #pragma unroll
   for (int i = 0; i < W; i++) {
-    if (kBranchAxes > 0 && !(m[0] >> i & 1)) continue;
+    bool inx;
+    const int c = cell(0, i, inx);
+    if (!inx) continue;
     const float wx = wt[0][i] * w;
-    const int rx = l[0][i] * PP;
+    const int rx = __mul24(c, PP);
 #pragma unroll
     for (int j = 0; j < W; j++) {
-      if (kBranchAxes > 1 && !(m[1] >> j & 1)) continue;
+      if (kBranchAxes > 1 && !iny[j]) continue;
       const float wxy = wx * wt[1][j];
       typename Acc<WIDE>::T *row = lds + rx + ry[j];
 #pragma unroll
       for (int k = 0; k < W; k++)
-        Acc<WIDE>::add(ZPAD ? row + k : row + l[2][k], wxy, wt[2][k], half);
+        Acc<WIDE>::add(WRAP ? row + zc[k] : row + k, wxy, wt[2][k], half);
     }
   }
 }
@@ -893,204 +910,320 @@ struct ZfCfg {
   static_assert(TX * TY == R && TY >= 4, "tile rows");
 };
 
-template <int SCHEME, bool INTLACE, bool WIDE, bool NT, int NZ>
+// Tile of a workgroup.
+struct DepTile {
+  int T[3], T0[3];
+  int mock;
+  uint32_t tile;
+};
+
+__device__ __forceinline__ DepTile dep_tile(const PshAssignGeom &g, uint32_t tile) {
+  // tile index -> (mock, x, y, z) tile; tile counts need not be powers of
+  // two (a grid of 3 * 2^k or 5 * 2^k cells has 3 or 5 times a power)
+  DepTile d;
+  const uint32_t nz = (uint32_t)g.ntile[2], ny = (uint32_t)g.ntile[1];
+  const uint32_t tpm = (uint32_t)g.ntile[0] * ny * nz;
+  d.tile = tile;
+  d.mock = (int)(tile / tpm);
+  const uint32_t tl = tile - (uint32_t)d.mock * tpm;
+  const uint32_t tyz = tl / nz;
+  const uint32_t tx = tyz / ny;
+#pragma unroll
+  for (int a = 0; a < 3; a++) d.T[a] = g.tile[a];
+  d.T0[0] = (int)tx * d.T[0];
+  d.T0[1] = (int)(tyz - tx * ny) * d.T[1];
+  d.T0[2] = (int)(tl - tyz * nz) * d.T[2];
+  return d;
+}
+
+template <class AT>
+__device__ __forceinline__ void clear_cells(AT *lds, int cells) {
+  uint4 *z4 = reinterpret_cast<uint4 *>(lds);   // cells: a multiple of 4
+  const int n4 = (int)(sizeof(AT) * cells / 16);
+  for (int i = threadIdx.x; i < n4; i += blockDim.x) z4[i] = make_uint4(0u, 0u, 0u, 0u);
+}
+
+// The records of a bucket over the workgroup's threads: visit(r) for each,
+// the next one loading while the current one is deposited.
+//  - At most one record per thread: on the fewest waves that hold them
+//    (nw = ceil(cnt / 64)), since a VALU-bound wave issues as many
+//    instructions for 20 live lanes as for 64 and the other waves go straight
+//    to the barrier.  Lane l of wave w < nw takes record l * nw + w (a
+//    bijection of [0, 64 nw)), so a wave's lanes hold records nw apart in
+//    fill order rather than neighbours.
+//  - More: groups of 2^gs neighbours in the
+//    order q -> (q * S) mod ngroups with S ~ 0.618 ngroups and
+//    gcd(S, ngroups) = 1 (a permutation): a wave's groups lie far apart in
+//    fill order, i.e. far apart in a space-ordered catalogue, so
+//    its lanes' windows rarely meet in one cell (record_group).
+template <class F>
+__device__ __forceinline__ void for_records(const Rec *__restrict__ recs, uint32_t cnt, uint32_t gs,
+                                            F visit) {
+  const uint32_t t = threadIdx.x, B = blockDim.x;
+  if (cnt <= B) {
+    const uint32_t nw = (cnt + 63u) >> 6, w = t >> 6;
+    const uint32_t j = (t & 63u) * nw + w;
+    const bool live = w < nw && j < cnt;
+    Rec r;
+    if (live) r = recs[j];
+    __syncthreads();   // the cells are cleared
+    if (live) visit(r);
+    return;
+  }
+  const uint32_t ng = (cnt + (1u << gs) - 1) >> gs;
+  uint32_t S = ((uint32_t)((float)ng * 0.618034f)) | 1u;
+  if (S >= ng) S = 1u;
+  for (;;) {
+    uint32_t a = S, b = ng;
+    while (b) {
+      const uint32_t q = a % b;
+      a = b;
+      b = q;
+    }
+    if (a == 1u) break;
+    S += 2u;
+    if (S >= ng) {
+      S = 1u;
+      break;
+    }
+  }
+  const uint32_t in = t & ((1u << gs) - 1u), step = B >> gs;
+  uint32_t q = t >> gs;
+  uint32_t x = (uint32_t)(((uint64_t)q * S) % ng);
+  const uint32_t D = (uint32_t)(((uint64_t)step * S) % ng);
+  auto index = [&]() -> uint32_t { return q < ng ? (x << gs) + in : cnt; };
+  auto next = [&]() {
+    q += step;
+    x += D;
+    if (x >= ng) x -= ng;
+  };
+  uint32_t i = index();
+  Rec r;
+  if (i < cnt) r = recs[i];
+  __syncthreads();   // the cells are cleared
+  const uint32_t iters = (ng + step - 1) / step;
+  for (uint32_t it = 0; it < iters; it++) {
+    next();
+    const uint32_t in2 = index();
+    Rec r2;
+    if (in2 < cnt) r2 = recs[in2];
+    if (i < cnt) visit(r);
+    i = in2;
+    r = r2;
+  }
+}
+
+// log2 of the records a wave reads from consecutive places of a bucket:
+// larger groups use more of the 128-byte lines they touch, smaller ones keep
+// the windows of a space-ordered catalogue's neighbours apart.  Ordered:
+// 2 records for the wide windows (N = 256 TSC, 32 mocks: 1.71, 1.69, 1.76 ms
+// for 1, 2, 4), 4 for NGP and CIC (N = 512, 2e7 particles: 301, 269, 247 us).
+// A bucket filled in ranges of a few records (fewer than 16 on average, from
+// the count pass's number of ranges) is in random order, where neighbours are
+// no closer than others: a whole wave's (survey, N = 512, 1e8 randoms:
+// 2.12 ms with 4, 1.82 with 64).
+template <int SCHEME>
+__device__ __forceinline__ uint32_t record_group(const uint32_t *starts, uint32_t ntiles,
+                                                 const int *flags) {
+  const bool random = starts[ntiles] / 16 < (uint32_t)flags[2];
+  return random ? 6u : (SCHEME >= 2 ? 1u : 2u);
+}
+
+// One record's window on the plain or the shifted grid of a tile.
+template <int SCHEME, bool WIDE>
+__device__ __forceinline__ void deposit_rec(typename Acc<WIDE>::T *lds, const DepTile &d,
+                                            const PshAssignGeom &g, int P2, bool wrap,
+                                            bool shifted, const Rec &r, float scale) {
+  int l[3] = {(int)(r.bxy & 0xffffu) - kRecBias, (int)(r.bxy >> 16) - kRecBias,
+              (int)(r.bz & 0xffffu) - kRecBias};
+  float f[3] = {r.f[0], r.f[1], r.f[2]};
+  if (shifted) {
+    const uint32_t dl = r.bz >> 16;
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+      const int s = (dl >> a) & 1;
+      l[a] += s;
+      f[a] = f[a] + 0.5f - (float)s;
+    }
+  }
+  const float ws = r.w * scale;
+  if (wrap) deposit_one<SCHEME, WIDE, true>(lds, d.T, g.Ng, P2, l, f, ws);
+  else deposit_one<SCHEME, WIDE, false>(lds, d.T, g.Ng, P2, l, f, ws);
+}
+
+// Bucket of a tile.  Records past the buffer were never written (overflow
+// flag set, the run is repeated with a larger buffer): never read beyond
+// rec_cap.
+struct DepBucket {
+  uint32_t s0, cnt;
+  float scale, inv;
+};
+
+template <int TOP>
+__device__ __forceinline__ DepBucket dep_bucket(const uint32_t *starts, uint32_t tile,
+                                                size_t rec_cap, const int *flags) {
+  const uint32_t cap = rec_cap < 0xffffffffu ? (uint32_t)rec_cap : 0xffffffffu;
+  const uint32_t s0 = min(starts[tile], cap), s1 = min(starts[tile + 1], cap);
+  DepBucket k;
+  k.s0 = s0;
+  k.cnt = s1 > s0 ? s1 - s0 : 0u;
+  const int sexp = tile_exponent<TOP>(flags, k.cnt);
+  k.scale = ldexpf(1.f, sexp);
+  k.inv = ldexpf(1.f, -sexp);
+  return k;
+}
+
+// Deposit of one grid (plain, or with INTLACE every second group of 8
+// workgroups the shifted one) of one tile per workgroup.  Bound: the LDS
+// atomics of the windows and the stores of the mesh; their phases alternate
+// within a workgroup, so it is other workgroups of the CU that overlap them.
+// One grid per workgroup halves the LDS tile: 4 workgroups of 512 threads per
+// CU instead of 2 for 32-bit cells, 2 instead of 1 for the survey's 64-bit
+// cells, for a second read of the records (the two grids of a tile follow
+// one another on one XCD: workgroups are dealt to the XCDs in turn).
+// Measured on MI355X (with the records' local cells, the next record in
+// flight and 16-byte LDS reads): N = 1024 PCS, 2e7 particles 2.72 -> 2.34 ms,
+// 8.6 GB of mesh at 3.7 TB/s; the survey's 64-bit CIC, N = 512, 1.5e8 records
+// 2.81 -> 1.64 ms; N = 512 CIC, 2e7 particles 0.31 -> 0.25 ms.
+template <int SCHEME, bool INTLACE, bool WIDE, bool NT>
 __global__ void __launch_bounds__(1024)
 assign_deposit(PshAssignGeom g, const uint32_t *__restrict__ starts,
                const Rec *__restrict__ recs, size_t rec_cap,
                float *__restrict__ meshA, float *__restrict__ meshB,
-               size_t mstride, const int *__restrict__ flags, size_t ntotal) {
+               size_t mstride, const int *__restrict__ flags, int P2, int lead, int cells,
+               uint32_t ntiles) {
+  using AT = typename Acc<WIDE>::T;
+  extern __shared__ __align__(16) long long ldsraw[];
+  AT *lds = reinterpret_cast<AT *>(ldsraw) + lead;
+  uint32_t tile = blockIdx.x;
+  bool shifted = false;
+  if (INTLACE) {
+    // blocks 16 n + (0..7) and 16 n + 8 + (0..7): the grids of tiles 8 n + (0..7)
+    const uint32_t b = blockIdx.x, half = gridDim.x >> 1;
+    if (half & 7) {
+      shifted = b & 1;
+      tile = b >> 1;
+    } else {
+      shifted = (b >> 3) & 1;
+      tile = (b >> 4) * 8 + (b & 7);
+    }
+  }
+  const DepBucket k = dep_bucket<Acc<WIDE>::TOP>(starts, tile, rec_cap, flags);
+  const DepTile d = dep_tile(g, tile);
+  const bool wrap = d.T[0] == g.Ng || d.T[1] == g.Ng || d.T[2] == g.Ng;
+  clear_cells(lds - lead, cells);
+  for_records(recs + k.s0, k.cnt, record_group<SCHEME>(starts, ntiles, flags), [&](const Rec &r) {
+    deposit_rec<SCHEME, WIDE>(lds, d, g, P2, wrap, shifted, r, k.scale);
+  });
+  __syncthreads();
+
+  // write the tile: rows of T[2] floats along z, 4 cells per thread
+  const int nrow = d.T[0] * d.T[1];
+  const int q4s = g.tile_shift[2] - 2;   // T[2] = 4 * 2^q4s (T[2] >= 4)
+  const int q4 = 1 << q4s;
+  float *out = (shifted ? meshB : meshA) + (size_t)d.mock * mstride;
+  for (int i = threadIdx.x; i < nrow * q4; i += blockDim.x) {
+    const int row = i >> q4s, q = i & (q4 - 1);
+    const int lx = row >> g.tile_shift[1], ly = row & (d.T[1] - 1);
+    const size_t gidx = ((size_t)(d.T0[0] + lx) * g.Ng + (d.T0[1] + ly)) * g.row_pitch +
+                        d.T0[2] + 4 * q;
+    const int li = row * P2 + SCHEME + 1 + 4 * q;
+    AT c[4];
+    if (((P2 | (lead + SCHEME + 1)) & 3) == 0) {   // 16-byte aligned rows
+      const uint4 *p = reinterpret_cast<const uint4 *>(lds + li);
+#pragma unroll
+      for (int h = 0; h < (int)(sizeof(c) / 16); h++) reinterpret_cast<uint4 *>(c)[h] = p[h];
+    } else {
+#pragma unroll
+      for (int h = 0; h < 4; h++) c[h] = lds[li + h];
+    }
+    const float4 v = make_float4((float)c[0] * k.inv, (float)c[1] * k.inv, (float)c[2] * k.inv,
+                                 (float)c[3] * k.inv);
+    store4<NT>(out + gidx, v);
+  }
+}
+
+// Deposit of both grids of a tile of whole z rows, transformed along z.
+template <int SCHEME, bool INTLACE, bool WIDE, bool NT, int NZ>
+__global__ void __launch_bounds__(1024)
+assign_deposit_z(PshAssignGeom g, const uint32_t *__restrict__ starts,
+                 const Rec *__restrict__ recs, size_t rec_cap,
+                 float *__restrict__ meshA, float *__restrict__ meshB,
+                 size_t mstride, const int *__restrict__ flags) {
   using AT = typename Acc<WIDE>::T;
   extern __shared__ __align__(16) long long ldsraw[];
   AT *ldsq = reinterpret_cast<AT *>(ldsraw);
-  const int T[3] = {g.tile[0], g.tile[1], g.tile[2]};
-  const int P2 = psh_tile_pitch(T[2], SCHEME);
-  const int gcells = (int)psh_tile_cells(T, SCHEME);   // per grid, padded
-  const bool zpad = T[2] + SCHEME + 1 < g.Ng;
+  const DepBucket k = dep_bucket<Acc<WIDE>::TOP>(starts, blockIdx.x, rec_cap, flags);
+  const DepTile d = dep_tile(g, blockIdx.x);
+  const int P2 = psh_tile_pitch(d.T[2], SCHEME);
+  const int gcells = (int)psh_tile_cells(d.T, SCHEME);   // per grid, padded
+  const bool wrap = d.T[0] == g.Ng || d.T[1] == g.Ng || d.T[2] == g.Ng;
   AT *ldsA = ldsq;
   AT *ldsB = ldsq + gcells;
-  // tile index -> (mock, x, y, z) tile; tile counts need not be powers of
-  // two (a grid of 3 * 2^k or 5 * 2^k cells has 3 or 5 times a power)
-  const uint32_t tile = blockIdx.x;
-  const uint32_t nz = (uint32_t)g.ntile[2], ny = (uint32_t)g.ntile[1];
-  const uint32_t tpm = (uint32_t)g.ntile[0] * ny * nz;
-  const int mock = (int)(tile / tpm);
-  const uint32_t tl = tile - (uint32_t)mock * tpm;
-  const uint32_t tyz = tl / nz;
-  const int tzi = (int)(tl - tyz * nz);
-  const int txi = (int)(tyz / ny);
-  const int tyi = (int)(tyz - (uint32_t)txi * ny);
-  const int T0[3] = {txi * T[0], tyi * T[1], tzi * T[2]};
-  (void)ntotal;
-  {
-    // both grids are contiguous in LDS: clear them with 16-byte stores
-    uint4 *z4 = reinterpret_cast<uint4 *>(ldsq);
-    const int n4 = (int)(sizeof(AT) * gcells * (INTLACE ? 2 : 1) / 16);
-    for (int i = threadIdx.x; i < n4; i += blockDim.x) z4[i] = make_uint4(0u, 0u, 0u, 0u);
-  }
+  const int *T0 = d.T0;
+  const int mock = d.mock;
+  const float inv = k.inv;
+  clear_cells(ldsq, gcells * (INTLACE ? 2 : 1));
+  for_records(recs + k.s0, k.cnt, record_group<SCHEME>(starts, gridDim.x, flags), [&](const Rec &r) {
+    deposit_rec<SCHEME, WIDE>(ldsA, d, g, P2, wrap, false, r, k.scale);
+    if (INTLACE) deposit_rec<SCHEME, WIDE>(ldsB, d, g, P2, wrap, true, r, k.scale);
+  });
   __syncthreads();
 
-  // records past the buffer were never written (overflow flag set, the run
-  // is repeated with a larger buffer): never read beyond rec_cap
-  const uint32_t cap = rec_cap < 0xffffffffu ? (uint32_t)rec_cap : 0xffffffffu;
-  const uint32_t s0 = min(starts[tile], cap), s1 = min(starts[tile + 1], cap);
-  const uint32_t cnt = s1 > s0 ? s1 - s0 : 0u;
-  const int sexp = tile_exponent<Acc<WIDE>::TOP>(flags, cnt);
-  const float scale = ldexpf(1.f, sexp);
-  const float inv = ldexpf(1.f, -sexp);
-  // Visit the bucket in the order i -> (i * S) mod cnt with S ~ 0.618 cnt and
-  // gcd(S, cnt) = 1 (a permutation): neighbouring lanes take records far
-  // apart in fill order, i.e. far apart in the (usually space-ordered)
-  // catalogue, so their windows rarely share LDS banks.
-  // (a bucket of at most one record per thread skips the search: the gcd
-  // loop and 64-bit remainders would cost more than they save)
-  uint32_t S = 1u;
-  if (cnt > blockDim.x) {
-    S = ((uint32_t)((float)cnt * 0.618034f)) | 1u;
-    if (S >= cnt) S = 1u;
-    for (;;) {
-      uint32_t a = S, b = cnt;
-      while (b) {
-        uint32_t t = a % b;
-        a = b;
-        b = t;
-      }
-      if (a == 1u) break;
-      S += 2u;
-      if (S >= cnt) {
-        S = 1u;
-        break;
-      }
-    }
-  }
-  auto deposit_rec = [&](const Rec &r) {
-    int b[3] = {(int)(r.bxy & 0xffffu), (int)(r.bxy >> 16), (int)(r.bz & 0xffffu)};
-    const float ws = r.w * scale;
-    auto dep = [&](AT *lds, const int *bb, const float *ff) {
-      if (zpad) deposit_one<SCHEME, WIDE, true>(lds, T, T0, g.Ng, P2, bb, ff, ws);
-      else deposit_one<SCHEME, WIDE, false>(lds, T, T0, g.Ng, P2, bb, ff, ws);
-    };
-    dep(ldsA, b, r.f);
-    if (INTLACE) {
-      const uint32_t dl = r.bz >> 16;
-      int bs[3];
-      float fs[3];
+  // The tile's rows, both grids, as NZ / 2-point complex lines (cells
+  // 2n, 2n + 1 of a row), transformed like the z pass (z_r2c_kernel) and
+  // split into the half-complex row X[0..NZ/2] (k_z <= kzlim stored):
+  // X[k] = E + W^k O, X[M - k] = conj(E - W^k O).
+  using namespace pshfft;
+  using Z = ZfCfg<NZ, INTLACE>;
+  constexpr int M = NZ / 2, C = Z::C, TT = Z::T, W = SCHEME + 1;
+  using LZ = Lds<M, C, false>;
+  constexpr int V = max_values<M, C, TT, false>();
+  float2 v[V];
+  pass_load<M, C, TT, 0, false>(v, [&](int c, int n) -> float2 {
+    const AT *row = (c < Z::R ? ldsA + c * P2 : ldsB + (c - Z::R) * P2) + W;
+    return make_float2((float)row[2 * n] * inv, (float)row[2 * n + 1] * inv);
+  });
+  __syncthreads();   // every cell read before the exchange tile overwrites them
+  float *xl = reinterpret_cast<float *>(ldsq);
+  Passes<M, C, TT, 0, false, false, 2>::run(v, xl, g.tw);
+  constexpr int NP = M / 2 + 1;
+  constexpr int NI = (C * NP + TT - 1) / TT;
+  float rk[NI], rmk[NI];
+  store_last<M, C, TT, false>(v, [&](int c, int n, float2 x) { xl[LZ::idx(c, n)] = x.x; });
+  __syncthreads();
 #pragma unroll
-      for (int a = 0; a < 3; a++) {
-        int d = (dl >> a) & 1;
-        bs[a] = b[a] + d;
-        if (bs[a] >= g.Ng) bs[a] -= g.Ng;
-        fs[a] = r.f[a] + 0.5f - (float)d;
-      }
-      dep(ldsB, bs, fs);
-    }
-  };
-  if (cnt <= blockDim.x) {
-    // at most one record per thread, on the fewest waves that hold them
-    // (nw = ceil(cnt / 64)): the deposit is VALU-bound, so a wave issues as
-    // many instructions for 20 live lanes as for 64, and the other waves go
-    // straight to the barrier.  Lane l of wave w < nw takes record l * nw + w
-    // (a bijection of [0, 64 nw)), so a wave's lanes hold records nw apart
-    // in fill order rather than neighbours.
-    const uint32_t nw = (cnt + 63u) >> 6, w = threadIdx.x >> 6;
-    const uint32_t j = (threadIdx.x & 63u) * nw + w;
-    if (w < nw && j < cnt) deposit_rec(recs[s0 + j]);
-  } else {
-    uint32_t x = (uint32_t)(((uint64_t)threadIdx.x * S) % cnt);
-    const uint32_t D = (uint32_t)(((uint64_t)blockDim.x * S) % cnt);
-    for (uint32_t i = threadIdx.x; i < cnt; i += blockDim.x) {
-      const Rec r = recs[s0 + x];
-      x += D;
-      if (x >= cnt) x -= cnt;
-      deposit_rec(r);
+  for (int it = 0; it < NI; it++) {
+    const int item = threadIdx.x + it * TT;
+    const int c = item / NP, k = item - c * NP;
+    if (item < C * NP) {
+      rk[it] = xl[LZ::idx(c, k)];
+      rmk[it] = xl[LZ::idx(c, mirror<M>(k))];
     }
   }
   __syncthreads();
-
-  if constexpr (NZ > 0) {
-    // The tile's rows, both grids, as NZ / 2-point complex lines (cells
-    // 2n, 2n + 1 of a row), transformed like the z pass (z_r2c_kernel) and
-    // split into the half-complex row X[0..NZ/2] (k_z <= kzlim stored):
-    // X[k] = E + W^k O, X[M - k] = conj(E - W^k O).
-    using namespace pshfft;
-    using Z = ZfCfg<NZ, INTLACE>;
-    constexpr int M = NZ / 2, C = Z::C, TT = Z::T, W = SCHEME + 1;
-    using LZ = Lds<M, C, false>;
-    constexpr int V = max_values<M, C, TT, false>();
-    float2 v[V];
-    pass_load<M, C, TT, 0, false>(v, [&](int c, int n) -> float2 {
-      const AT *row = (c < Z::R ? ldsA + c * P2 : ldsB + (c - Z::R) * P2) + W;
-      return make_float2((float)row[2 * n] * inv, (float)row[2 * n + 1] * inv);
-    });
-    __syncthreads();   // every cell read before the exchange tile overwrites them
-    float *xl = reinterpret_cast<float *>(ldsq);
-    Passes<M, C, TT, 0, false, false, 2>::run(v, xl, g.tw);
-    constexpr int NP = M / 2 + 1;
-    constexpr int NI = (C * NP + TT - 1) / TT;
-    float rk[NI], rmk[NI];
-    store_last<M, C, TT, false>(v, [&](int c, int n, float2 x) { xl[LZ::idx(c, n)] = x.x; });
-    __syncthreads();
+  store_last<M, C, TT, false>(v, [&](int c, int n, float2 x) { xl[LZ::idx(c, n)] = x.y; });
+  __syncthreads();
+  float2 *cA = reinterpret_cast<float2 *>(meshA + (size_t)mock * mstride);
+  float2 *cB = INTLACE ? reinterpret_cast<float2 *>(meshB + (size_t)mock * mstride) : nullptr;
+  const int H = g.row_pitch / 2;
 #pragma unroll
-    for (int it = 0; it < NI; it++) {
-      const int item = threadIdx.x + it * TT;
-      const int c = item / NP, k = item - c * NP;
-      if (item < C * NP) {
-        rk[it] = xl[LZ::idx(c, k)];
-        rmk[it] = xl[LZ::idx(c, mirror<M>(k))];
-      }
-    }
-    __syncthreads();
-    store_last<M, C, TT, false>(v, [&](int c, int n, float2 x) { xl[LZ::idx(c, n)] = x.y; });
-    __syncthreads();
-    float2 *cA = reinterpret_cast<float2 *>(meshA + (size_t)mock * mstride);
-    float2 *cB = INTLACE ? reinterpret_cast<float2 *>(meshB + (size_t)mock * mstride) : nullptr;
-    const int H = g.row_pitch / 2;
-#pragma unroll
-    for (int it = 0; it < NI; it++) {
-      const int item = threadIdx.x + it * TT;
-      const int c = item / NP, k = item - c * NP;
-      if (item >= C * NP) continue;
-      const float ik = xl[LZ::idx(c, k)];
-      const float imk = xl[LZ::idx(c, mirror<M>(k))];
-      const float2 E = make_float2(0.5f * (rk[it] + rmk[it]), 0.5f * (ik - imk));
-      const float2 O = make_float2(0.5f * (ik + imk), -0.5f * (rk[it] - rmk[it]));
-      const float2 WO = cmul(g.tw[k], O);
-      const int grid = c / Z::R, row = c - grid * Z::R;
-      const int lx = row / Z::TY, ly = row - lx * Z::TY;
-      float2 *orow = (grid ? cB : cA) + ((size_t)(T0[0] + lx) * g.Ng + (T0[1] + ly)) * H;
-      if (k <= g.kzlim) mesh_store<NT>(orow + k, cadd(E, WO));
-      if (M - k != k && M - k <= g.kzlim) {
-        const float2 d = csub(E, WO);
-        mesh_store<NT>(orow + (M - k), make_float2(d.x, -d.y));
-      }
-    }
-    return;
-  }
-
-  // write the tile: rows of T[2] floats along z, 4 cells per thread
-  float *outA = meshA + (size_t)mock * mstride;
-  float *outB = INTLACE ? meshB + (size_t)mock * mstride : nullptr;
-  const int nrow = T[0] * T[1];
-  const int q4s = g.tile_shift[2] - 2;   // T[2] = 4 * 2^q4s (T[2] >= 4)
-  const int q4 = 1 << q4s;
-  for (int i = threadIdx.x; i < nrow * q4; i += blockDim.x) {
-    const int row = i >> q4s, q = i & (q4 - 1);
-    const int lx = row >> g.tile_shift[1], ly = row & (T[1] - 1);
-    const size_t gidx = ((size_t)(T0[0] + lx) * g.Ng + (T0[1] + ly)) * g.row_pitch +
-                        T0[2] + 4 * q;
-    const int li = row * P2 + SCHEME + 1 + 4 * q;
-    float4 va;
-    va.x = (float)ldsA[li] * inv;
-    va.y = (float)ldsA[li + 1] * inv;
-    va.z = (float)ldsA[li + 2] * inv;
-    va.w = (float)ldsA[li + 3] * inv;
-    store4<NT>(outA + gidx, va);
-    if (INTLACE) {
-      float4 vb;
-      vb.x = (float)ldsB[li] * inv;
-      vb.y = (float)ldsB[li + 1] * inv;
-      vb.z = (float)ldsB[li + 2] * inv;
-      vb.w = (float)ldsB[li + 3] * inv;
-      store4<NT>(outB + gidx, vb);
+  for (int it = 0; it < NI; it++) {
+    const int item = threadIdx.x + it * TT;
+    const int c = item / NP, k = item - c * NP;
+    if (item >= C * NP) continue;
+    const float ik = xl[LZ::idx(c, k)];
+    const float imk = xl[LZ::idx(c, mirror<M>(k))];
+    const float2 E = make_float2(0.5f * (rk[it] + rmk[it]), 0.5f * (ik - imk));
+    const float2 O = make_float2(0.5f * (ik + imk), -0.5f * (rk[it] - rmk[it]));
+    const float2 WO = cmul(g.tw[k], O);
+    const int grid = c / Z::R, row = c - grid * Z::R;
+    const int lx = row / Z::TY, ly = row - lx * Z::TY;
+    float2 *orow = (grid ? cB : cA) + ((size_t)(T0[0] + lx) * g.Ng + (T0[1] + ly)) * H;
+    if (k <= g.kzlim) mesh_store<NT>(orow + k, cadd(E, WO));
+    if (M - k != k && M - k <= g.kzlim) {
+      const float2 d = csub(E, WO);
+      mesh_store<NT>(orow + (M - k), make_float2(d.x, -d.y));
     }
   }
 }
@@ -1099,62 +1232,78 @@ template <int SCHEME>
 hipError_t launch_deposit(const PshAssignGeom &g, size_t ntiles,
                           const uint32_t *starts, const Rec *recs,
                           size_t rec_cap, float *meshA, float *meshB,
-                          size_t mstride, const int *flags, size_t ntotal,
-                          hipStream_t s) {
-  const size_t lds = (g.wide ? sizeof(long long) : sizeof(int)) *
-                     psh_tile_cells(g.tile, SCHEME) * (g.intlace ? 2 : 1);
-  if (lds > 160 * 1024) return hipErrorInvalidValue;
+                          size_t mstride, const int *flags, hipStream_t s) {
+  // one grid per workgroup, except where the z transform is fused in
+  const size_t cell = g.wide ? sizeof(long long) : sizeof(int);
+  size_t cells = psh_tile_cells(g.tile, SCHEME) * (g.intlace && g.zfuse ? 2 : 1);
+  // rows whose cells start on 16 bytes: a pitch of whole quads and `lead`
+  // cells before the first, where the LDS holds them (the write-out then
+  // reads quads: word by word, a wave's lanes stride 16 bytes and meet
+  // four-fold in the banks)
+  constexpr int W = SCHEME + 1;
+  int pitch = psh_tile_pitch(g.tile[2], SCHEME), lead = 0;
+  const size_t quads = (size_t)g.tile[0] * g.tile[1] * ((pitch + 3) & ~3) + 4;
+  if (!g.zfuse && cell * quads <= 160 * 1024) {
+    pitch = (pitch + 3) & ~3;
+    lead = (4 - W % 4) % 4;
+    cells = quads;
+  }
+  const size_t lds = cell * cells;
   // non-temporal mesh stores when the launch's meshes outgrow the 256 MB
   // Infinity Cache (every cell is written once and read by the next pass
   // only after the whole launch)
   const bool stream = sizeof(float) * (size_t)g.tile[0] * g.tile[1] * g.tile[2] * ntiles *
                           (g.intlace ? 2 : 1) >
                       ((size_t)256 << 20);
-  auto k = stream
-               ? (g.wide ? (g.intlace ? assign_deposit<SCHEME, true, true, true, 0>
-                                      : assign_deposit<SCHEME, false, true, true, 0>)
-                         : (g.intlace ? assign_deposit<SCHEME, true, false, true, 0>
-                                      : assign_deposit<SCHEME, false, false, true, 0>))
-               : (g.wide ? (g.intlace ? assign_deposit<SCHEME, true, true, false, 0>
-                                      : assign_deposit<SCHEME, false, true, false, 0>)
-                         : (g.intlace ? assign_deposit<SCHEME, true, false, false, 0>
-                                      : assign_deposit<SCHEME, false, false, false, 0>));
+  if (lds > 160 * 1024) return hipErrorInvalidValue;
+  auto raise = [&](const void *k) {
+    if (lds > 64 * 1024)
+      (void)hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  };
   if (g.zfuse) {
     // the fused z transform writes half-complex rows, 8 B per stored mode
-    auto pick = [&](auto nz) {
+    auto go = [&](auto nz) {
       constexpr int NZ = decltype(nz)::value;
-      constexpr bool W = ZfCfg<NZ, true>::WIDE;
+      constexpr bool WD = ZfCfg<NZ, true>::WIDE;
       const int tx = g.intlace ? ZfCfg<NZ, true>::TX : ZfCfg<NZ, false>::TX;
       const int ty = g.intlace ? ZfCfg<NZ, true>::TY : ZfCfg<NZ, false>::TY;
-      if (g.tile[0] != tx || g.tile[1] != ty || g.tile[2] != NZ || (g.wide != 0) != W) {
-        k = nullptr;
-        return;
-      }
-      k = stream ? (g.intlace ? assign_deposit<SCHEME, true, W, true, NZ>
-                              : assign_deposit<SCHEME, false, W, true, NZ>)
-                 : (g.intlace ? assign_deposit<SCHEME, true, W, false, NZ>
-                              : assign_deposit<SCHEME, false, W, false, NZ>);
+      if (g.tile[0] != tx || g.tile[1] != ty || g.tile[2] != NZ || (g.wide != 0) != WD)
+        return hipErrorInvalidValue;
+      auto k = stream ? (g.intlace ? assign_deposit_z<SCHEME, true, WD, true, NZ>
+                                   : assign_deposit_z<SCHEME, false, WD, true, NZ>)
+                      : (g.intlace ? assign_deposit_z<SCHEME, true, WD, false, NZ>
+                                   : assign_deposit_z<SCHEME, false, WD, false, NZ>);
+      raise((const void *)k);
+      hipLaunchKernelGGL(k, dim3((unsigned)ntiles), dim3(1024), lds, s, g, starts, recs, rec_cap,
+                         meshA, meshB, mstride, flags);
+      return hipGetLastError();
     };
     switch (g.Ng) {
-      case 128: pick(std::integral_constant<int, 128>{}); break;
-      case 256: pick(std::integral_constant<int, 256>{}); break;
-      case 512: pick(std::integral_constant<int, 512>{}); break;
-      case 1024: pick(std::integral_constant<int, 1024>{}); break;
-      default: k = nullptr;
+      case 128: return go(std::integral_constant<int, 128>{});
+      case 256: return go(std::integral_constant<int, 256>{});
+      case 512: return go(std::integral_constant<int, 512>{});
+      case 1024: return go(std::integral_constant<int, 1024>{});
+      default: return hipErrorInvalidValue;
     }
-    if (!k) return hipErrorInvalidValue;
   }
-  if (lds > 64 * 1024)
-    (void)hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              (int)lds);
-  // one thread per 16 cells, 256..1024: a large tile fills its CU alone (its
-  // LDS admits no second workgroup), so it brings its own waves
+  auto k = stream ? (g.wide ? (g.intlace ? assign_deposit<SCHEME, true, true, true>
+                                         : assign_deposit<SCHEME, false, true, true>)
+                            : (g.intlace ? assign_deposit<SCHEME, true, false, true>
+                                         : assign_deposit<SCHEME, false, false, true>))
+                  : (g.wide ? (g.intlace ? assign_deposit<SCHEME, true, true, false>
+                                         : assign_deposit<SCHEME, false, true, false>)
+                            : (g.intlace ? assign_deposit<SCHEME, true, false, false>
+                                         : assign_deposit<SCHEME, false, false, false>));
+  raise((const void *)k);
+  // one thread per 16 cells (per 8 of 64 bits, whose LDS admits half the
+  // workgroups: survey, N = 512, 1.89 -> 1.64 ms), 256..1024
   const size_t tcells = (size_t)g.tile[0] * g.tile[1] * g.tile[2];
+  const size_t per = g.wide ? 8 : 16;
   unsigned threads = 256;
-  while (threads < 1024 && threads * 16 < tcells) threads *= 2;
-  if (g.zfuse) threads = 1024;   // the fused transform's block shape
-  hipLaunchKernelGGL(k, dim3((unsigned)ntiles), dim3(threads), lds, s, g, starts, recs, rec_cap,
-                     meshA, meshB, mstride, flags, ntotal);
+  while (threads < 1024 && threads * per < tcells) threads *= 2;
+  hipLaunchKernelGGL(k, dim3((unsigned)(ntiles * (g.intlace ? 2 : 1))), dim3(threads), lds, s, g,
+                     starts, recs, rec_cap, meshA, meshB, mstride, flags, pitch, lead, (int)cells,
+                     (uint32_t)ntiles);
   return hipGetLastError();
 }
 
@@ -1276,9 +1425,9 @@ hipError_t psh_assign_run(const PshAssignGeom &g, PshDevPart *d_parts, const Psh
   if ((e = bucket(true)) != hipSuccess) return e;
   if (ev_deposit) (void)hipEventRecord(ev_deposit, s);
   switch (g.scheme) {
-    case 0: return launch_deposit<0>(g, ntiles, starts, recs, rec_cap, meshA, meshB, mstride, d_flags, ntotal, s);
-    case 1: return launch_deposit<1>(g, ntiles, starts, recs, rec_cap, meshA, meshB, mstride, d_flags, ntotal, s);
-    case 2: return launch_deposit<2>(g, ntiles, starts, recs, rec_cap, meshA, meshB, mstride, d_flags, ntotal, s);
-    default: return launch_deposit<3>(g, ntiles, starts, recs, rec_cap, meshA, meshB, mstride, d_flags, ntotal, s);
+    case 0: return launch_deposit<0>(g, ntiles, starts, recs, rec_cap, meshA, meshB, mstride, d_flags, s);
+    case 1: return launch_deposit<1>(g, ntiles, starts, recs, rec_cap, meshA, meshB, mstride, d_flags, s);
+    case 2: return launch_deposit<2>(g, ntiles, starts, recs, rec_cap, meshA, meshB, mstride, d_flags, s);
+    default: return launch_deposit<3>(g, ntiles, starts, recs, rec_cap, meshA, meshB, mstride, d_flags, s);
   }
 }

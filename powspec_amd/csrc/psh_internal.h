@@ -125,8 +125,9 @@ size_t psh_assign_scan_bytes(size_t ntiles);
 // (meshA) and shifted (meshB, interlacing only) meshes of nmock mocks; mock
 // m's meshes start at meshA + m*mstride, meshB + m*mstride.
 // counts, starts (ntiles+1), cursors: uint32 scratch; records: rec_cap
-// records; flags (4 words, cleared first): bit 0 record overflow, bit 1
-// inconsistent shifted base, bit 2 coordinate outside the box.  The part
+// records; flags (4 words, cleared first): [0] bit 0 record overflow, bit 1
+// inconsistent shifted base, bit 2 coordinate outside the box; [1] the largest
+// |weight|; [2] the number of ranges that fill the buckets.  The part
 // table is written to d_parts from h_parts (nullptr: it is there already, as
 // a captured run needs it).
 hipError_t psh_assign_run(const PshAssignGeom &g, PshDevPart *d_parts,

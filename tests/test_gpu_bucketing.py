@@ -93,3 +93,22 @@ def test_record_overflow_reruns(psh, oracle):
             got = (ctx.run_device(dev, n, float(n)) if graph is None else
                    ctx.run_batch(dev, [0, n], [float(n)], graph=graph)[0])
             _check(got, ref, [0, 2, 4], ref["shot"][0])
+
+
+@pytest.mark.parametrize("scheme,tile,n", [
+    (2, (32, 32, 32), 50000),    # rows of whole quads would not fit the LDS
+    (1, (8, 16, 32), 600000),    # many records per thread, aligned rows
+    (0, (4, 4, 64), 60000),      # one tile spans z, odd row offset
+    (3, (64, 4, 4), 60000),      # one tile spans x
+])
+@pytest.mark.parametrize("order", ["sorted", "shuffled"])
+def test_deposit_tiles(psh, oracle, scheme, tile, n, order):
+    d = _catalogue(n, 64, 7, False)
+    if order == "shuffled":
+        d = d[np.random.default_rng(2).permutation(n)]
+    kw = dict(gsize=64, assign=scheme, intlace=False, bsize=L, kbin=0.02, poles=[0, 2, 4])
+    ctx = psh.Context(psh.make_conf(**kw))
+    ctx.set_tiles(tile)
+    got = ctx.run_device(psh.DeviceArray.from_numpy(d), n, float(d[:, 3].sum()))
+    ref = oracle.run(oracle.make_conf(**kw), [d])
+    _check(got, ref, [0, 2, 4], ref["shot"][0])
