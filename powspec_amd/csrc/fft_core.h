@@ -464,17 +464,36 @@ __device__ __forceinline__ void store_last(const float2 *v, ST st) {
 // (r, c, j): with r a compile-time constant after unrolling, a caller forms
 // the address as a per-tile uniform row base (r) plus one per-lane offset
 // (c, j) shared by all values of the thread, which keeps 64-bit addresses
-// out of the registers.
+// out of the registers.  Lengths 3 2^a and 5 2^a leave some threads without
+// a butterfly: one branch around a butterfly's loads keeps them all in flight
+// (a branch per value waited for each: the y pass of both N = 640 fields took
+// 1070 us instead of 830).
 template <int N, int C, int T, bool COLMAP, class LD, int PL = 0>
 __device__ __forceinline__ void pass_load_rows(float2 *v, LD ld) {
   using G = PassGeom<N, C, T, 0, COLMAP, PL>;
 #pragma unroll
   for (int q = 0; q < G::NB; q++) {
     int c, j;
-    const bool ok = G::map(q, c, j);
+    if (G::map(q, c, j)) {
 #pragma unroll
-    for (int r = 0; r < G::R; r++)
-      v[q * G::R + r] = ok ? ld(r, c, j) : make_float2(0.f, 0.f);
+      for (int r = 0; r < G::R; r++) v[q * G::R + r] = ld(r, c, j);
+    } else {
+#pragma unroll
+      for (int r = 0; r < G::R; r++) v[q * G::R + r] = make_float2(0.f, 0.f);
+    }
+  }
+}
+
+// Where pass_load_rows branched: the values as they are after the branch.
+// Without it the compiler folds arithmetic on the idle threads' zeros into
+// the branch, away from the products it otherwise fuses with, and the last
+// bits of the transform depend on the shape of the code around it.
+template <int N, int C, int T, bool COLMAP, int PL = 0>
+__device__ __forceinline__ void settle_rows(float2 *v) {
+  using G = PassGeom<N, C, T, 0, COLMAP, PL>;
+  if constexpr (G::NBT % T != 0) {
+#pragma unroll
+    for (int i = 0; i < G::NB * G::R; i++) asm("" : "+v"(v[i].x), "+v"(v[i].y));
   }
 }
 
@@ -482,33 +501,8 @@ template <int N, int C, int T, bool COLMAP, bool INV, int TWS, class LD, int PL 
 __device__ __forceinline__ void transform_rows(float2 *v, float *lds,
                                                const float2 *__restrict__ tw, LD ld) {
   pass_load_rows<N, C, T, COLMAP, LD, PL>(v, ld);
+  settle_rows<N, C, T, COLMAP, PL>(v);
   Passes<N, C, T, 0, COLMAP, INV, TWS, PL>::run(v, lds, tw);
-}
-
-// Two fields of the same tile advanced pass by pass together (each exchanged
-// through the same LDS buffer in turn), so that neither sits finished in
-// registers while the other is transformed.
-template <int N, int C, int T, int P, bool COLMAP, bool INV, int TWS>
-struct Passes2 {
-  __device__ static __forceinline__ void run(float2 *va, float2 *vb, float *lds,
-                                             const float2 *__restrict__ tw) {
-    pass_compute<N, C, T, P, COLMAP, INV, TWS>(va, tw);
-    pass_compute<N, C, T, P, COLMAP, INV, TWS>(vb, tw);
-    if constexpr (P + 1 < npasses(N)) {
-      exchange<N, C, T, P, COLMAP>(va, lds);
-      exchange<N, C, T, P, COLMAP>(vb, lds);
-      Passes2<N, C, T, P + 1, COLMAP, INV, TWS>::run(va, vb, lds, tw);
-    }
-  }
-};
-
-template <int N, int C, int T, bool COLMAP, bool INV, int TWS, class LDA, class LDB>
-__device__ __forceinline__ void transform_rows2(float2 *va, float2 *vb, float *lds,
-                                                const float2 *__restrict__ tw, LDA lda,
-                                                LDB ldb) {
-  pass_load_rows<N, C, T, COLMAP>(va, lda);
-  pass_load_rows<N, C, T, COLMAP>(vb, ldb);
-  Passes2<N, C, T, 0, COLMAP, INV, TWS>::run(va, vb, lds, tw);
 }
 
 // Natural-order outputs of the last pass: element j + r*NS of line c.

@@ -470,13 +470,12 @@ col_kernel(const float2 *__restrict__ in, float2 *__restrict__ out, int ntz,
   // columns q*C + c < H always lie inside the padded row (the row holds
   // M + 1 + 15 columns, so a tile of C columns starting at or before M ends
   // inside it when C <= 16; 32-column tiles are clipped below); those past
-  // kz = M are read and discarded
+  // kz = M are read, transformed (a column never meets another) and not stored
   float2 v[V];
   auto ld = [&](int r, int c, int j) -> float2 {
     if (C > 16 && q * C + c >= M + 1 + 15) return make_float2(0.f, 0.f);
-    const float2 x = mesh_load<NT>(row_elem<RS::BYTE32>(in + base + (size_t)(r * RS::LOAD) * ES,
-                                                         (uint32_t)j * (uint32_t)ES + c));
-    return c < ncv ? x : make_float2(0.f, 0.f);
+    return mesh_load<NT>(row_elem<RS::BYTE32>(in + base + (size_t)(r * RS::LOAD) * ES,
+                                              (uint32_t)j * (uint32_t)ES + c));
   };
   transform_rows<N, C, T, true, INV, 1, decltype(ld), PL>(v, lds, tw, ld);
   // outputs k_y = i' (i = j + r STORE) past the column's live bound are
@@ -526,6 +525,7 @@ struct XBinDev {
   float legc[PSH_MAX_NL][4];
   int oddmask;
   int even024;   // the poles are exactly 0, 2, 4 (the common request)
+  float nmuf;    // (float)bins.nmu
   const int *ylive;   // per k_z tile, the largest |k_y| with binned modes, or nullptr
 };
 
@@ -543,14 +543,13 @@ __device__ __forceinline__ int mode_bin(double kmod2, const PshBins &b,
 
 // x pass: up to 1024 threads (16 waves, 128 VGPRs).  The plain kernel takes
 // 16-column tiles (128-byte row segments) and 16 values per thread.  The
-// interlaced kernel transforms both fields pass by pass together, also in
-// 16-column tiles up to N = 1024 (16 values per thread and field there; the
-// register limit spills a few values outside the butterflies, which costs
-// far less than the 50 % of extra HBM reads of 8-column tiles: 5.05 -> 4.25
-// ms at N = 1024); at N = 2048 8 columns (64-byte half lines, completed by
-// the neighbouring tile on the same XCD, see xcd_tile).  With T a multiple of
-// C, a thread works on the same column (kz) in every pass and in the binning
-// loop.
+// interlaced kernel transforms the two fields one after the other, also in
+// 16-column tiles up to N = 1024 (16 values per thread and field there, 14
+// of them spilled, which costs far less than the 50 % of extra HBM reads of
+// 8-column tiles: 5.05 -> 4.25 ms when they were introduced); at N = 2048 8
+// columns (64-byte half lines, completed by the neighbouring tile on the same
+// XCD, see xcd_tile).  With T a multiple of C, a thread works on the same
+// column (kz) in every pass and in the binning loop.
 template <int N, bool IL>
 struct XCfg {
   static constexpr int C = N <= 1024 ? 16 : 8;
@@ -566,20 +565,18 @@ struct XCfg {
   // workgroups share a CU and hide each other's barriers; the small
   // interlaced kernel holds 2 x 16 values per thread and gets 2 (256 VGPRs)
   static constexpr int WAVES = SMALL ? 2 : 4;
-  // the next tile's rows loaded during phase 2 (see x_bin_kernel): 2 every
-  // field, 1 the first field only (the second loads when the tile starts),
-  // 0 none.  The interlaced kernel from N = 640 holds both fields' 16 values
-  // per thread and spills registers when both prefetches are in flight as
-  // well (measured on MI355X at N = 1024: 4.31 ms with both, 4.00 ms with
-  // the first field's, 3.46 ms without)
-  static constexpr int PREFETCH = (IL && N >= 640) ? 0 : 2;
+  // the next tile's rows loaded during phase 2 (see x_bin_kernel).  Where the
+  // interlaced kernel holds 16 values per thread and field (N = 1024,
+  // 2048) the rows in flight spill; measured on MI355X with / without:
+  // N = 1024 3.14 / 3.02 ms, N = 768 1.46 / 1.56 ms, N = 640 1.33 / 1.47 ms.
+  static constexpr bool PREFETCH = !(IL && !SMALL && C * N >= 16 * T);
   static_assert(T % C == 0, "a thread keeps one column");
 };
 
 // LDS of the x pass besides the bins: the tile maximum, ksq_x (FP64; read
-// from global memory by the GS layout), xtab, twiddles, exchange tile.  The twiddles are read from LDS: read from global memory
-// they are invariant over the persistent tile loop and stay live in
-// registers.
+// from global memory by the GS layout), xtab, twiddles, exchange tile.  The
+// twiddles are read from LDS: read from global memory they are invariant over
+// the persistent tile loop and stay live in registers.
 template <int N, bool IL, bool GS = false>
 constexpr size_t xbin_static_lds() {
   return sizeof(double) * 2 + (GS ? 0 : sizeof(double) * N) + sizeof(float4) * N +
@@ -606,18 +603,27 @@ __device__ __forceinline__ void acc_fixed(long long *ib, float x, double sdown) 
   atomicAdd(reinterpret_cast<unsigned long long *>(ib), (unsigned long long)q);
 }
 
-// Bin of a mode from its FP32 |k|, kmodf: -1 outside the bins, -2 when
-// undecided.  t = (|k| - kedge0) / dk evaluated in FP32 errs by less than
-// 2e-6 (|t| + kedge0/dk + 8), so when t lies farther than that from an
-// integer, floor(t) is the bin the FP64 expression gives.  Log bins are
-// always undecided.
-__device__ __forceinline__ int bin_fast(const PshBins &b, float kmodf) {
-  const float tf = (kmodf - b.kedge0f) * b.invdkf;
+// Bin of a mode from its FP32 |k|^2 and |k|, k2f and kmodf: -1 outside the
+// bins, -2 when undecided.  t = (q - kedge0) / dk with q = |k| or, for log
+// bins, log10 |k| = log2(|k|^2) log10(2) / 2, evaluated in FP32, errs by less
+// than 2e-6 (|t| + kedge0/dk + 8), so when t lies farther than that from an
+// integer, floor(t) is the bin the FP64 expression gives.  The logarithm adds
+// its own error: one ulp of log2 and 4e-7 of |k|^2 are less than
+// 4e-6 (|q| + 1) in q.  (k = 0 gives -inf and so no decision.)
+// Log bins used to take one FP64 logarithm per mode pair.
+__device__ __forceinline__ int bin_fast(const PshBins &b, float k2f, float kmodf) {
+  float q = kmodf, eps = 0.f;
+  if (b.logscale) {
+    q = 0.150514998f * __builtin_amdgcn_logf(k2f);
+    eps = 4e-6f * (fabsf(q) + 1.f) * b.invdkf;
+  }
+  const float tf = (q - b.kedge0f) * b.invdkf;
   const float fl = floorf(tf);
   const float fr = tf - fl;
-  const float eps = 2e-6f * (fabsf(tf) + b.k0dk + 8.f);
-  if (b.logscale || !(fr > eps && fr < 1.f - eps)) return -2;
-  return (fl >= 0.f && fl < (float)b.nbin) ? (int)fl : -1;
+  eps += 2e-6f * (fabsf(tf) + b.k0dk + 8.f);
+  if (!(fr > eps && fr < 1.f - eps)) return -2;
+  const int kb = (int)fl;   // saturates
+  return (unsigned)kb < (unsigned)b.nbin ? kb : -1;
 }
 
 // The FP64 bin of the reference: |k|^2 = (ksq_x + ksq_y) + ksq_z with ksq_z
@@ -631,6 +637,16 @@ __device__ __forceinline__ int bin_exact(const PshBins &b, double ksqx, double k
   return mode_bin(kmod2, b, kmod);
 }
 
+// What bounds it: up to N = 640 the row reads, from N = 768 on the transforms'
+// LDS exchanges and instructions as well (N = 1024, interlaced, 5.2 GB of live
+// rows: 1.4 ms without the transforms and the binning, the transforms add
+// 1.2 ms, the binning 0.4).  Rows prefetched through the whole of phase 2
+// (nothing in it waits on memory: tables from LDS or scalar loads, no select
+// on a loaded value) and binning without address arithmetic or FP64 took,
+// on MI355X, start of the tuning -> now: plain 256^3 47 -> 33 us, interlaced
+// 640^3 log bins 1.72 -> 1.34 ms, 1024^3 3.40 -> 3.02 ms, 32 interlaced 256^3
+// 1.31 -> 1.14 ms, alias-corrected 512^3 with |mu| cells 343 -> 257 us.
+//
 // Forward x transform of one (y, kz-tile) column tile fused with the
 // interlace combine and the binning of its modes.  Two phases per tile:
 //  1. (registers, unrolled) F = (F_A + e^{i pi (i'+j'+k)/N} F_B) / 2
@@ -650,7 +666,10 @@ __device__ __forceinline__ int bin_exact(const PshBins &b, double ksqx, double k
 // GS: the workgroup's FP64 sums live in its row of the partials and ksq_x
 // is read from global memory, which halves the LDS (two workgroups per CU
 // for the plain pass with |mu| cells).
-template <int N, int EPI, bool INTLACE, bool NT, bool GS>
+// GEN (boxes): any set of poles and line of sight; without it the poles are
+// 0, 2, 4 and the line of sight has no x component, so both modes of a pair
+// share every weight.
+template <int N, int EPI, bool INTLACE, bool NT, bool GS, bool GEN>
 __global__ void __launch_bounds__((XCfg<N, INTLACE>::T), (XCfg<N, INTLACE>::WAVES))
 x_bin_kernel(XBinDev a, int ntz, int H, const float2 *__restrict__ tw) {
   constexpr int C = XCfg<N, INTLACE>::C, T = XCfg<N, INTLACE>::T, M = N / 2;
@@ -676,7 +695,10 @@ x_bin_kernel(XBinDev a, int ntz, int H, const float2 *__restrict__ tw) {
   double *out = a.partials + ((size_t)mock * gridDim.x + blockIdx.x) * a.nacc_full;
   const int nmu_o = EPI == PSH_EPI_SIM ? b.nmu : 1;
   const int stride_o = a.nbw * nmu_o;
+  const bool all_bins = a.nbw == b.nbin;   // one window: the layouts agree
+  typedef __attribute__((address_space(1))) double gdouble;
   auto out_idx = [&](int i) -> size_t {
+    if (all_bins) return (size_t)i;
     const int l = i / stride_o;
     return (size_t)(l * b.nbin + a.kb0) * nmu_o + (i - l * stride_o);
   };
@@ -692,7 +714,7 @@ x_bin_kernel(XBinDev a, int ntz, int H, const float2 *__restrict__ tw) {
     if (!GS) ksqx[i] = a.ax.ksq[0][i];
     twl[i] = tw[i];
   }
-  if (EPI == PSH_EPI_SIM && threadIdx.x < PSH_MAX_NL) {
+  if (EPI == PSH_EPI_SIM && GEN && threadIdx.x < PSH_MAX_NL) {
     const int l = threadIdx.x;
     legl[l] = make_float4(a.legc[l][0], a.legc[l][1], a.legc[l][2], a.legc[l][3]);
   }
@@ -703,47 +725,53 @@ x_bin_kernel(XBinDev a, int ntz, int H, const float2 *__restrict__ tw) {
   using RS = RowSplit<N, C, T, true>;
   static_assert(G::NS == RS::STORE, "phase 1 walks the last pass outputs");
   static_assert(PSH_PAD == 16 && RS::XSPAN < (1ull << 32), "lane offsets are 32-bit");
-  const size_t ntiles = (size_t)N * ntz;
-  const size_t t0 = xcd_tile(blockIdx.x, gridDim.x);
-  // tile -> (y, kz block q); rows of the block start at base
-  auto tile_base = [&](size_t t, int &y, int &q) -> size_t {
-    y = (int)(t / ntz);
-    q = (int)(t - (size_t)y * ntz);
+  // Tiles (y, kz block q), q fastest, every gridDim.x-th one: stepped by
+  // additions (a division per tile, 64-bit at that, stood between a tile and
+  // its first load).  Rows of a tile start at tile_base.
+  const int dy = (int)(gridDim.x / (unsigned)ntz), dq = (int)(gridDim.x % (unsigned)ntz);
+  auto advance = [&](int &y, int &q) {
+    y += dy;
+    q += dq;
+    if (q >= ntz) {
+      q -= ntz;
+      y++;
+    }
+  };
+  auto tile_base = [&](int y, int q) -> size_t {
     return mock * a.mstride_c + (size_t)y * H + (size_t)q * C;
   };
   // columns q*C + c < H always lie inside the padded row; those past
-  // kz = M are read and discarded
-  auto ld_field = [&](const float2 *f, size_t base, int ncv) {
+  // kz = M are read and transformed like the others (a column never meets
+  // another) and left out of phase 1.  They are not masked here: a select on
+  // a loaded value waits for it, and the prefetch with it.
+  auto ld_field = [&](const float2 *f, size_t base) {
     return [=](int r, int cc, int j) -> float2 {
-      const float2 x = mesh_load<NT>(
+      return mesh_load<NT>(
           row_elem<RS::BYTE32>(f + base + (size_t)(r * RS::LOAD) * ES, (uint32_t)j * ES32 + cc));
-      return cc < ncv ? x : make_float2(0.f, 0.f);
     };
   };
   // The next tile's rows are loaded into va/vb as soon as phase 1 has
   // consumed them, so their HBM latency hides behind phase 2 (one block per
-  // CU: nothing else would overlap it) -- as far as the registers hold them
-  // (XCfg::PREFETCH: the fields not prefetched load when the tile starts).
-  constexpr int PF = XCfg<N, INTLACE>::PREFETCH;
+  // CU: nothing else would overlap it) -- where the registers hold them
+  // (XCfg::PREFETCH; otherwise they load when the tile starts).
+  constexpr bool PF = XCfg<N, INTLACE>::PREFETCH;
   float2 va[V];
   float2 vb[INTLACE ? V : 1];
-  auto load_field = [&](size_t t, bool second) {
-    int ty, tq;
-    const size_t tb = tile_base(t, ty, tq);
-    const int tn = min(C, M + 1 - tq * C);
-    if (!second) pass_load_rows<N, C, T, true>(va, ld_field(a.A, tb, tn));
-    else if (INTLACE) pass_load_rows<N, C, T, true>(vb, ld_field(a.B, tb, tn));
+  auto load_field = [&](int ty, int tq, bool second) {
+    const size_t tb = tile_base(ty, tq);
+    if (!second) pass_load_rows<N, C, T, true>(va, ld_field(a.A, tb));
+    else if (INTLACE) pass_load_rows<N, C, T, true>(vb, ld_field(a.B, tb));
   };
   // field f of a SURVEYL group (f = 0 is A)
-  auto load_group_field = [&](size_t t, int f) {
-    int ty, tq;
-    const size_t tb = tile_base(t, ty, tq);
-    const int tn = min(C, M + 1 - tq * C);
-    pass_load_rows<N, C, T, true>(va, ld_field(a.A + (size_t)f * a.fstride_c, tb, tn));
+  auto load_group_field = [&](int ty, int tq, int f) {
+    const size_t tb = tile_base(ty, tq);
+    pass_load_rows<N, C, T, true>(va, ld_field(a.A + (size_t)f * a.fstride_c, tb));
   };
-  auto prefetch = [&](size_t t) {
-    if (PF >= 1) load_field(t, false);
-    if (PF >= 2) load_field(t, true);
+  auto prefetch = [&](int ty, int tq) {
+    if (PF) {
+      load_field(ty, tq, false);
+      load_field(ty, tq, true);
+    }
   };
   // A tile whose nearest mode (k_x = 0, lowest k_z) already lies at or past
   // the last bin edge has no mode in the bins: its x transform is skipped.
@@ -752,29 +780,34 @@ x_bin_kernel(XBinDev a, int ntz, int H, const float2 *__restrict__ tw) {
   // and k_z); with k_max = k_Ny about 1 - pi/4 of the (k_y, k_z) tiles are
   // skipped.  nullptr (the survey l = 0 pass, whose stored field is
   // transformed back in full, and log bins): every tile.
-  auto live = [&](size_t t) -> bool {
+  typedef __attribute__((address_space(4))) const int cint;       // uniform tables:
+  typedef __attribute__((address_space(4))) const float cfloat;   // scalar loads
+  auto live = [&](int ty, int tq) -> bool {
     if (!a.ylive) return true;
-    int ty, tq;
-    (void)tile_base(t, ty, tq);
     const int ay = ty <= M ? ty : N - ty;
-    return ay <= a.ylive[tq];
+    return ay <= ((cint *)a.ylive)[tq];
   };
-  auto next_live = [&](size_t t) -> size_t {
-    while (t < ntiles && !live(t)) t += gridDim.x;
-    return t;
-  };
-  size_t tile = next_live(t0);
-  if (tile < ntiles) prefetch(tile);
-  for (; tile < ntiles;) {
-    int y, q;
-    const size_t base = tile_base(tile, y, q);
-    if (PF < 1) load_field(tile, false);
-    if (PF < 2) load_field(tile, true);
+  const unsigned t0 = (unsigned)xcd_tile(blockIdx.x, gridDim.x);
+  int ny = (int)(t0 / (unsigned)ntz), nq = (int)(t0 - (unsigned)ny * (unsigned)ntz);
+  while (ny < N && !live(ny, nq)) advance(ny, nq);
+  if (ny < N) prefetch(ny, nq);
+  while (ny < N) {
+    const int y = ny, q = nq;
+    const size_t base = tile_base(y, q);
+    if (!PF) {
+      load_field(y, q, false);
+      load_field(y, q, true);
+    }
     const int ncv = min(C, M + 1 - q * C);
-    if (INTLACE)
-      Passes2<N, C, T, 0, true, false, 1>::run(va, vb, lds, twl);
-    else
-      Passes<N, C, T, 0, true, false, 1>::run(va, lds, twl);
+    settle_rows<N, C, T, true>(va);
+    Passes<N, C, T, 0, true, false, 1>::run(va, lds, twl);
+    if (INTLACE) {
+      // one field after the other: a scheduler that mixes the two holds both
+      // fields' twiddles and spills
+      __builtin_amdgcn_sched_barrier(0);
+      settle_rows<N, C, T, true>(vb);
+      Passes<N, C, T, 0, true, false, 1>::run(vb, lds, twl);
+    }
     const int c = opaque_tid<T>() % C;   // the thread's column in every pass
     const bool colok = c < ncv;
     const int kz = min(q * C + c, M);
@@ -792,7 +825,8 @@ x_bin_kernel(XBinDev a, int ntz, int H, const float2 *__restrict__ tw) {
         if (f > 0) {
           // every thread has read the previous transform's last exchange
           __syncthreads();
-          load_group_field(tile, f);
+          load_group_field(y, q, f);
+          settle_rows<N, C, T, true>(va);
           Passes<N, C, T, 0, true, false, 1>::run(va, lds, twl);
         }
         const YlmPoly &yp = a.yp[f];
@@ -822,7 +856,20 @@ x_bin_kernel(XBinDev a, int ntz, int H, const float2 *__restrict__ tw) {
 
     // phase 1
     float2 pyz = make_float2(1.f, 0.f);
-    if (INTLACE) pyz = cmul(a.phase[y], a.phase[kz]);
+    // Phase, alias and |k| tables: the phases and alias factors are functions
+    // of the index alone, one table for the three axes, so those of y and k_z
+    // come from the LDS copy of the x axis.  Nothing but the next tile's rows
+    // is read from memory between here and the next tile: vector loads
+    // return in order, and a table value asked for after the prefetch would
+    // wait for it.
+    const float4 xy = xtab[y], xz = xtab[kz];
+    if (INTLACE) pyz = cmul(make_float2(xy.z, xy.w), make_float2(xz.z, xz.w));
+    const bool single = (kz == 0) || (kz == M);
+    const float wyz =
+        xy.x * xz.x * ((single ? 1.f : 2.f) * (INTLACE && EPI == PSH_EPI_SIM ? 0.25f : 1.f));
+    const float ksqyz = ((cfloat *)a.ax.ksqf[1])[y] + a.ax.ksqf[2][kz];
+    const float dyz =
+        __builtin_fmaf(((cfloat *)a.ax.kvf[1])[y], b.losf[1], a.ax.kvf[2][kz] * b.losf[2]);
     // The tile's fixed-point scale follows the contributions it sums: the
     // thread's largest |v| (the simulation's DC mode, never binned, left
     // out) times its column's weight w_yz; the largest x alias factor is in
@@ -859,8 +906,8 @@ x_bin_kernel(XBinDev a, int ntz, int H, const float2 *__restrict__ tw) {
         const int i = j + r * G::NS;
         float2 F = EPI == PSH_EPI_SURVEYL ? gsum[qq * G::R + r] : va[qq * G::R + r];
         if (INTLACE) {
-          const float4 xt = xtab[i];
-          const float2 t = cmul(cmul(make_float2(xt.z, xt.w), pyz), vb[qq * G::R + r]);
+          const float2 ph = *reinterpret_cast<const float2 *>(&xtab[i].z);
+          const float2 t = cmul(cmul(ph, pyz), vb[qq * G::R + r]);
           // the simulation epilogue takes |F_A + t|^2 and applies the
           // (1/2)^2 with the per-column weight in phase 2
           if (EPI == PSH_EPI_SIM) F = make_float2(F.x + t.x, F.y + t.y);
@@ -888,13 +935,25 @@ x_bin_kernel(XBinDev a, int ntz, int H, const float2 *__restrict__ tw) {
     }
     // largest |v| w_yz of the tile (non-negative floats order as their bits)
     if (colok) {
-      vmax *= a.ax.alf[1][y] * a.ax.alf[2][kz] * ((kz == 0 || kz == M) ? 1.f : 2.f) *
-              (INTLACE && EPI == PSH_EPI_SIM ? 0.25f : 1.f);
+      vmax *= wyz;
       if (vmax > 0.f) atomicMax(tmaxp, __float_as_uint(vmax));
     }
     __syncthreads();
-    const size_t next = next_live(tile + gridDim.x);
-    if (next < ntiles) prefetch(next);
+    do advance(ny, nq);
+    while (ny < N && !live(ny, nq));
+    if (ny < N) {
+      prefetch(ny, nq);
+    } else if (INTLACE && N >= 640) {
+      // last tile: nothing of this one's values is kept.  (Known to be dead,
+      // idle threads' butterflies sink into the branches around their stores,
+      // and other products are fused: the sizes that did not prefetch before
+      // keep the last bits they had.)
+#pragma unroll
+      for (int i = 0; i < V; i++) {
+        va[i] = make_float2(0.f, 0.f);
+        if (INTLACE) vb[INTLACE ? i : 0] = make_float2(0.f, 0.f);
+      }
+    }
 
     // phase 2: column c, pairs (i, N - i) with i = threadIdx.x / C + k T / C
     // up to M.  The tile's integer sums take the scale 2^E with
@@ -913,133 +972,182 @@ x_bin_kernel(XBinDev a, int ntz, int H, const float2 *__restrict__ tw) {
     }
     const double sdown = ldexp(1.0, -E);
     if (colok) {
-      const float ksqyz = a.ax.ksqf[1][y] + a.ax.ksqf[2][kz];
-      const float dyz = a.ax.kvf[1][y] * b.losf[1] + a.ax.kvf[2][kz] * b.losf[2];
-      const bool single = (kz == 0) || (kz == M);
-      const float wyz = a.ax.alf[1][y] * a.ax.alf[2][kz] *
-                        ((single ? 1.f : 2.f) * (INTLACE && EPI == PSH_EPI_SIM ? 0.25f : 1.f));
-      const double ksqy = a.ax.ksq[1][y], ksqz = a.ax.ksq[2][kz];
       const bool dcrow = (EPI == PSH_EPI_SIM) && y == 0 && kz == 0;
-      // the two half-spaces cancel odd poles off the kz = 0, M planes
-      const int lmask = single ? ~0 : ~a.oddmask;
-      constexpr int S = T / C;   // rows between a thread's modes
+      const int nmu = EPI == PSH_EPI_SIM ? b.nmu : 1;
+      const int stride = a.nbw * nmu;
+      constexpr int S = T / C;        // rows between a thread's modes
+      constexpr int KMAX = M / S;     // its pairs: k = 0..KMAX, i = i0 + k S <= M
       const int i0 = opaque_tid<T>() / C;
+      // A pair's operands: |v| and alias of mode i and of its partner N - i.
+      // Partners of i = 0 (none) and the Nyquist index M (itself) read a valid
+      // entry that `pair` discards.  From S = 8 on the padded LDS addresses of
+      // a thread's rows are one base and constant offsets.
+      struct Ops {
+        float ax, ks, v, vp, ap;
+      };
+      constexpr bool LIN = S % 8 == 0;
       const float *vrow = lds + L::idx(c, i0);
-      // One mode pair: its bin, weights and accumulations.  xt, v, vp, ap
-      // come from LDS, read one pair ahead by the loop below.
-      auto mode_pair = [&](int i, float4 xt, float v, float vp, float ap) {
-        const float k2f = xt.y + ksqyz;
-        const float rs = rsqrtf(k2f);
-        int kb = bin_fast(b, k2f * rs);
-        if (kb == -2) kb = bin_exact(b, GS ? a.ax.ksq[0][i] : ksqx[i], ksqy, ksqz, kz);
-        if (dcrow && i == 0) kb = -1;   // DC mode skipped
-        kb -= a.kb0;
-        if (kb < 0 || kb >= a.nbw) return;
+      // row N - i0 - KMAX S (past the tile for i0 = 0 and KMAX = 0 only)
+      const float *prow = LIN ? lds + L::idx(c, N - i0 - KMAX * S) : nullptr;
+      const float4 *xrow = xtab + i0, *xprow = xtab + (N - i0 - KMAX * S);
+      auto fetch = [&](int k) -> Ops {
+        Ops o;
+        const int i = i0 + k * S;
+        const float2 x = *reinterpret_cast<const float2 *>(xrow + k * S);
+        o.ax = x.x;
+        o.ks = x.y;
+        if (LIN) {
+          const bool none = k == 0 && i0 == 0;
+          o.v = vrow[L::off(k * S)];
+          o.vp = *(none ? vrow : prow + L::off((KMAX - k) * S));
+          o.ap = (none ? xrow : xprow + (KMAX - k) * S)->x;
+        } else {
+          const int ip = i == 0 ? 0 : N - i;
+          o.v = lds[L::idx(c, i)];
+          o.vp = lds[L::idx(c, ip)];
+          o.ap = xtab[ip].x;
+        }
+        return o;
+      };
+      // One mode pair in bin kb (relative to the window) with 1 / |k| = rs.
+      auto add_pair = [&](int i, int kb, float rs, const Ops &o) {
+        // sums of products are fused where written so: left to the compiler,
+        // the fusions, and with them the last bits, follow the code around
+#pragma clang fp contract(off)
         // the partner k_x = -i (none for i = 0 and the Nyquist index M)
         const bool pair = i != 0 && i != M;
-        if (!pair) {
-          vp = 0.f;
-          ap = 0.f;
+        const float al = o.ax * wyz;
+        const float wp = pair ? o.vp * (o.ap * wyz) : 0.f;
+        if (EPI != PSH_EPI_SIM) {   // SURVEYL's Y_lm weights are in v already
+          acc_fixed(&ibins[kb], __builtin_fmaf(o.v, al, wp), sdown);
+          return;
         }
-        const float w = v * (xt.x * wyz);
-        const float wp = vp * (ap * wyz);
-        if (EPI == PSH_EPI_SIM) {
-          const float kvx = (float)i * a.vec0f;
-          const float mu = (kvx * b.losf[0] + dyz) * rs;
-          const float mup = (-kvx * b.losf[0] + dyz) * rs;
-          // accumulator of pole slot l, bin kb and |mu| cell c:
-          // (l nbw + kb) nmu + c (nmu = 1: no cells)
-          const int nmu = b.nmu;
-          const int stride = a.nbw * nmu;
-          int cm = 0, cp = 0;
-          if (nmu > 1) {
-            cm = min((int)(fabsf(mu) * (float)nmu), nmu - 1);
-            cp = min((int)(fabsf(mup) * (float)nmu), nmu - 1);
+        const float w = o.v * al;
+        // accumulator of pole slot l, bin kb and |mu| cell c:
+        // (l nbw + kb) nmu + c (nmu = 1: no cells)
+        if (!GEN) {   // both modes of the pair share mu, and so the cell
+          const float mu = dyz * rs;
+          int base = kb;
+          if (nmu > 1) base = kb * nmu + min((int)(fabsf(mu) * a.nmuf), nmu - 1);
+          // L_0 = 1, L_2 and L_4 by Horner in mu^2
+          const float x2 = mu * mu;
+          const float p2 = __builtin_fmaf(1.5f, x2, -0.5f);
+          const float p4 = __builtin_fmaf(__builtin_fmaf(4.375f, x2, -3.75f), x2, 0.375f);
+          const float s0 = w + wp;
+          acc_fixed(&ibins[base], s0, sdown);
+          acc_fixed(&ibins[stride + base], s0 * p2, sdown);
+          acc_fixed(&ibins[2 * stride + base], s0 * p4, sdown);
+          return;
+        }
+        const float kvx = (float)i * a.vec0f;
+        const float mu = __builtin_fmaf(b.losf[0], kvx, dyz) * rs;
+        const float mup = __builtin_fmaf(-b.losf[0], kvx, dyz) * rs;
+        int cm = 0, cp = 0;
+        if (nmu > 1) {
+          cm = min((int)(fabsf(mu) * a.nmuf), nmu - 1);
+          cp = min((int)(fabsf(mup) * a.nmuf), nmu - 1);
+        }
+        const int base = kb * nmu + cm, basep = kb * nmu + cp;
+        const float x2 = mu * mu, y2 = mup * mup;
+        if (a.even024) {
+          const float p2 = __builtin_fmaf(1.5f, x2, -0.5f);
+          const float p4 = __builtin_fmaf(__builtin_fmaf(4.375f, x2, -3.75f), x2, 0.375f);
+          const float q2 = __builtin_fmaf(1.5f, y2, -0.5f);
+          const float q4 = __builtin_fmaf(__builtin_fmaf(4.375f, y2, -3.75f), y2, 0.375f);
+          if (cm == cp) {
+            acc_fixed(&ibins[base], w + wp, sdown);
+            acc_fixed(&ibins[stride + base], __builtin_fmaf(wp, q2, w * p2), sdown);
+            acc_fixed(&ibins[2 * stride + base], __builtin_fmaf(w, p4, wp * q4), sdown);
+          } else {
+            acc_fixed(&ibins[base], w, sdown);
+            acc_fixed(&ibins[stride + base], w * p2, sdown);
+            acc_fixed(&ibins[2 * stride + base], w * p4, sdown);
+            acc_fixed(&ibins[basep], wp, sdown);
+            acc_fixed(&ibins[stride + basep], wp * q2, sdown);
+            acc_fixed(&ibins[2 * stride + basep], wp * q4, sdown);
           }
-          const int base = kb * nmu + cm;
-          if (a.even024) {
-            // L_0 = 1, L_2 and L_4 by Horner in mu^2
-            const float x2 = mu * mu;
-            const float p2 = __builtin_fmaf(1.5f, x2, -0.5f);
-            const float p4 = __builtin_fmaf(__builtin_fmaf(4.375f, x2, -3.75f), x2, 0.375f);
-            if (a.losx0) {   // both modes of the pair share mu, and so the cell
-              const float s0 = w + wp;
-              acc_fixed(&ibins[base], s0, sdown);
-              acc_fixed(&ibins[stride + base], s0 * p2, sdown);
-              acc_fixed(&ibins[2 * stride + base], s0 * p4, sdown);
-              return;
-            }
-            const float y2 = mup * mup;
-            const float q2 = __builtin_fmaf(1.5f, y2, -0.5f);
-            const float q4 = __builtin_fmaf(__builtin_fmaf(4.375f, y2, -3.75f), y2, 0.375f);
-            if (cm == cp) {
-              acc_fixed(&ibins[base], w + wp, sdown);
-              acc_fixed(&ibins[stride + base], w * p2 + wp * q2, sdown);
-              acc_fixed(&ibins[2 * stride + base], w * p4 + wp * q4, sdown);
-            } else {
-              const int basep = kb * nmu + cp;
-              acc_fixed(&ibins[base], w, sdown);
-              acc_fixed(&ibins[stride + base], w * p2, sdown);
-              acc_fixed(&ibins[2 * stride + base], w * p4, sdown);
-              acc_fixed(&ibins[basep], wp, sdown);
-              acc_fixed(&ibins[stride + basep], wp * q2, sdown);
-              acc_fixed(&ibins[2 * stride + basep], wp * q4, sdown);
-            }
-            return;
-          }
-          const float x2 = mu * mu, y2 = mup * mup;
-          const int basep = kb * nmu + cp;
-          // the general pole set (rare): a rolled loop keeps its registers
-          // out of the common path's
+          return;
+        }
+        // the general pole set: a rolled loop keeps its registers out of the
+        // common path's.  The two half-spaces cancel odd poles off the
+        // kz = 0, M planes.
+        const int lmask = single ? ~0 : ~a.oddmask;
 #pragma unroll 1
-          for (int l = 0; l < PSH_MAX_NL; l++) {
-            if (l >= b.nl) break;
-            if (!((lmask >> l) & 1)) continue;
-            const float4 cf = legl[l];
-            float pl = ((cf.w * x2 + cf.z) * x2 + cf.y) * x2 + cf.x;
-            float ql = ((cf.w * y2 + cf.z) * y2 + cf.y) * y2 + cf.x;
-            if ((a.oddmask >> l) & 1) {
-              pl *= mu;
-              ql *= mup;
-            }
-            if (cm == cp) {
-              acc_fixed(&ibins[l * stride + base], w * pl + wp * ql, sdown);
-            } else {
-              acc_fixed(&ibins[l * stride + base], w * pl, sdown);
-              acc_fixed(&ibins[l * stride + basep], wp * ql, sdown);
-            }
+        for (int l = 0; l < b.nl; l++) {
+          if (!((lmask >> l) & 1)) continue;
+          const float4 cf = legl[l];
+          float pl = __builtin_fmaf(__builtin_fmaf(__builtin_fmaf(cf.w, x2, cf.z), x2, cf.y), x2,
+                                    cf.x);
+          float ql = __builtin_fmaf(__builtin_fmaf(__builtin_fmaf(cf.w, y2, cf.z), y2, cf.y), y2,
+                                    cf.x);
+          if ((a.oddmask >> l) & 1) {
+            pl *= mu;
+            ql *= mup;
           }
-        } else {   // SURVEY0, and SURVEYL, whose Y_lm weights are in v already
-          acc_fixed(&ibins[kb], w + wp, sdown);
+          if (cm == cp) {
+            acc_fixed(&ibins[l * stride + base], __builtin_fmaf(wp, ql, w * pl), sdown);
+          } else {
+            acc_fixed(&ibins[l * stride + base], w * pl, sdown);
+            acc_fixed(&ibins[l * stride + basep], wp * ql, sdown);
+          }
         }
       };
+      // Bin of pair k and 1 / |k|; -1 outside the window, -2 undecided in
+      // FP32.  |k|^2 is far from the denormal range: the bare reciprocal
+      // square root.
+      auto pair_bin = [&](int k, const Ops &o, float &rs) -> int {
+        const float k2f = o.ks + ksqyz;
+        rs = __builtin_amdgcn_rsqf(k2f);
+        const int kb = bin_fast(b, k2f, k2f * rs);
+        return (k == 0 && dcrow && i0 == 0) ? -1 : kb;   // the DC mode is skipped
+      };
+      const int kend = i0 + KMAX * S <= M ? KMAX : KMAX - 1;
       // The next pair's operands are read before the current pair's
       // accumulations: the compiler cannot tell the accumulators from the
       // tile and would otherwise wait for each pair's atomics before
-      // reading the next pair.  Partner indices outside the pairs (i = 0,
-      // M) read a valid entry that mode_pair discards.
-      auto fetch = [&](int k, float4 &xt, float &v, float &vp, float &ap) {
-        const int i = i0 + k * S;
-        const int ip = (i != 0 && i != M) ? N - i : i;
-        xt = xtab[i];
-        v = vrow[L::off(k * S)];
-        vp = lds[L::idx(c, ip)];
-        ap = xtab[ip].x;
+      // reading the next pair.  The loop is unrolled (constant LDS offsets,
+      // no address arithmetic: 32 interlaced 256^3 grids 1142 us, rolled
+      // 1171); the rare undecided pairs wait for a second, rolled one with the
+      // FP64 expressions (one body instead of KMAX + 1).
+      unsigned undecided = 0;
+      auto step = [&](int k, const Ops &o) {
+        float rs;
+        const int kb = pair_bin(k, o, rs);
+        if (kb == -2) {
+          undecided |= 1u << k;
+        } else {
+          const int kw = kb - a.kb0;
+          if (kb >= 0 && (unsigned)kw < (unsigned)a.nbw) add_pair(i0 + k * S, kw, rs, o);
+        }
       };
-      const int kend = i0 <= M ? (M - i0) / S : -1;   // last k with i <= M
-      float4 xt = make_float4(0.f, 0.f, 0.f, 0.f);
-      float v = 0.f, vp = 0.f, ap = 0.f;
-      if (kend >= 0) fetch(0, xt, v, vp, ap);
+      static_assert(KMAX < 32, "one bit per pair");
+      Ops o = fetch(0);
+      if constexpr (!GEN && KMAX <= 16) {
+#pragma unroll
+        for (int k = 0; k <= KMAX; k++) {
+          const Ops cur = o;
+          if (k < KMAX) o = fetch(k + 1);
+          if (k < KMAX || kend == KMAX) step(k, cur);
+        }
+      } else {
 #pragma unroll 1
-      for (int k = 0; k <= kend; k++) {
-        float4 xtn = xt;
-        float vn = 0.f, vpn = 0.f, apn = 0.f;
-        if (k < kend) fetch(k + 1, xtn, vn, vpn, apn);
-        mode_pair(i0 + k * S, xt, v, vp, ap);
-        xt = xtn;
-        v = vn;
-        vp = vpn;
-        ap = apn;
+        for (int k = 0; k <= kend; k++) {
+          const Ops cur = o;
+          if (k < KMAX) o = fetch(k + 1);
+          step(k, cur);
+        }
+      }
+      if (__ballot(undecided != 0)) {
+        const double ksqy = a.ax.ksq[1][y], ksqz = a.ax.ksq[2][kz];
+#pragma unroll 1
+        for (; undecided; undecided &= undecided - 1) {
+          const int k = __ffs((int)undecided) - 1, i = i0 + k * S;
+          const Ops u = fetch(k);
+          const int kb = bin_exact(b, GS ? a.ax.ksq[0][i] : ksqx[i], ksqy, ksqz, kz);
+          const int kw = kb - a.kb0;
+          if (kb >= 0 && (unsigned)kw < (unsigned)a.nbw)
+            add_pair(i, kw, __builtin_amdgcn_rsqf(u.ks + ksqyz), u);
+        }
       }
     }
     __syncthreads();
@@ -1049,14 +1157,15 @@ x_bin_kernel(XBinDev a, int ntz, int H, const float2 *__restrict__ tw) {
     for (int q2 = threadIdx.x; q2 < a.nacc; q2 += T) {
       const long long t = ibins[q2];
       if (t) {
-        if (GS) out[out_idx(q2)] += (double)t * sup;
+        // (GS: a no-return add to the workgroup's own row, which only this
+        // thread adds to: nothing waits for it)
+        if (GS) __builtin_amdgcn_global_atomic_fadd_f64((gdouble *)(out + out_idx(q2)), (double)t * sup);
         else bins[q2] += (double)t * sup;
         ibins[q2] = 0;
       }
     }
     if (threadIdx.x == 0) *tmaxp = 0u;
     __syncthreads();
-    tile = next;
   }
   // the window's accumulators into the workgroup's row of all bins
   if (!GS)
@@ -1200,7 +1309,7 @@ struct XBin {
   // the learned correction's plain N_g = 512 pass with 8 |mu| cells: one
   // workgroup per CU otherwise).
   template <bool NT>
-  static KFn pick(int epi, bool il, int nacc, size_t &shmem, int &T) {
+  static KFn pick(int epi, bool il, int nacc, bool gen, size_t &shmem, int &T) {
     const size_t stat = il ? xbin_static_lds<N, true>() : xbin_static_lds<N, false>();
     const size_t np = (size_t)((nacc + 1) & ~1);
     T = il ? XCfg<N, true>::T : XCfg<N, false>::T;
@@ -1212,17 +1321,21 @@ struct XBin {
       shmem = shmem_gs;
     }
     KFn k = nullptr;
-#define PSH_XB(E, I)                                                 \
+#define PSH_XB(E, I, G)                                                 \
   {                                                                     \
-    k = x_bin_kernel<N, E, I, NT, false>;                               \
-    if (!(I) && gs) k = x_bin_kernel<N, E, false, NT, true>;            \
+    k = x_bin_kernel<N, E, I, NT, false, G>;                            \
+    if (!(I) && gs) k = x_bin_kernel<N, E, false, NT, true, G>;         \
   }
     if (epi == PSH_EPI_SIM) {
-      if (il) PSH_XB(PSH_EPI_SIM, true) else PSH_XB(PSH_EPI_SIM, false)
+      if (gen) {
+        if (il) PSH_XB(PSH_EPI_SIM, true, true) else PSH_XB(PSH_EPI_SIM, false, true)
+      } else {
+        if (il) PSH_XB(PSH_EPI_SIM, true, false) else PSH_XB(PSH_EPI_SIM, false, false)
+      }
     } else if (epi == PSH_EPI_SURVEY0) {
-      if (il) PSH_XB(PSH_EPI_SURVEY0, true) else PSH_XB(PSH_EPI_SURVEY0, false)
+      if (il) PSH_XB(PSH_EPI_SURVEY0, true, false) else PSH_XB(PSH_EPI_SURVEY0, false, false)
     } else {
-      PSH_XB(PSH_EPI_SURVEYL, false)
+      PSH_XB(PSH_EPI_SURVEYL, false, false)
     }
 #undef PSH_XB
     if (shmem > 64 * 1024)
@@ -1241,7 +1354,7 @@ struct XBin {
       constexpr bool NT = decltype(ntc)::value;
       size_t shmem;
       int T;
-      KFn k = pick<NT>(epi, il, d.nacc, shmem, T);
+      KFn k = pick<NT>(epi, il, d.nacc, !(d.even024 && d.losx0), shmem, T);
       if (shmem > kXbinLdsMax) return hipErrorInvalidValue;
       hipLaunchKernelGGL(k, dim3(grid, nmock), dim3(T), shmem, s, dd, ntz, H, tw);
       return hipGetLastError();
@@ -1256,10 +1369,10 @@ struct XBin {
 // Workgroups per CU of the x pass kernel for a window of nacc accumulators.
 template <int N>
 struct XBinOcc {
-  static hipError_t run(int epi, bool il, int nacc, int *per_cu) {
+  static hipError_t run(int epi, bool il, int nacc, bool gen, int *per_cu) {
     size_t shmem;
     int T;
-    auto k = XBin<N>::template pick<true>(epi, il, nacc, shmem, T);
+    auto k = XBin<N>::template pick<true>(epi, il, nacc, gen, shmem, T);
     if (shmem > kXbinLdsMax) return hipErrorInvalidValue;
     return hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, (const void *)k, T, shmem);
   }
@@ -1407,9 +1520,16 @@ int psh_xbin_window_bins(int Ng, bool il, int per_bin) {
   return nb > (1 << 30) ? (1 << 30) : (int)nb;
 }
 
-int psh_xbin_per_cu(int Ng, int epi, bool il, int nacc) {
+namespace {
+bool poles_024(const PshBins &b) {
+  return b.nl == 3 && b.poles[0] == 0 && b.poles[1] == 2 && b.poles[2] == 4;
+}
+}  // namespace
+
+int psh_xbin_per_cu(int Ng, int epi, bool il, int nacc, const PshBins &b) {
   int nb = 0;
-  if (dispatch_n<XBinOcc>(Ng, epi, il, nacc, &nb) != hipSuccess) return 0;
+  const bool gen = !(poles_024(b) && b.losf[0] == 0.f);
+  if (dispatch_n<XBinOcc>(Ng, epi, il, nacc, gen, &nb) != hipSuccess) return 0;
   return nb;
 }
 
@@ -1473,7 +1593,7 @@ hipError_t psh_fft_x_bin(int Ng, const PshXBinArgs &a, const float2 *tw,
     for (int t = 0; t < 4; t++) d.legc[l][t] = kLeg[ell][t];
     if (ell & 1) d.oddmask |= 1 << l;
   }
-  d.even024 = a.bins.nl == 3 && a.bins.poles[0] == 0 && a.bins.poles[1] == 2 &&
-              a.bins.poles[2] == 4;
+  d.even024 = poles_024(a.bins);
+  d.nmuf = (float)a.bins.nmu;
   return dispatch_n<XBin>(Ng, d, a.epi, a.B != nullptr, a.grid, a.nmock, tw, s);
 }

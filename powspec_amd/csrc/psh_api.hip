@@ -434,7 +434,7 @@ int make_bins(psh_ctx *ctx) {
       ncu > 0)
     ctx->ncu = ncu;
   auto res = [&](int epi, bool il, int nacc) {
-    const int r = psh_xbin_per_cu(ctx->Ng, epi, il, nacc);
+    const int r = psh_xbin_per_cu(ctx->Ng, epi, il, nacc, b);
     return r > 0 ? r : 1;
   };
   if (c.issim) {
