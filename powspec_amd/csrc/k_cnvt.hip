@@ -4,6 +4,9 @@
 #include <math.h>
 #include <string.h>
 
+#include <algorithm>
+#include <mutex>
+#include <type_traits>
 #include <vector>
 
 #include <hip/hip_runtime.h>
@@ -63,15 +66,16 @@ struct Cosmo {
   double om, ol, ok, widx;
 };
 
-// c/100/E(z) with the terms in the reference's order (src/cnvt_coord.c:241-252)
-__host__ __device__ inline double integrand(const Cosmo &c, double z) {
+// E(z)^2 with the terms in the reference's order (src/cnvt_coord.c:241-252)
+__host__ __device__ inline double efunc2(const Cosmo &c, double z) {
+#pragma clang fp contract(off)
   double z1 = z + 1;
   double z2 = z1 * z1;
   double d = c.om * z2 * z1;
   if (c.ok) d += c.ok * z2;
   if (c.widx) d += c.ol * pow(z1, c.widx);
   else d += c.ol;
-  return kCH / sqrt(d);
+  return d;
 }
 
 struct RuleDev {
@@ -79,11 +83,19 @@ struct RuleDev {
   double x[kMaxOrder / 2 + 1], w[kMaxOrder / 2 + 1], w0;
 };
 
+// The order search compares distances of successive orders: written without
+// fused operations, host and device round alike (but for pow, see
+// psh_cnvt_device) and settle on the same order.
 __host__ __device__ inline double cmvdist(const Cosmo &c, const RuleDev &r, double z) {
+#pragma clang fp contract(off)
+  auto f = [&](double t) {
+#pragma clang fp contract(off)
+    return kCH / sqrt(efunc2(c, t));
+  };
   double zp = z * 0.5, sum = 0;
   for (int k = 0; k < r.n / 2; k++)
-    sum += r.w[k] * (integrand(c, zp * (1 + r.x[k])) + integrand(c, zp * (1 - r.x[k])));
-  if (r.n & 1) sum += r.w0 * integrand(c, zp);
+    sum += r.w[k] * (f(zp * (1 + r.x[k])) + f(zp * (1 - r.x[k])));
+  if (r.n & 1) sum += r.w0 * f(zp);
   return sum * zp;
 }
 
@@ -99,16 +111,142 @@ RuleDev rule_dev(int n) {
 
 __device__ inline void to_cartesian(double *p, double dist) {
   const double ra = p[0] * kDeg, dec = p[1] * kDeg;
-  p[0] = dist * cos(dec) * cos(ra);
-  p[1] = dist * cos(dec) * sin(ra);
-  p[2] = dist * sin(dec);
+  double sr, cr, sd, cd;   // (one argument reduction for both)
+  sincos(ra, &sr, &cr);
+  sincos(dec, &sd, &cd);
+  p[0] = dist * cd * cr;
+  p[1] = dist * cd * sr;
+  p[2] = dist * sd;
 }
 
-__global__ void __launch_bounds__(256) integr_kernel(double *d, size_t n, Cosmo c, RuleDev r) {
+// Workspace of the integrated conversion on the device.
+struct CnvtDev {
+  double zmin, zmax;   // of the arrays seen so far
+  int order;           // > 0 found; 0 nothing to convert; -1 error
+  RuleDev rules[kMaxOrder + 2 - kMinOrder];   // orders kMinOrder..kMaxOrder + 1
+};
+
+// 1 / E(z): the distance integral with reciprocal square roots, whose
+// rounding (1 ulp against 1/2 + 1/2 of a root and a division) is far below
+// the quadrature's error, and a third of their instructions: 2e7 records at
+// order 5 took 377 us, bound by FP64 arithmetic, now 286 us; moving their
+// 1.28 GB takes 266 us.
+template <bool K, bool W>
+__device__ inline double distance(const Cosmo &c, const RuleDev &r, double z) {
+  auto f = [&](double t) -> double {
+    const double z1 = t + 1, z2 = z1 * z1;
+    double d = W ? c.ol * pow(z1, c.widx) : c.ol;
+    d = __builtin_fma(c.om * z2, z1, d);
+    if (K) d = __builtin_fma(c.ok, z2, d);
+    return rsqrt(d);
+  };
+  const double zp = z * 0.5;
+  double sum = 0;
+  for (int k = 0; k < r.n / 2; k++)
+    sum = __builtin_fma(r.w[k], f(__builtin_fma(zp, r.x[k], zp)) + f(__builtin_fma(-zp, r.x[k], zp)),
+                        sum);
+  if (r.n & 1) sum = __builtin_fma(r.w0, f(zp), sum);
+  return sum * (zp * kCH);
+}
+
+template <bool K, bool W>
+__global__ void __launch_bounds__(256)
+integr_kernel(double *d, size_t n, Cosmo c, const CnvtDev *ws) {
+  const int order = ws->order;
+  if (order <= 0) return;
+  const RuleDev &r = ws->rules[order - kMinOrder];
   for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n;
        i += (size_t)gridDim.x * blockDim.x) {
     double *p = d + 4 * i;
-    to_cartesian(p, cmvdist(c, r, p[2]));
+    to_cartesian(p, distance<K, W>(c, r, p[2]));
+  }
+}
+
+// Smallest order at which the integral to z has converged
+// (src/cnvt_coord.c:306-341): orders are tried from kMinOrder up; the test
+// reaches order kMaxOrder + 1 before it gives up (the reference reads that
+// rule past the end of its table; here it is computed), -1 when that does not
+// converge either.
+__host__ __device__ inline int order_at(const Cosmo &c, const RuleDev *rules, double err,
+                                        double z) {
+#pragma clang fp contract(off)
+  double oint, nint = 0;
+  int n = kMinOrder - 1;
+  do {
+    if (n > kMaxOrder) return -1;
+    oint = nint;
+    ++n;
+    nint = cmvdist(c, rules[n - kMinOrder], z);
+  } while (fabs(nint - oint) > nint * err);
+  return n;
+}
+
+// i-th of the kNumZ redshifts of the convergence test
+__host__ __device__ inline double test_z(double zmin, double zmax, int i) {
+#pragma clang fp contract(off)
+  return zmin + i * (zmax - zmin) / (kNumZ - 1);
+}
+
+// The order of a redshift range: the largest of the test redshifts' (-1 when
+// one of them does not converge).
+int choose_order(const Cosmo &c, const RuleDev *rules, double err, double zmin, double zmax) {
+  int order = 0;
+  for (int i = 0; i < kNumZ; i++) {
+    const int n = order_at(c, rules, err, test_z(zmin, zmax, i));
+    if (n < 0) return -1;
+    if (order < n) order = n;
+  }
+  return order;
+}
+
+// Takes the redshift bounds of one array's blocks into ws; with `last`, finds
+// the order, one test redshift per thread.  One workgroup.  (On the host the
+// same search, the copies to and from it and the tables of its 30 rules, made
+// anew on each call, took 330 us.)
+__global__ void __launch_bounds__(256)
+order_kernel(CnvtDev *ws, const double *__restrict__ part, int blocks, int first, int last,
+             Cosmo c, double err, double *__restrict__ hout) {
+  __shared__ double mn[256], mx[256];
+  __shared__ int worst;
+  const int t = threadIdx.x;
+  double a = DBL_MAX, b = -DBL_MAX;
+  for (int i = t; i < blocks; i += 256) {
+    a = fmin(a, part[PSH_BOUNDS_STRIDE * i + 2]);
+    b = fmax(b, part[PSH_BOUNDS_STRIDE * i + 5]);
+  }
+  mn[t] = a;
+  mx[t] = b;
+  if (t == 0) worst = 0;
+  __syncthreads();
+  for (int k = 128; k > 0; k >>= 1) {
+    if (t < k) {
+      mn[t] = fmin(mn[t], mn[t + k]);
+      mx[t] = fmax(mx[t], mx[t + k]);
+    }
+    __syncthreads();
+  }
+  double zmin = mn[0], zmax = mx[0];
+  if (!first) {
+    zmin = fmin(zmin, ws->zmin);
+    zmax = fmax(zmax, ws->zmax);
+  }
+  __syncthreads();   // (every thread has read the earlier bounds)
+  const bool any = zmin <= zmax && zmin >= 0;   // something to convert, no negative redshift
+  if (last && any && t < kNumZ) {
+    const int n = order_at(c, ws->rules, err, test_z(zmin, zmax, t));
+    atomicMax(&worst, n < 0 ? kMaxOrder + 2 : n);
+  }
+  __syncthreads();
+  if (t == 0) {
+    ws->zmin = zmin;
+    ws->zmax = zmax;
+    if (last) {
+      const int order = zmin > zmax ? 0 : (!any || worst > kMaxOrder + 1) ? -1 : worst;
+      ws->order = order;
+      hout[0] = zmin;
+      hout[1] = zmax;
+      hout[2] = (double)order;
+    }
   }
 }
 
@@ -151,34 +289,135 @@ std::vector<double> spline_ypp(const double *x, const double *y, size_t n) {
   return ypp;
 }
 
-// Order by the reference's convergence test on kNumZ redshifts spanning
-// [zmin, zmax] (src/cnvt_coord.c:306-341): orders are tried from kMinOrder
-// up; the test reaches order kMaxOrder + 1 before it gives up (the reference
-// reads that rule past the end of its table; here it is computed), -1 when
-// that does not converge either.
-int choose_order(const Cosmo &c, double err, double zmin, double zmax) {
-  std::vector<RuleDev> rules;
-  for (int n = kMinOrder; n <= kMaxOrder + 1; n++) rules.push_back(rule_dev(n));
-  int order = 0;
-  for (int i = 0; i < kNumZ; i++) {
-    const double z = zmin + i * (zmax - zmin) / (kNumZ - 1);
-    double oint, nint = 0;
-    int n = kMinOrder - 1;
-    do {
-      if (n > kMaxOrder) return -1;
-      oint = nint;
-      ++n;
-      nint = cmvdist(c, rules[n - kMinOrder], z);
-    } while (fabs(nint - oint) > nint * err);
-    if (order < n) order = n;
-  }
-  return order;
-}
-
 unsigned blocks_for(size_t n) {
   size_t b = (n + 255) / 256;
   if (b > 8192) b = 8192;
   return (unsigned)(b ? b : 1);
+}
+
+// Workspace of one call: the device block, per-block bounds and the pinned
+// results.  Calls take one and give it back when their work is done; at most
+// kKeep of them stay for later calls.
+constexpr int kBoundsBlocks = 1024;
+struct Workspace {
+  int device = -1;
+  CnvtDev *dev = nullptr;
+  double *part = nullptr;
+  double *hout = nullptr;   // zmin, zmax, order
+};
+
+void free_workspace(Workspace &w) {
+  if (w.dev) (void)hipFree(w.dev);
+  if (w.part) (void)hipFree(w.part);
+  if (w.hout) (void)hipHostFree(w.hout);
+  w = Workspace{};
+}
+
+struct Workspaces {
+  static constexpr size_t kKeep = 4;
+  std::mutex m;
+  std::vector<Workspace> idle;
+
+  bool take(const std::vector<RuleDev> &rules, Workspace &w) {
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return false;
+    {
+      std::lock_guard<std::mutex> lock(m);
+      for (size_t i = 0; i < idle.size(); i++)
+        if (idle[i].device == dev) {
+          w = idle[i];
+          idle.erase(idle.begin() + (long)i);
+          return true;
+        }
+    }
+    w.device = dev;
+    if (hipMalloc((void **)&w.dev, sizeof(CnvtDev)) == hipSuccess &&
+        hipMalloc((void **)&w.part, sizeof(double) * PSH_BOUNDS_STRIDE * kBoundsBlocks) ==
+            hipSuccess &&
+        hipHostMalloc((void **)&w.hout, 3 * sizeof(double), hipHostMallocDefault) == hipSuccess &&
+        hipMemcpy(w.dev->rules, rules.data(), sizeof(w.dev->rules), hipMemcpyHostToDevice) ==
+            hipSuccess)
+      return true;
+    free_workspace(w);
+    return false;
+  }
+  void give(Workspace &w) {
+    {
+      std::lock_guard<std::mutex> lock(m);
+      if (idle.size() < kKeep) {
+        idle.push_back(w);
+        return;
+      }
+    }
+    free_workspace(w);
+  }
+};
+
+// (never destroyed: the HIP runtime may end before static destructors run)
+Workspaces &workspaces() {
+  static Workspaces *w = new Workspaces;
+  return *w;
+}
+
+// The quadrature rules of the orders kMinOrder..kMaxOrder + 1.
+const std::vector<RuleDev> &all_rules() {
+  static const std::vector<RuleDev> rules = [] {
+    std::vector<RuleDev> r;
+    for (int n = kMinOrder; n <= kMaxOrder + 1; n++) r.push_back(rule_dev(n));
+    return r;
+  }();
+  return rules;
+}
+
+// Redshift range of everything to be converted (src/cnvt_coord.c:138-226),
+// its order and the conversion, on one stream with one wait at the end.
+int integrate(const psh_cnvt *cv, const Cosmo &c, psh_data *const *d_data, const size_t *n,
+              int narr, const Workspace &w, hipStream_t s, int *order_out) {
+  int lasta = -1;
+  for (int a = 0; a < narr; a++)
+    if (n[a]) lasta = a;
+  if (order_out) *order_out = 0;
+  if (lasta < 0) return PSH_OK;   // nothing to convert
+  bool first = true;
+  for (int a = 0; a <= lasta; a++) {
+    if (!n[a]) continue;
+    int blocks = (int)std::min<size_t>((n[a] + 255) / 256, kBoundsBlocks);
+    if (psh_coord_bounds((const double *)d_data[a], n[a], w.part, blocks, s) != hipSuccess)
+      return PSH_ERR_DEVICE;
+    hipLaunchKernelGGL(order_kernel, dim3(1), dim3(256), 0, s, w.dev, w.part, blocks, (int)first,
+                       (int)(a == lasta), c, cv->ecdst, w.hout);
+    if (hipGetLastError() != hipSuccess) return PSH_ERR_DEVICE;
+    first = false;
+  }
+  if (c.widx) {
+    // pow of the host and of the device may differ in the last bit, and the
+    // order with it where a test is that close: the host decides
+    if (hipStreamSynchronize(s) != hipSuccess) return PSH_ERR_DEVICE;
+    int order = (int)w.hout[2];
+    if (w.hout[0] <= w.hout[1] && w.hout[0] >= 0) {
+      order = choose_order(c, all_rules().data(), cv->ecdst, w.hout[0], w.hout[1]);
+      if (order < 0) return PSH_ERR_CNVT;
+      if (hipMemcpy(&w.dev->order, &order, sizeof order, hipMemcpyHostToDevice) != hipSuccess)
+        return PSH_ERR_DEVICE;
+      w.hout[2] = (double)order;
+    }
+  }
+  for (int a = 0; a <= lasta; a++) {
+    if (!n[a]) continue;
+    auto go = [&](auto k, auto x) {
+      hipLaunchKernelGGL((integr_kernel<decltype(k)::value, decltype(x)::value>),
+                         dim3(blocks_for(n[a])), dim3(256), 0, s, (double *)d_data[a], n[a], c,
+                         w.dev);
+    };
+    if (c.ok) c.widx ? go(std::true_type{}, std::true_type{}) : go(std::true_type{}, std::false_type{});
+    else c.widx ? go(std::false_type{}, std::true_type{}) : go(std::false_type{}, std::false_type{});
+    if (hipGetLastError() != hipSuccess) return PSH_ERR_DEVICE;
+  }
+  if (hipStreamSynchronize(s) != hipSuccess) return PSH_ERR_DEVICE;
+  const int order = (int)w.hout[2];
+  if (order < 0) return PSH_ERR_CNVT;   // negative redshift, or no convergence
+  if (order_out) *order_out = order;
+  return PSH_OK;
 }
 
 }  // namespace
@@ -214,47 +453,15 @@ extern "C" int psh_cnvt_device(const psh_cnvt *cv, psh_data *const *d_data, cons
     if (order_out) *order_out = 0;
     return ok ? PSH_OK : PSH_ERR_DEVICE;
   }
-  // redshift range of everything to be converted (src/cnvt_coord.c:138-226)
-  double zmin = DBL_MAX, zmax = -DBL_MAX;
-  double *part = nullptr;
-  const int pb = 1024;
-  if (hipMalloc(&part, sizeof(double) * PSH_BOUNDS_STRIDE * pb) != hipSuccess)
-    return PSH_ERR_MEMORY;
-  std::vector<double> h(PSH_BOUNDS_STRIDE * pb);
-  for (int a = 0; a < narr; a++) {
-    if (!n[a]) continue;
-    int blocks = (int)((n[a] + 255) / 256);
-    if (blocks > pb) blocks = pb;
-    if (psh_coord_bounds((const double *)d_data[a], n[a], part, blocks, s) != hipSuccess ||
-        hipMemcpy(h.data(), part, sizeof(double) * PSH_BOUNDS_STRIDE * blocks,
-                  hipMemcpyDeviceToHost) !=
-            hipSuccess) {
-      (void)hipFree(part);
-      return PSH_ERR_DEVICE;
-    }
-    for (int b = 0; b < blocks; b++) {
-      zmin = fmin(zmin, h[PSH_BOUNDS_STRIDE * b + 2]);
-      zmax = fmax(zmax, h[PSH_BOUNDS_STRIDE * b + 5]);
-    }
-  }
-  (void)hipFree(part);
-  if (zmin > zmax) {   // nothing to convert
-    if (order_out) *order_out = 0;
-    return PSH_OK;
-  }
-  if (zmin < 0) return PSH_ERR_CNVT;   // negative redshift
-  const int order = choose_order(c, cv->ecdst, zmin, zmax);
-  if (order < 0) return PSH_ERR_CNVT;
-  const RuleDev r = rule_dev(order);
-  for (int a = 0; a < narr; a++) {
-    if (!n[a]) continue;
-    hipLaunchKernelGGL(integr_kernel, dim3(blocks_for(n[a])), dim3(256), 0, s,
-                       (double *)d_data[a], n[a], c, r);
-    if (hipGetLastError() != hipSuccess) return PSH_ERR_DEVICE;
-  }
-  if (hipStreamSynchronize(s) != hipSuccess) return PSH_ERR_DEVICE;
-  if (order_out) *order_out = order;
-  return PSH_OK;
+  Workspace w;
+  if (!workspaces().take(all_rules(), w)) return PSH_ERR_MEMORY;
+  int order = 0;
+  const int rc = integrate(cv, c, d_data, n, narr, w, s, &order);
+  // an error may have left work in flight that writes the workspace
+  if (rc == PSH_ERR_DEVICE) (void)hipStreamSynchronize(s);
+  workspaces().give(w);
+  if (rc == PSH_OK && order_out) *order_out = order;
+  return rc;
 }
 
 extern "C" int psh_cnvt_coord(const psh_cnvt *cv, psh_cata *cat) {
