@@ -106,6 +106,12 @@ PSH_HD inline void mul10_add(uint64_t &hi, uint64_t &lo, uint32_t d) {
   hi = hi * 10 + (t1 >> 32);
 }
 
+// M * 10 + d for an M of nd digits: up to 19 digits fit 64 bits.
+PSH_HD inline void append_digit(uint64_t &hi, uint64_t &lo, int nd, uint32_t d) {
+  if (nd < 19) lo = lo * 10 + d;
+  else mul10_add(hi, lo, d);
+}
+
 PSH_HD inline int msb128(uint64_t hi, uint64_t lo) { return hi ? 64 + msb64(hi) : msb64(lo); }
 
 // Correctly rounded double of M 10^E (M = hi:lo >= 1), plus an
@@ -206,7 +212,7 @@ PSH_HD inline bool parse_double(const char *p, const char *e, double *out) {
       continue;
     }
     if (nd < 38) {
-      mul10_add(Mhi, Mlo, (uint32_t)d);
+      append_digit(Mhi, Mlo, nd, (uint32_t)d);
       nd++;
     } else {
       dexp++;
@@ -222,7 +228,7 @@ PSH_HD inline bool parse_double(const char *p, const char *e, double *out) {
       if (nd == 0 && d == 0) {
         dexp--;
       } else if (nd < 38) {
-        mul10_add(Mhi, Mlo, (uint32_t)d);
+        append_digit(Mhi, Mlo, nd, (uint32_t)d);
         nd++;
         dexp--;
       } else if (d) {
