@@ -2044,10 +2044,6 @@ extern "C" int psh_ctx_run_host(psh_ctx *ctx, psh_cata *cat, psh_pk *out) {
   if (cat->num != ctx->conf.ndata)
     return set_err(ctx, PSH_ERR_ARG, "catalogue count %d != ndata %d", cat->num, ctx->conf.ndata);
   int rc;
-  double mn[3], mx[3], swd[2] = {0, 0}, swr[2] = {0, 0};
-  scan_cat(ctx, cat, mn, mx, swd, swr);
-  if ((rc = def_box(ctx, mn, mx))) return rc;
-  if ((rc = ensure_geometry(ctx))) return rc;
   size_t need = 0;
   for (int c = 0; c < cat->num; c++) need += cat->ndata[c] + (ctx->survey ? cat->nrand[c] : 0);
   if (need > ctx->d_cat_cap) {
@@ -2056,22 +2052,35 @@ extern "C" int psh_ctx_run_host(psh_ctx *ctx, psh_cata *cat, psh_pk *out) {
   }
   CatDev cd[2] = {};
   size_t off = 0;
-  const double vol = ctx->L[0] * ctx->L[1] * ctx->L[2];
+  // the arrays in upload order; their bounds and weight sums from the device
+  // (a host pass over them took longer than the upload)
+  const double *arr[4];
+  size_t len[4];
+  int narr = 0;
   for (int c = 0; c < cat->num; c++) {
-    cd[c].data = ctx->d_cat + 4 * off;
-    cd[c].nd = cat->ndata[c];
+    arr[narr] = cd[c].data = ctx->d_cat + 4 * off;
+    len[narr++] = cd[c].nd = cat->ndata[c];
     if ((rc = stage_host(ctx, cat->data[c], cat->ndata[c], off))) return rc;
     off += cat->ndata[c];
     if (ctx->survey) {
-      cd[c].rand = ctx->d_cat + 4 * off;
-      cd[c].nr = cat->nrand[c];
+      arr[narr] = cd[c].rand = ctx->d_cat + 4 * off;
+      len[narr++] = cd[c].nr = cat->nrand[c];
       if ((rc = stage_host(ctx, cat->rand[c], cat->nrand[c], off))) return rc;
       off += cat->nrand[c];
+    }
+  }
+  double mn[3] = {DBL_MAX, DBL_MAX, DBL_MAX}, mx[3] = {-DBL_MAX, -DBL_MAX, -DBL_MAX}, sw[4];
+  if ((rc = bounds_device(ctx, arr, len, narr, mn, mx, sw))) return rc;
+  if ((rc = def_box(ctx, mn, mx))) return rc;
+  if ((rc = ensure_geometry(ctx))) return rc;
+  const double vol = ctx->L[0] * ctx->L[1] * ctx->L[2];
+  for (int c = 0, i = 0; c < cat->num; c++) {
+    cd[c].sw_d = sw[i++];
+    if (ctx->survey) {
+      cd[c].sw_r = sw[i++];
       cd[c].alpha = cat->alpha[c];
       cd[c].shot = cat->shot[c];
       cd[c].norm = cat->norm[c];
-      cd[c].sw_d = swd[c];
-      cd[c].sw_r = swr[c];
     } else {
       // shot/norm of simulation boxes (src/genr_mesh.c:904-910)
       const double w = cat->wdata[c];
