@@ -525,6 +525,10 @@ struct XBinDev {
   float legc[PSH_MAX_NL][4];
   int oddmask;
   int even024;   // the poles are exactly 0, 2, 4 (the common request)
+  // any other set of poles 0..4: accumulator offset of pole ell, -1 when it
+  // is not asked for; low4 0 when a pole is above 4
+  int low4;
+  int acc4[5];
   float nmuf;    // (float)bins.nmu
   const int *ylive;   // per k_z tile, the largest |k_y| with binned modes, or nullptr
 };
@@ -644,7 +648,7 @@ __device__ __forceinline__ int bin_exact(const PshBins &b, double ksqx, double k
 // (nothing in it waits on memory: tables from LDS or scalar loads, no select
 // on a loaded value) and binning without address arithmetic or FP64 took,
 // on MI355X, start of the tuning -> now: plain 256^3 47 -> 33 us, interlaced
-// 640^3 log bins 1.72 -> 1.34 ms, 1024^3 3.40 -> 3.02 ms, 32 interlaced 256^3
+// 640^3 log bins 1.72 -> 1.20 ms, 1024^3 3.40 -> 3.02 ms, 32 interlaced 256^3
 // 1.31 -> 1.14 ms, alias-corrected 512^3 with |mu| cells 343 -> 257 us.
 //
 // Forward x transform of one (y, kz-tile) column tile fused with the
@@ -779,7 +783,7 @@ x_bin_kernel(XBinDev a, int ntz, int H, const float2 *__restrict__ tw) {
   // the host with the binning's FP64 |k|, which only grows with |k_x|, |k_y|
   // and k_z); with k_max = k_Ny about 1 - pi/4 of the (k_y, k_z) tiles are
   // skipped.  nullptr (the survey l = 0 pass, whose stored field is
-  // transformed back in full, and log bins): every tile.
+  // transformed back in full): every tile.
   typedef __attribute__((address_space(4))) const int cint;       // uniform tables:
   typedef __attribute__((address_space(4))) const float cfloat;   // scalar loads
   auto live = [&](int ty, int tq) -> bool {
@@ -1010,10 +1014,12 @@ x_bin_kernel(XBinDev a, int ntz, int H, const float2 *__restrict__ tw) {
         return o;
       };
       // One mode pair in bin kb (relative to the window) with 1 / |k| = rs.
-      auto add_pair = [&](int i, int kb, float rs, const Ops &o) {
+      // low4: the poles are among 0..4 (GEN only).
+      auto add_pair = [&](auto low4, int i, int kb, float rs, const Ops &o) {
         // sums of products are fused where written so: left to the compiler,
         // the fusions, and with them the last bits, follow the code around
 #pragma clang fp contract(off)
+        constexpr bool LOW4 = decltype(low4)::value;
         // the partner k_x = -i (none for i = 0 and the Nyquist index M)
         const bool pair = i != 0 && i != M;
         const float al = o.ax * wyz;
@@ -1068,9 +1074,33 @@ x_bin_kernel(XBinDev a, int ntz, int H, const float2 *__restrict__ tw) {
           }
           return;
         }
-        // the general pole set: a rolled loop keeps its registers out of the
-        // common path's.  The two half-spaces cancel odd poles off the
-        // kz = 0, M planes.
+        // The two half-spaces cancel odd poles off the kz = 0, M planes.
+        if constexpr (LOW4) {
+          // the polynomials of both modes by Horner in mu^2
+          auto add = [&](int off, float pl, float ql) {
+            if (cm == cp) {
+              acc_fixed(&ibins[off + base], __builtin_fmaf(wp, ql, w * pl), sdown);
+            } else {
+              acc_fixed(&ibins[off + base], w * pl, sdown);
+              acc_fixed(&ibins[off + basep], wp * ql, sdown);
+            }
+          };
+          if (a.acc4[0] >= 0) add(a.acc4[0], 1.f, 1.f);
+          if (a.acc4[2] >= 0)
+            add(a.acc4[2], __builtin_fmaf(1.5f, x2, -0.5f), __builtin_fmaf(1.5f, y2, -0.5f));
+          if (a.acc4[4] >= 0)
+            add(a.acc4[4], __builtin_fmaf(__builtin_fmaf(4.375f, x2, -3.75f), x2, 0.375f),
+                __builtin_fmaf(__builtin_fmaf(4.375f, y2, -3.75f), y2, 0.375f));
+          if (single) {
+            if (a.acc4[1] >= 0) add(a.acc4[1], mu, mup);
+            if (a.acc4[3] >= 0)
+              add(a.acc4[3], __builtin_fmaf(2.5f, x2, -1.5f) * mu,
+                  __builtin_fmaf(2.5f, y2, -1.5f) * mup);
+          }
+          return;
+        }
+        // poles above 4: a rolled loop (for any poles, as it was before, the
+        // interlaced 640^3 pass with poles 0..4 took 1.33 ms, now 1.20)
         const int lmask = single ? ~0 : ~a.oddmask;
 #pragma unroll 1
         for (int l = 0; l < b.nl; l++) {
@@ -1110,32 +1140,41 @@ x_bin_kernel(XBinDev a, int ntz, int H, const float2 *__restrict__ tw) {
       // 1171); the rare undecided pairs wait for a second, rolled one with the
       // FP64 expressions (one body instead of KMAX + 1).
       unsigned undecided = 0;
-      auto step = [&](int k, const Ops &o) {
+      auto step = [&](auto low4, int k, const Ops &o) {
         float rs;
         const int kb = pair_bin(k, o, rs);
         if (kb == -2) {
           undecided |= 1u << k;
         } else {
           const int kw = kb - a.kb0;
-          if (kb >= 0 && (unsigned)kw < (unsigned)a.nbw) add_pair(i0 + k * S, kw, rs, o);
+          if (kb >= 0 && (unsigned)kw < (unsigned)a.nbw) add_pair(low4, i0 + k * S, kw, rs, o);
         }
       };
       static_assert(KMAX < 32, "one bit per pair");
       Ops o = fetch(0);
-      if constexpr (!GEN && KMAX <= 16) {
+      auto unrolled = [&]() {
 #pragma unroll
         for (int k = 0; k <= KMAX; k++) {
           const Ops cur = o;
           if (k < KMAX) o = fetch(k + 1);
-          if (k < KMAX || kend == KMAX) step(k, cur);
+          if (k < KMAX || kend == KMAX) step(std::true_type{}, k, cur);
         }
-      } else {
+      };
+      auto rolled = [&](auto low4) {
 #pragma unroll 1
         for (int k = 0; k <= kend; k++) {
           const Ops cur = o;
           if (k < KMAX) o = fetch(k + 1);
-          step(k, cur);
+          step(low4, k, cur);
         }
+      };
+      const bool low = !GEN || a.low4;
+      if constexpr (KMAX <= 16) {
+        if (low) unrolled();
+        else rolled(std::false_type{});
+      } else {
+        if (low) rolled(std::true_type{});
+        else rolled(std::false_type{});
       }
       if (__ballot(undecided != 0)) {
         const double ksqy = a.ax.ksq[1][y], ksqz = a.ax.ksq[2][kz];
@@ -1146,7 +1185,7 @@ x_bin_kernel(XBinDev a, int ntz, int H, const float2 *__restrict__ tw) {
           const int kb = bin_exact(b, GS ? a.ax.ksq[0][i] : ksqx[i], ksqy, ksqz, kz);
           const int kw = kb - a.kb0;
           if (kb >= 0 && (unsigned)kw < (unsigned)a.nbw)
-            add_pair(i, kw, __builtin_amdgcn_rsqf(u.ks + ksqyz), u);
+            add_pair(std::false_type{}, i, kw, __builtin_amdgcn_rsqf(u.ks + ksqyz), u);
         }
       }
     }
@@ -1594,6 +1633,12 @@ hipError_t psh_fft_x_bin(int Ng, const PshXBinArgs &a, const float2 *tw,
     if (ell & 1) d.oddmask |= 1 << l;
   }
   d.even024 = poles_024(a.bins);
+  d.low4 = 1;
+  for (int &o : d.acc4) o = -1;
+  for (int l = 0; l < a.bins.nl; l++) {
+    if (a.bins.poles[l] > 4 || d.acc4[a.bins.poles[l]] >= 0) d.low4 = 0;   // (or repeated)
+    else d.acc4[a.bins.poles[l]] = l * d.nbw * (a.epi == PSH_EPI_SIM ? a.bins.nmu : 1);
+  }
   d.nmuf = (float)a.bins.nmu;
   return dispatch_n<XBin>(Ng, d, a.epi, a.B != nullptr, a.grid, a.nmock, tw, s);
 }
