@@ -499,24 +499,26 @@ int make_tables(psh_ctx *ctx) {
   // k_z = q CX) lies before the last bin edge, with the binning's own FP64
   // |k| = sqrt((k_x^2 + k_y^2) + k_z^2) (src/multipole.c:147-158), which
   // only grows with |k_x|, |k_y| and k_z.  The y pass stores no output past
-  // it and the x pass skips the tiles; -1 when no k_y is live.  Log bins
-  // keep every tile.
-  ctx->kzlim = 1 << 30;
-  if (ctx->conf.logscale) {
-    ctx_free(ctx, ctx->d_ylive);
-    ctx->d_ylive = nullptr;
-  } else {
+  // it and the x pass skips the tiles; -1 when no k_y is live.  For log bins
+  // the host's and the device's log10 may differ in the last bits: tiles
+  // within 1e-9 of the edge stay live.
+  {
     const int CX = psh_xbin_tile_cols(N);
     const int ntzx = (N / 2 + 1 + CX - 1) / CX;
     const double *ksqy = h.data() + (size_t)(4 * 1 + 1) * N;
     const double *ksqz = h.data() + (size_t)(4 * 2 + 1) * N;
     std::vector<int> yl(ntzx, -1);
+    const double edge = ctx->bins.kedgeN;
+    auto before_edge = [&](double m2) {
+      return ctx->conf.logscale ? 0.5 * log10(m2) < edge + 1e-9 * (1 + fabs(edge))
+                                : sqrt(m2) < edge;
+    };
     for (int q = 0; q < ntzx; q++) {
       const int kz0 = q * CX;
       for (int ky = 0; ky <= N / 2; ky++) {
         double m2 = ksqy[ky];
         if (kz0 > 0) m2 = m2 + ksqz[kz0];
-        if (!(sqrt(m2) < ctx->bins.kedgeN)) break;
+        if (!before_edge(m2)) break;
         yl[q] = ky;
       }
     }
