@@ -257,6 +257,35 @@ bounds_kernel(const double *__restrict__ xyzw, size_t n,
   if (threadIdx.x < 7) partial[blockIdx.x * PSH_BOUNDS_STRIDE + threadIdx.x] = sh[threadIdx.x][0];
 }
 
+// One workgroup per array: its blocks' bounds and weight sums, in a fixed tree.
+__global__ void __launch_bounds__(256)
+bounds_fold_kernel(const double *__restrict__ partial, int blocks0, int blocks1,
+                   double *__restrict__ out) {
+  const int t = threadIdx.x, blocks = blockIdx.x ? blocks1 : blocks0;
+  const double *p = partial + (blockIdx.x ? (size_t)blocks0 * PSH_BOUNDS_STRIDE : 0);
+  double v[7] = {DBL_MAX, DBL_MAX, DBL_MAX, -DBL_MAX, -DBL_MAX, -DBL_MAX, 0.0};
+  auto join = [](double *a, const double *b) {
+    for (int i = 0; i < 3; i++) {
+      a[i] = fmin(a[i], b[i]);
+      a[3 + i] = fmax(a[3 + i], b[3 + i]);
+    }
+    a[6] += b[6];
+  };
+  for (int i = t; i < blocks; i += 256) {
+    double b[7];
+    for (int c = 0; c < 7; c++) b[c] = p[(size_t)i * PSH_BOUNDS_STRIDE + c];
+    join(v, b);
+  }
+  __shared__ double sh[256][7];
+  for (int c = 0; c < 7; c++) sh[t][c] = v[c];
+  __syncthreads();
+  for (int k = 128; k > 0; k >>= 1) {
+    if (t < k) join(sh[t], sh[t + k]);
+    __syncthreads();
+  }
+  if (t < 7) out[blockIdx.x * PSH_BOUNDS_STRIDE + t] = sh[0][t];
+}
+
 }  // namespace
 
 size_t psh_geometry_scratch_bytes(const PshBins &b) {
@@ -323,5 +352,11 @@ hipError_t psh_reduce_partials(const double *partials, int nmock, int grid, int 
 hipError_t psh_coord_bounds(const double *xyzw, size_t n, double *partial,
                             int blocks, hipStream_t s) {
   hipLaunchKernelGGL(bounds_kernel, dim3(blocks), dim3(256), 0, s, xyzw, n, partial);
+  return hipGetLastError();
+}
+
+hipError_t psh_fold_bounds(const double *partial, int blocks0, int blocks1, double *out,
+                           hipStream_t s) {
+  hipLaunchKernelGGL(bounds_fold_kernel, dim3(2), dim3(256), 0, s, partial, blocks0, blocks1, out);
   return hipGetLastError();
 }

@@ -268,6 +268,10 @@ hipError_t psh_fill_zero_u32(uint32_t *p, size_t n, hipStream_t s);
 #define PSH_BOUNDS_STRIDE 7
 hipError_t psh_coord_bounds(const double *xyzw, size_t n, double *partial,
     int blocks, hipStream_t s);
+// Folds the partials of two arrays (blocks0 and blocks1 of them, adjacent) into
+// PSH_BOUNDS_STRIDE values each at out (device or pinned host memory).
+hipError_t psh_fold_bounds(const double *partial, int blocks0, int blocks1, double *out,
+                           hipStream_t s);
 
 // ---------------------------------------------------------------------------
 // Learned alias correction (k_mlp.hip)
