@@ -812,6 +812,16 @@ x_bin_kernel(XBinDev a, int ntz, int H, const float2 *__restrict__ tw) {
       settle_rows<N, C, T, true>(vb);
       Passes<N, C, T, 0, true, false, 1>::run(vb, lds, twl);
     }
+    if constexpr (EPI == PSH_EPI_SURVEY0 && INTLACE && G::R == 3 && N < 640) {
+      // where a butterfly's outputs are computed decides which of their
+      // products are fused (see settle_rows): lengths 3 2^a keep the roundings
+      // of their last butterfly, made here and not at phase 1's branches
+#pragma unroll
+      for (int i = (G::NB - 1) * G::R; i < G::NB * G::R; i++) {
+        asm("" : "+v"(va[i].x), "+v"(va[i].y));
+        asm("" : "+v"(vb[INTLACE ? i : 0].x), "+v"(vb[INTLACE ? i : 0].y));
+      }
+    }
     const int c = opaque_tid<T>() % C;   // the thread's column in every pass
     const bool colok = c < ncv;
     const int kz = min(q * C + c, M);
