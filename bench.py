@@ -146,8 +146,8 @@ def roofline(stages, Ng, nmesh, npart, x_live=1.0):
     cands = {k: stages[k] for k in ("deposit", "z_r2c", "y_fft", "x_fft_bin")}
     dom = max(cands, key=lambda k: cands[k])
     per_launch = b[dom]
-    # the z and y passes launch once per mesh (plain and shifted grid); the
-    # deposit and the fused x pass cover both meshes in one launch
+    # z and y cover both meshes (plain and shifted grid) in one launch, like the
+    # deposit and the fused x pass; their figures are given per mesh
     launches = nmesh if dom in ("z_r2c", "y_fft") else 1
     t = stages[dom] / launches
     ach = per_launch / launches / (t * 1e-3) / 1e9
