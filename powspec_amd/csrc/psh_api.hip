@@ -915,16 +915,25 @@ int run_assign(psh_ctx *ctx, const std::vector<PshDevPart> &hp, int nmock,
   return PSH_OK;
 }
 
-// Forward z and y passes of the nmesh consecutive meshes from A on (real
-// fields `in`, which may be A itself).
-int fft_zy(psh_ctx *ctx, const float *in, float2 *A, int nmesh, const int *ylive, int kzlim) {
+// Forward z and y passes of the nmesh meshes from A on and, with B, of as
+// many from B on (real fields inA and inB, which may be A and B themselves;
+// nullptr: the meshes hold half-complex rows already).  One launch of a pass
+// takes both when B's meshes follow A's.  Every z pass comes before the first
+// y pass: the stage times split there.
+int fft_zy(psh_ctx *ctx, const float *inA, float2 *A, const float *inB, float2 *B, int nmesh,
+           const int *ylive, int kzlim) {
   const PshYlmR noy{};
-  if (in)
-    HIPCHK(ctx, psh_fft_z_r2c(ctx->Ng, in, A, nmesh, ctx->mstride, ctx->tw, noy, ctx->stream,
-                              kzlim));
+  const bool joined = B && B == A + (size_t)nmesh * (ctx->mstride / 2);
+  const int np = B && !joined ? 2 : 1;
+  const int n = joined ? 2 * nmesh : nmesh;
+  if (inA)
+    for (int p = 0; p < np; p++)
+      HIPCHK(ctx, psh_fft_z_r2c(ctx->Ng, p ? inB : inA, p ? B : A, n, ctx->mstride, ctx->tw, noy,
+                                ctx->stream, kzlim));
   ev_record(ctx, E_ZDONE);
-  HIPCHK(ctx, psh_fft_y(ctx->Ng, A, nmesh, ctx->mstride, ctx->tw, 0, ctx->stream, ylive,
-                        ctx->ysched));
+  for (int p = 0; p < np; p++)
+    HIPCHK(ctx, psh_fft_y(ctx->Ng, p ? B : A, n, ctx->mstride, ctx->tw, 0, ctx->stream, ylive,
+                          ctx->ysched));
   ev_record(ctx, E_YDONE);
   return PSH_OK;
 }
@@ -936,13 +945,10 @@ int run_sim_fft_bin(psh_ctx *ctx, int nmock, double *out_bins /*[nmock][nacc]*/)
   float2 *A = reinterpret_cast<float2 *>(ctx->meshA);
   float2 *B = ctx->conf.intlace ? reinterpret_cast<float2 *>(ctx->meshB) : nullptr;
   int rc;
-  // with the fused deposit the meshes hold half-complex rows already; the
-  // shifted grid's meshes follow the plain ones when every mock is in use
-  const float *real = ctx->ag.zfuse ? nullptr : ctx->meshA;
-  const bool joined = B && nmock == ctx->nmock_max;
-  if ((rc = fft_zy(ctx, real, A, nmock * (joined ? 2 : 1), ctx->d_ylive, ctx->kzlim))) return rc;
-  if (B && !joined &&
-      (rc = fft_zy(ctx, real ? ctx->meshB : nullptr, B, nmock, ctx->d_ylive, ctx->kzlim)))
+  // with the fused deposit the meshes hold half-complex rows already
+  const bool real = !ctx->ag.zfuse;
+  if ((rc = fft_zy(ctx, real ? ctx->meshA : nullptr, A, real ? ctx->meshB : nullptr, B, nmock,
+                   ctx->d_ylive, ctx->kzlim)))
     return rc;
   const int grid = xgrid_for(ctx, nmock, ctx->xres_sim);
   const int nacc = psh_xbin_nacc(ctx->bins, PSH_EPI_SIM);
@@ -1050,8 +1056,8 @@ int survey_run(psh_ctx *ctx, const std::vector<PshDevPart> &hp, std::vector<doub
 
   float2 *A = reinterpret_cast<float2 *>(ctx->meshA);
   float2 *B = reinterpret_cast<float2 *>(ctx->meshB);
-  // interlaced: A and B (adjacent) in place, else B out of place into A
-  if ((rc = fft_zy(ctx, plain, A, il ? 2 : 1, nullptr, 1 << 30))) return rc;
+  // interlaced: A and B in place, else B out of place into A
+  if ((rc = fft_zy(ctx, plain, A, ctx->meshB, il ? B : nullptr, 1, nullptr, 1 << 30))) return rc;
   PshXBinArgs a{};
   a.epi = PSH_EPI_SURVEY0;
   a.A = A;
