@@ -1723,6 +1723,7 @@ int sim_raw(psh_ctx *ctx, const std::vector<PshDevPart> &hp, std::vector<double>
   std::vector<double> sums((size_t)nacc + (mlp ? (size_t)nl * nb : 0));
   rc = kRerun;
   for (int attempt = 0; rc == kRerun; attempt++) {
+    if (attempt) ev_record(ctx, E_START);   // the stage times are the last attempt's
     if ((rc = run_assign(ctx, hp, 1, ctx->meshA, ctx->conf.intlace ? ctx->meshB : nullptr)))
       return rc;
     if ((rc = run_sim_fft_bin(ctx, 1, ctx->d_bins))) return rc;

@@ -1,5 +1,6 @@
 """Stage times (psh_ctx_timings) where a run is more than one chain of
-launches: a batch that fills only part of its context's meshes."""
+launches: a batch that fills only part of its context's meshes, and a run
+repeated after its records overflowed their buffer."""
 import numpy as np
 import pytest
 
@@ -36,3 +37,25 @@ def test_zy_split_of_a_partial_batch(psh):
             reps.append(ms[6] / (ms[5] + ms[6]))
         share[nm] = float(np.median(reps))
     assert abs(share[nmax] - share[nmax - 1]) < 0.12, share
+
+
+def test_assignment_time_after_an_overflow(psh):
+    """Particles at corners of eight tiles overflow the record buffer once;
+    the assignment time of the run that is reported holds none of the first
+    run's transforms."""
+    Ng, n = 512, 100000
+    rng = np.random.default_rng(2)
+    d = np.empty((n, 4))
+    d[:, :3] = (8 * rng.integers(0, Ng // 8, (n, 3)) + 7.6) * (L / Ng)
+    d[:, 3] = 1.0
+    conf = psh.make_conf(gsize=Ng, assign=psh.PCS, intlace=True, bsize=L, kbin=0.02)
+    ctx = psh.Context(conf)
+    ctx.set_tiles((8, 8, 8))
+    ctx.set_profiling(True)
+    few = psh.DeviceArray.from_numpy(_uniform(100, 3))
+    for _ in range(2):
+        ctx.run_device(few, 100, 100.0)
+    ctx.run_device(psh.DeviceArray.from_numpy(d), n, float(n))
+    ms = ctx.timings()
+    # [0] less the bucketing and deposit kernels: what came before them
+    assert ms[0] - ms[4] - ms[7] < 0.5 * (ms[1] + ms[2]), ms
