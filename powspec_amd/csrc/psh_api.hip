@@ -1718,8 +1718,6 @@ int sim_raw(psh_ctx *ctx, const std::vector<PshDevPart> &hp, std::vector<double>
   if ((rc = ensure_partials(ctx, 1, xgrid_for(ctx, 1, ctx->xres_sim), nacc, 1))) return rc;
   if (mlp && (rc = ensure_alias_rows(ctx))) return rc;
   ensure_results(ctx, (size_t)nacc + (size_t)nl * nb);
-  ctx->last_norm = norm;
-  ctx->last_shot = shot;
   std::vector<double> sums((size_t)nacc + (mlp ? (size_t)nl * nb : 0));
   rc = kRerun;
   for (int attempt = 0; rc == kRerun; attempt++) {
@@ -1752,7 +1750,10 @@ int sim_raw(psh_ctx *ctx, const std::vector<PshDevPart> &hp, std::vector<double>
   }
   if (rc == PSH_ERR_CATA) return sim_box_error(ctx, hp);
   if (rc) return rc;
+  // the cells and their normalisation together: a failed run leaves both
   ctx->cells.assign(sums.begin(), sums.begin() + nacc);
+  ctx->last_norm = norm;
+  ctx->last_shot = shot;
   if (mlp) {
     raw.assign(sums.begin() + nacc, sums.end());
   } else {
