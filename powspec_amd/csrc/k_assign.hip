@@ -22,6 +22,7 @@
 #include "psh_internal.h"
 #include "fft_core.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace {
@@ -1091,16 +1092,16 @@ assign_deposit(PshAssignGeom g, const uint32_t *__restrict__ starts,
                const Rec *__restrict__ recs, size_t rec_cap,
                float *__restrict__ meshA, float *__restrict__ meshB,
                size_t mstride, const int *__restrict__ flags, int P2, int lead, int cells,
-               uint32_t ntiles) {
+               uint32_t ntiles, uint32_t b0) {
   using AT = typename Acc<WIDE>::T;
   extern __shared__ __align__(16) long long ldsraw[];
   AT *lds = reinterpret_cast<AT *>(ldsraw) + lead;
-  uint32_t tile = blockIdx.x;
+  const uint32_t b = blockIdx.x + b0;
+  uint32_t tile = b;
   bool shifted = false;
   if (INTLACE) {
     // blocks 16 n + (0..7) and 16 n + 8 + (0..7): the grids of tiles 8 n + (0..7)
-    const uint32_t b = blockIdx.x, half = gridDim.x >> 1;
-    if (half & 7) {
+    if (ntiles & 7) {
       shifted = b & 1;
       tile = b >> 1;
     } else {
@@ -1301,9 +1302,14 @@ hipError_t launch_deposit(const PshAssignGeom &g, size_t ntiles,
   const size_t per = g.wide ? 8 : 16;
   unsigned threads = 256;
   while (threads < 1024 && threads * per < tcells) threads *= 2;
-  hipLaunchKernelGGL(k, dim3((unsigned)(ntiles * (g.intlace ? 2 : 1))), dim3(threads), lds, s, g,
-                     starts, recs, rec_cap, meshA, meshB, mstride, flags, pitch, lead, (int)cells,
-                     (uint32_t)ntiles);
+  // one launch, unless its threads pass the 32 bits that a launch counts them
+  // in (both grids of N = 1024 in 4x4x8 tiles: 2^32)
+  const size_t blocks = ntiles * (g.intlace ? 2 : 1);
+  const size_t most = (0xffffffffu / threads) & ~15u;   // whole rounds of the XCDs
+  for (size_t b0 = 0; b0 < blocks; b0 += most)
+    hipLaunchKernelGGL(k, dim3((unsigned)std::min(most, blocks - b0)), dim3(threads), lds, s, g,
+                       starts, recs, rec_cap, meshA, meshB, mstride, flags, pitch, lead,
+                       (int)cells, (uint32_t)ntiles, (uint32_t)b0);
   return hipGetLastError();
 }
 
