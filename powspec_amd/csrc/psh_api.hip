@@ -702,8 +702,7 @@ int ensure_assign_scratch(psh_ctx *ctx, int nmock, int nparts, size_t ntotal) {
     if ((rc = dev_alloc(ctx, &ctx->counts, ntiles + 1))) return rc;
     if ((rc = dev_alloc(ctx, &ctx->starts, ntiles + 1))) return rc;
     if ((rc = dev_alloc(ctx, &ctx->cursors, ntiles + 1))) return rc;
-    if ((rc = dev_alloc(ctx, &ctx->scan_tmp, psh_assign_scan_bytes(ntiles) / 4 + 64)))
-      return rc;
+    if ((rc = dev_alloc(ctx, &ctx->scan_tmp, psh_assign_scan_bytes(ntiles) / 4))) return rc;
     ctx->tiles_cap = ntiles + 1;
   }
   if (nparts > ctx->parts_cap) {
@@ -1255,7 +1254,9 @@ void normalise_survey(const psh_ctx *ctx, const double *raw, double shot, double
 // the first bucketing kernel, now for 37, both in a profiler's trace).
 int bounds_device(psh_ctx *ctx, const double *const *d, const size_t *n, int narr, double mn[3],
                   double mx[3], double *wsum = nullptr) {
-  constexpr int kBlocks = 1024;
+  // in the static scratch, which may hold little more than the run, both
+  // arrays' partials share what one array's take otherwise
+  const int kBlocks = ctx->arena ? 511 : 1024;
   int rc;
   if (!ctx->d_bounds &&
       (rc = dev_alloc(ctx, &ctx->d_bounds, (size_t)2 * (kBlocks + 1) * PSH_BOUNDS_STRIDE)))
