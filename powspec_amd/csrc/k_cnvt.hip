@@ -331,13 +331,14 @@ struct Workspaces {
         }
     }
     w.device = dev;
-    if (hipMalloc((void **)&w.dev, sizeof(CnvtDev)) == hipSuccess &&
-        hipMalloc((void **)&w.part, sizeof(double) * PSH_BOUNDS_STRIDE * kBoundsBlocks) ==
+    if (psh_malloc(&w.dev, sizeof(CnvtDev)) == hipSuccess &&
+        psh_malloc(&w.part, sizeof(double) * PSH_BOUNDS_STRIDE * kBoundsBlocks) ==
             hipSuccess &&
         hipHostMalloc((void **)&w.hout, 3 * sizeof(double), hipHostMallocDefault) == hipSuccess &&
         hipMemcpy(w.dev->rules, rules.data(), sizeof(w.dev->rules), hipMemcpyHostToDevice) ==
             hipSuccess)
       return true;
+    (void)hipGetLastError();   // (of the host allocation or the copy)
     free_workspace(w);
     return false;
   }
@@ -434,7 +435,7 @@ extern "C" int psh_cnvt_device(const psh_cnvt *cv, psh_data *const *d_data, cons
     if (!cv->dsp || cv->nsp < 2) return PSH_ERR_ARG;
     std::vector<double> ypp = spline_ypp(cv->zsp, cv->dsp, cv->nsp);
     double *tab = nullptr;
-    if (hipMalloc(&tab, sizeof(double) * 3 * cv->nsp) != hipSuccess) return PSH_ERR_MEMORY;
+    if (psh_malloc(&tab, sizeof(double) * 3 * cv->nsp) != hipSuccess) return PSH_ERR_MEMORY;
     bool ok = hipMemcpy(tab, cv->zsp, sizeof(double) * cv->nsp, hipMemcpyHostToDevice) ==
                   hipSuccess &&
               hipMemcpy(tab + cv->nsp, cv->dsp, sizeof(double) * cv->nsp,
@@ -481,7 +482,7 @@ extern "C" int psh_cnvt_coord(const psh_cnvt *cv, psh_cata *cat) {
   int rc = PSH_OK;
   for (size_t a = 0; a < host.size(); a++) {
     psh_data *d = nullptr;
-    if (hipMalloc(&d, sizeof(psh_data) * cnt[a]) != hipSuccess ||
+    if (psh_malloc(&d, sizeof(psh_data) * cnt[a]) != hipSuccess ||
         hipMemcpy(d, host[a], sizeof(psh_data) * cnt[a], hipMemcpyHostToDevice) !=
             hipSuccess) {
       if (d) (void)hipFree(d);

@@ -262,11 +262,11 @@ extern "C" int psh_gen_clustered_box(const psh_box_spec *g, psh_data **d_out, si
   const int pblocks = 1024;
   uint32_t total = 0;
   auto ok = [](hipError_t e) { return e == hipSuccess; };
-  if (!ok(hipMalloc(&R, sizeof(float) * mfl)) || !ok(hipMalloc(&Z, sizeof(float) * mfl)) ||
-      !ok(hipMalloc(&counts, sizeof(uint32_t) * ncell)) ||
-      !ok(hipMalloc(&starts, sizeof(uint32_t) * (ncell + 1))) ||
-      !ok(hipMalloc(&tmp, psh_assign_scan_bytes(ncell))) ||
-      !ok(hipMalloc(&part, sizeof(double) * 2 * pblocks))) {
+  if (!ok(psh_malloc(&R, sizeof(float) * mfl)) || !ok(psh_malloc(&Z, sizeof(float) * mfl)) ||
+      !ok(psh_malloc(&counts, sizeof(uint32_t) * ncell)) ||
+      !ok(psh_malloc(&starts, sizeof(uint32_t) * (ncell + 1))) ||
+      !ok(psh_malloc(&tmp, psh_assign_scan_bytes(ncell))) ||
+      !ok(psh_malloc(&part, sizeof(double) * 2 * pblocks))) {
     rc = PSH_ERR_MEMORY;
     goto done;
   }
@@ -313,7 +313,7 @@ extern "C" int psh_gen_clustered_box(const psh_box_spec *g, psh_data **d_out, si
       !ok(hipMemcpyAsync(&total, starts + ncell, sizeof(uint32_t), hipMemcpyDeviceToHost, s)) ||
       !ok(hipStreamSynchronize(s)))
     goto done;
-  if (!ok(hipMalloc((void **)d_out, sizeof(psh_data) * (total ? total : 1)))) {
+  if (!ok(psh_malloc(d_out, sizeof(psh_data) * (total ? total : 1)))) {
     rc = PSH_ERR_MEMORY;
     goto done;
   }

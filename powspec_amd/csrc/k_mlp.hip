@@ -535,8 +535,8 @@ extern "C" int psh_mlp_grad(const float *d_params, const float *d_X, const float
   if (!d_params || !d_X || !d_T || !d_grads || B < 1) return PSH_ERR_ARG;
   float *d_loss = nullptr;
   long long *G = nullptr;
-  if (hipMalloc(&d_loss, sizeof(float)) != hipSuccess) return PSH_ERR_MEMORY;
-  if (hipMalloc(&G, sizeof(long long) * NPAR) != hipSuccess) {
+  if (psh_malloc(&d_loss, sizeof(float)) != hipSuccess) return PSH_ERR_MEMORY;
+  if (psh_malloc(&G, sizeof(long long) * NPAR) != hipSuccess) {
     (void)hipFree(d_loss);
     return PSH_ERR_MEMORY;
   }
@@ -558,8 +558,8 @@ extern "C" int psh_mlp_train(float *d_params, const float *d_X, const float *d_T
   if (!d_params || !d_X || !d_T || B < 1 || batch < 16 || epochs < 0) return PSH_ERR_ARG;
   float *buf = nullptr;
   long long *G = nullptr;
-  if (hipMalloc(&buf, sizeof(float) * (2 * NPAR + 1)) != hipSuccess) return PSH_ERR_MEMORY;
-  if (hipMalloc(&G, sizeof(long long) * NPAR) != hipSuccess) {
+  if (psh_malloc(&buf, sizeof(float) * (2 * NPAR + 1)) != hipSuccess) return PSH_ERR_MEMORY;
+  if (psh_malloc(&G, sizeof(long long) * NPAR) != hipSuccess) {
     (void)hipFree(buf);
     return PSH_ERR_MEMORY;
   }

@@ -335,7 +335,7 @@ int ctx_malloc(psh_ctx *ctx, void **p, size_t bytes) {
   if (fault_alloc_now())
     return set_err(ctx, PSH_ERR_MEMORY,
                    "device allocation of %zu bytes failed: injected fault", bytes);
-  hipError_t e = hipMalloc(p, bytes);
+  hipError_t e = psh_malloc(p, bytes);
   if (e != hipSuccess) {
     *p = nullptr;
     return set_err(ctx, PSH_ERR_MEMORY, "device allocation of %zu bytes failed: %s", bytes,
@@ -2317,7 +2317,7 @@ extern "C" int psh_device_malloc(void **ptr, size_t bytes) {
   *ptr = nullptr;
   int n = 0;
   if (hipGetDeviceCount(&n) != hipSuccess || n < 1) return PSH_ERR_DEVICE;
-  return hipMalloc(ptr, bytes) == hipSuccess ? PSH_OK : PSH_ERR_MEMORY;
+  return psh_malloc(ptr, bytes) == hipSuccess ? PSH_OK : PSH_ERR_MEMORY;
 }
 
 extern "C" int psh_device_free(void *ptr) {
@@ -2607,7 +2607,7 @@ extern "C" int psh_autotune(const psh_conf *conf, const psh_data *d_data, const 
     for (int m = 0; m < nmock; m++) ws[m] = (double)(off[m + 1] - off[m]);
   } else {
     const size_t ntot = npart * (size_t)nmock;
-    if (hipMalloc(&d, sizeof(psh_data) * ntot) != hipSuccess) {
+    if (psh_malloc(&d, sizeof(psh_data) * ntot) != hipSuccess) {
       psh_ctx_destroy(ctx);
       return PSH_ERR_MEMORY;
     }

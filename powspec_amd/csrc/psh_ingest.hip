@@ -417,7 +417,7 @@ int ensure_partial(psh_ingest *g, size_t blocks) {
   if (g->partial) (void)hipFree(g->partial);
   g->partial = nullptr;
   g->partial_cap = 0;
-  if (hipMalloc((void **)&g->partial, sizeof(double) * 3 * blocks) != hipSuccess)
+  if (psh_malloc(&g->partial, sizeof(double) * 3 * blocks) != hipSuccess)
     return ing_err(g, PSH_ERR_MEMORY, "device allocation of the ingest sums failed");
   g->partial_cap = blocks;
   return PSH_OK;
@@ -503,7 +503,7 @@ int grow(psh_ingest *g, T **p, size_t &cap, size_t need) {
   *p = nullptr;
   cap = 0;
   const size_t n = need + need / 4 + 1024;
-  if (hipMalloc((void **)p, sizeof(T) * n) != hipSuccess)
+  if (psh_malloc(p, sizeof(T) * n) != hipSuccess)
     return ing_err(g, PSH_ERR_MEMORY, "device allocation for the ASCII parser failed");
   cap = n;
   return PSH_OK;
@@ -563,7 +563,7 @@ int run_ascii(psh_ingest *g, AsciiJob job, int sim, double *d_out, size_t cap) {
   std::vector<double> hp;
   int rc;
   if (!job.prog.empty()) {
-    if (!g->dprog && hipMalloc((void **)&g->dprog, sizeof(pshexpr::Ins) * 7 * pshexpr::kMaxIns))
+    if (!g->dprog && psh_malloc(&g->dprog, sizeof(pshexpr::Ins) * 7 * pshexpr::kMaxIns))
       return ing_err(g, PSH_ERR_MEMORY, "cannot allocate the expression programs");
     ICHK(g, hipMemcpyAsync(g->dprog, job.prog.data(), sizeof(pshexpr::Ins) * job.prog.size(),
                            hipMemcpyHostToDevice, g->stream));
@@ -718,7 +718,7 @@ extern "C" int psh_ingest_create(size_t chunk_objects, psh_ingest **out) {
   }
   for (int s = 0; s < 2; s++) {
     if (hipHostMalloc(&g->pinned[s], bytes, hipHostMallocDefault) != hipSuccess ||
-        hipMalloc(&g->stage[s], bytes) != hipSuccess ||
+        psh_malloc(&g->stage[s], bytes) != hipSuccess ||
         hipEventCreateWithFlags(&g->done[s], hipEventDisableTiming) != hipSuccess ||
         hipEventRecord(g->done[s], g->stream) != hipSuccess) {
       psh_ingest_destroy(g);

@@ -19,6 +19,15 @@
 // fields of one survey pole l > 0 that one x pass bins together (2 l + 1 <= 13)
 #define PSH_MAX_YLM_FIELDS 13
 
+// hipMalloc whose failure is the caller's to report and nobody else's: left
+// in place, the next launch check of any call on this thread returns it.
+template <class T>
+inline hipError_t psh_malloc(T **p, size_t bytes) {
+  const hipError_t e = hipMalloc((void **)p, bytes);
+  if (e != hipSuccess) (void)hipGetLastError();
+  return e;
+}
+
 // Per-axis FP64 tables used by the binning epilogues, device resident.
 // For axis a and index i (signed frequency i' for x,y; i for z):
 //   kv[a][i] = vec_a * i'          (vec_a = 2 pi / L_a)
