@@ -109,7 +109,7 @@ struct psh_ctx {
   PshAssignGeom ag{};
   size_t ntiles_mock = 0;
   uint32_t *counts = nullptr, *starts = nullptr, *cursors = nullptr;
-  uint32_t *whist = nullptr;   // per-workgroup tile histograms of the count pass
+  uint32_t *whist = nullptr;   // per workgroup, where its ranges of the buckets begin
   size_t whist_cap = 0, whist_words = 0;
   uint32_t *scan_tmp = nullptr;
   size_t tiles_cap = 0;
@@ -691,6 +691,25 @@ void drop_graph(psh_ctx *ctx) {
   ctx->graph = nullptr;
 }
 
+// A buffer of `need` records.  The bucket ranges, which a run can do without,
+// give way when there is no memory for both.
+int alloc_records(psh_ctx *ctx, size_t need) {
+  drop_graph(ctx);
+  ctx_free(ctx, ctx->records);
+  ctx->records = nullptr;
+  ctx->rec_cap = 0;
+  const std::string keep = ctx->err;
+  int rc = ctx_malloc(ctx, &ctx->records, need * psh_assign_record_bytes());
+  if (rc && ctx->whist) {
+    ctx_free(ctx, ctx->whist);
+    ctx->whist = nullptr;
+    ctx->whist_cap = ctx->whist_words = 0;
+    if (!(rc = ctx_malloc(ctx, &ctx->records, need * psh_assign_record_bytes()))) ctx->err = keep;
+  }
+  if (!rc) ctx->rec_cap = need;
+  return rc;
+}
+
 int ensure_assign_scratch(psh_ctx *ctx, int nmock, int nparts, size_t ntotal) {
   int rc;
   const size_t ntiles = ctx->ntiles_mock * nmock;
@@ -714,13 +733,20 @@ int ensure_assign_scratch(psh_ctx *ctx, int nmock, int nparts, size_t ntotal) {
   if (!ctx->d_flags) {
     if ((rc = dev_alloc(ctx, &ctx->d_flags, 4))) return rc;
   }
+  // expected (particle, tile) pairs: prod_a (1 + (W' - 1) / T_a), W' the
+  // union window; 1.5x margin, grown on overflow
+  const int W = ctx->conf.assign + 1 + (ctx->conf.intlace ? 1 : 0);
+  double dup = 1.0;
+  for (int a = 0; a < 3; a++) dup *= 1.0 + (double)(W - 1) / ctx->ag.tile[a];
+  size_t need = (size_t)(ntotal * dup * 1.5) + 4096;
+  if (need > ctx->rec_cap && (rc = alloc_records(ctx, need))) return rc;
   ctx->whist_words = psh_assign_whist_words(ctx->ag, ntotal);
   if (ctx->whist_words > ctx->whist_cap) {
     drop_graph(ctx);
     ctx_free(ctx, ctx->whist);
     ctx->whist = nullptr;
     ctx->whist_cap = 0;
-    // optional: without the histograms the fill pass recounts
+    // optional: without them the fill pass recounts
     const std::string keep = ctx->err;
     if (ctx_malloc(ctx, (void **)&ctx->whist, sizeof(uint32_t) * ctx->whist_words) == PSH_OK) {
       ctx->whist_cap = ctx->whist_words;
@@ -729,34 +755,10 @@ int ensure_assign_scratch(psh_ctx *ctx, int nmock, int nparts, size_t ntotal) {
       ctx->err = keep;
     }
   }
-  // expected (particle, tile) pairs: prod_a (1 + (W' - 1) / T_a), W' the
-  // union window; 1.5x margin, grown on overflow
-  const int W = ctx->conf.assign + 1 + (ctx->conf.intlace ? 1 : 0);
-  double dup = 1.0;
-  for (int a = 0; a < 3; a++) dup *= 1.0 + (double)(W - 1) / ctx->ag.tile[a];
-  size_t need = (size_t)(ntotal * dup * 1.5) + 4096;
-  if (need > ctx->rec_cap) {
-    drop_graph(ctx);
-    ctx_free(ctx, ctx->records);
-    ctx->records = nullptr;
-    ctx->rec_cap = 0;
-    if ((rc = ctx_malloc(ctx, &ctx->records, need * psh_assign_record_bytes()))) return rc;
-    ctx->rec_cap = need;
-  }
   return PSH_OK;
 }
 
-int grow_records(psh_ctx *ctx) {
-  drop_graph(ctx);
-  const size_t need = ctx->rec_cap * 2;
-  ctx_free(ctx, ctx->records);
-  ctx->records = nullptr;
-  ctx->rec_cap = 0;
-  int rc;
-  if ((rc = ctx_malloc(ctx, &ctx->records, need * psh_assign_record_bytes()))) return rc;
-  ctx->rec_cap = need;
-  return PSH_OK;
-}
+int grow_records(psh_ctx *ctx) { return alloc_records(ctx, ctx->rec_cap * 2); }
 
 int ensure_partials(psh_ctx *ctx, int nmock, int grid, int nacc, int slots) {
   int rc;
