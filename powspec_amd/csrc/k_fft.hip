@@ -1133,8 +1133,8 @@ x_bin_kernel(XBinDev a, int ntz, int H, const float2 *__restrict__ tw) {
         }
       };
       // Bin of pair k and 1 / |k|; -1 outside the window, -2 undecided in
-      // FP32.  |k|^2 is far from the denormal range: the bare reciprocal
-      // square root.
+      // FP32.  The bare reciprocal square root takes a denormal |k|^2 for zero:
+      // |k| is then infinite or no number, and the pair undecided.
       auto pair_bin = [&](int k, const Ops &o, float &rs) -> int {
         const float k2f = o.ks + ksqyz;
         rs = __builtin_amdgcn_rsqf(k2f);
@@ -1195,7 +1195,7 @@ x_bin_kernel(XBinDev a, int ntz, int H, const float2 *__restrict__ tw) {
           const int kb = bin_exact(b, GS ? a.ax.ksq[0][i] : ksqx[i], ksqy, ksqz, kz);
           const int kw = kb - a.kb0;
           if (kb >= 0 && (unsigned)kw < (unsigned)a.nbw)
-            add_pair(std::false_type{}, i, kw, __builtin_amdgcn_rsqf(u.ks + ksqyz), u);
+            add_pair(std::false_type{}, i, kw, rsqrtf(u.ks + ksqyz), u);
         }
       }
     }
