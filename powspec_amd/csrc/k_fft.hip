@@ -965,7 +965,7 @@ x_bin_kernel(XBinDev a, int ntz, int H, const float2 *__restrict__ tw) {
 #pragma unroll
       for (int i = 0; i < V; i++) {
         va[i] = make_float2(0.f, 0.f);
-        if (INTLACE) vb[INTLACE ? i : 0] = make_float2(0.f, 0.f);
+        vb[INTLACE ? i : 0] = make_float2(0.f, 0.f);
       }
     }
 
@@ -1160,7 +1160,7 @@ x_bin_kernel(XBinDev a, int ntz, int H, const float2 *__restrict__ tw) {
           if (kb >= 0 && (unsigned)kw < (unsigned)a.nbw) add_pair(low4, i0 + k * S, kw, rs, o);
         }
       };
-      static_assert(KMAX < 32, "one bit per pair");
+      static_assert(KMAX <= 16, "pairs to unroll, one bit each");
       Ops o = fetch(0);
       auto unrolled = [&]() {
 #pragma unroll
@@ -1170,22 +1170,17 @@ x_bin_kernel(XBinDev a, int ntz, int H, const float2 *__restrict__ tw) {
           if (k < KMAX || kend == KMAX) step(std::true_type{}, k, cur);
         }
       };
-      auto rolled = [&](auto low4) {
+      auto rolled = [&]() {
 #pragma unroll 1
         for (int k = 0; k <= kend; k++) {
           const Ops cur = o;
           if (k < KMAX) o = fetch(k + 1);
-          step(low4, k, cur);
+          step(std::false_type{}, k, cur);
         }
       };
       const bool low = !GEN || a.low4;
-      if constexpr (KMAX <= 16) {
-        if (low) unrolled();
-        else rolled(std::false_type{});
-      } else {
-        if (low) rolled(std::true_type{});
-        else rolled(std::false_type{});
-      }
+      if (low) unrolled();
+      else rolled();
       if (__ballot(undecided != 0)) {
         const double ksqy = a.ax.ksq[1][y], ksqz = a.ax.ksq[2][kz];
 #pragma unroll 1
