@@ -5,15 +5,18 @@
 //
 // Design:
 //  1. count:   per particle, the FP64 cell coordinate decides the base cell of
-//              the window on the plain grid and on the half-cell-shifted grid
-//              (same operation order as the reference, contraction off); the
-//              union window is mapped to the 1..8 mesh tiles it touches and a
-//              per-tile counter is incremented.
+//              the window on the plain grid (same operation order as the
+//              reference, contraction off) and the half-cell-shifted grid's
+//              offset from it; the union window is mapped to the 1..8 mesh
+//              tiles it touches and each tile's counter, in an LDS window of
+//              counters per workgroup, is incremented.
 //  2. scan:    exclusive prefix sum of the tile counters.
-//  3. fill:    each (particle, tile) pair is written as a 24-byte record.
-//  4. deposit: one workgroup per tile accumulates its records into an LDS
-//              copy of the tile (fixed-point integer LDS atomics, both grids)
-//              and writes the tile to HBM once with coalesced row stores.
+//  3. fill:    each (particle, tile) pair is written as a 24-byte record of
+//              cells relative to the tile.
+//  4. deposit: one workgroup per tile and grid accumulates the tile's records
+//              into an LDS copy of the tile (fixed-point integer LDS atomics)
+//              and writes the tile to HBM once with coalesced row stores
+//              (tiles of whole z rows: both grids, and their z transform).
 //              Every mesh cell is written exactly once: no zeroing pass, no
 //              global atomics.
 // Surveys assign data and randoms into the same tiles with weights w and

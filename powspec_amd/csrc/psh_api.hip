@@ -230,8 +230,9 @@ bool is_pow2(int n) { return n > 0 && (n & (n - 1)) == 0; }
 // window width W = scheme + 1 along every axis (a window plus the shifted
 // grid's extra cell then meets at most two tiles per axis, which the
 // bucketing assumes), rows of at least 4 cells along z, LDS of both grids
-// (z rows padded for the window) within 160 KB at `cell_bytes` per cell
-// (4: 32-bit fixed point of boxes, 8: 64-bit of surveys).
+// (z rows padded for the window; a workgroup of the fused z transform holds
+// both) within 160 KB at `cell_bytes` per cell (4: 32-bit fixed point of
+// boxes, 8: 64-bit of surveys).
 bool tiles_ok(const int t[3], int scheme, int intlace, int cell_bytes) {
   for (int a = 0; a < 3; a++)
     if (!is_pow2(t[a]) || t[a] > 2048 || t[a] < scheme + 1) return false;
