@@ -332,8 +332,9 @@ __device__ __forceinline__ uint32_t run_increment(uint32_t *hist, uint32_t t, bo
 // sizes -- and counts their (particle, tile) pairs in LDS, in a window of
 // the tiles of its first particle's mock: all of them up to kWinTiles, else
 // kWinTilesBig around the first particle's tile (a catalogue ordered by x
-// stays inside; the x tile index is the slowest).  Pairs outside the window
-// or of another mock are singles, counted and placed with global atomics.
+// stays inside; the x tile index is the slowest), or none of them for few
+// particles (kWinParticles).  Pairs outside the window or of another mock are
+// singles, counted and placed with global atomics.
 //  count: each nonzero window counter is added to the tile's count with one
 //         atomic, whose return value -- the place of the workgroup's range in
 //         the bucket -- goes to whist;
@@ -356,10 +357,18 @@ __device__ __forceinline__ uint32_t run_increment(uint32_t *hist, uint32_t t, bo
 constexpr int kChunkMax = 16384;
 constexpr int kWinTiles = 32768;      // 128 KB of LDS, one workgroup per CU
 constexpr int kWinTilesBig = 16384;   // 64 KB, two
+// ... and none of them for fewer particles than this, whose few workgroups of
+// at least half a window would take longer than global atomics for every
+// pair.  Count + scan + fill, global / window, interlaced: 2e4 random
+// particles and 262144 tiles, CIC 0.04 / 0.20 ms, PCS 0.05 / 0.36; 131072
+// tiles (N = 1024), CIC 0.04 / 0.14, 5e5 0.11 / 0.14, 1e6 0.18 / 0.17, in
+// space order 2e5 0.07 / 0.08, 5e5 0.09 / 0.09, 4e6 0.44 / 0.26.
+constexpr size_t kWinParticles = (size_t)1 << 19;
 constexpr int kBucketThreads = 1024;
 
-__host__ __device__ inline uint32_t window_tiles(uint32_t tpm) {
-  return tpm <= (uint32_t)kWinTiles ? tpm : (uint32_t)kWinTilesBig;
+__host__ __device__ inline uint32_t window_tiles(uint32_t tpm, size_t ntotal) {
+  if (tpm <= (uint32_t)kWinTiles) return tpm;
+  return ntotal < kWinParticles ? 0u : (uint32_t)kWinTilesBig;
 }
 
 // Particles per workgroup: as many as leave two workgroups for each of the
@@ -367,7 +376,7 @@ __host__ __device__ inline uint32_t window_tiles(uint32_t tpm) {
 // (whose clearing and flushing a chunk pays for).
 inline size_t bucket_chunk(const PshAssignGeom &g, size_t ntotal) {
   if (g.lean) return kChunkMax;
-  const uint32_t win = window_tiles((uint32_t)g.ntile[0] * g.ntile[1] * g.ntile[2]);
+  const uint32_t win = window_tiles((uint32_t)g.ntile[0] * g.ntile[1] * g.ntile[2], ntotal);
   size_t c = 256;
   while (c < (size_t)kChunkMax && (2 * c * 512 <= ntotal || c * 2 < win)) c *= 2;
   return c;
@@ -381,14 +390,14 @@ assign_bucket(PshAssignGeom g, const DevPart *__restrict__ parts, int nparts, si
               int *__restrict__ flags, uint32_t *__restrict__ whist) {
   extern __shared__ uint32_t hist[];
   const uint32_t tpm = (uint32_t)g.ntile[0] * g.ntile[1] * g.ntile[2];
-  const uint32_t win = window_tiles(tpm);
+  const uint32_t win = window_tiles(tpm, ntotal);
   const uint32_t T = blockDim.x;
   const size_t c0 = (size_t)blockIdx.x * chunk;
   const size_t c1 = min(ntotal, c0 + (size_t)chunk);
   const UPart P0 = uniform_part(parts, nparts, c0);
   const int mock0 = P0.mock;
   uint32_t wbase = 0;
-  if (win < tpm) {
+  if (win && win < tpm) {
     // a quarter of the window below the first particle's tile
     const Loaded L0 = load_particle(parts, nparts, P0, c0, true);
     PartTiles pt;
@@ -478,7 +487,7 @@ assign_bucket(PshAssignGeom g, const DevPart *__restrict__ parts, int nparts, si
   }
   if (wh) {
     for (uint32_t i = threadIdx.x; i < win; i += T) hist[i] = starts[mbase0 + i] + wh[i];
-  } else {
+  } else if (win) {
     clear();
     count_pairs(std::false_type{}, false);
     for (uint32_t i = threadIdx.x; i < win; i += T)
@@ -1372,7 +1381,7 @@ size_t psh_assign_whist_words(const PshAssignGeom &g, size_t ntotal) {
   const uint32_t tpm = (uint32_t)g.ntile[0] * g.ntile[1] * g.ntile[2];
   if (ntotal == 0 || (g.lean && tpm > (uint32_t)kWinTiles)) return 0;
   const size_t chunk = bucket_chunk(g, ntotal);
-  const size_t words = (ntotal + chunk - 1) / chunk * window_tiles(tpm);
+  const size_t words = (ntotal + chunk - 1) / chunk * window_tiles(tpm, ntotal);
   return words <= ((size_t)1 << 30) ? words : 0;   // at most 4 GB
 }
 
@@ -1402,7 +1411,7 @@ hipError_t launch_bucket(bool fill, const PshAssignGeom &g, const PshDevPart *pa
                          const uint32_t *starts, Rec *recs, size_t rec_cap, int *flags,
                          uint32_t *whist, hipStream_t s) {
   const uint32_t tpm = (uint32_t)g.ntile[0] * g.ntile[1] * g.ntile[2];
-  const size_t lds = sizeof(uint32_t) * window_tiles(tpm);
+  const size_t lds = sizeof(uint32_t) * window_tiles(tpm, ntotal);
   const uint32_t chunk = (uint32_t)bucket_chunk(g, ntotal);
   // two particles per thread at least, for the loads in flight
   unsigned threads = kBucketThreads;

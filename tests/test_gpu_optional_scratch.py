@@ -26,11 +26,12 @@ def faults(psh):
 @pytest.mark.parametrize("graph", [None, False, True])
 @pytest.mark.parametrize("k", [1, 2])
 def test_one_allocation_less_for_a_larger_run(faults, k, graph):
-    """A context that ran a small catalogue (262144 tiles) grows its buffers
-    for a larger one; any one of the two allocations may fail."""
+    """A context that ran a small catalogue (262144 tiles, enough particles
+    for the ranges) grows its buffers for a larger one; any one of the two
+    allocations may fail."""
     P = faults
-    n = 300000
-    small, large = _uniform(1000, 1), _uniform(n, 2)
+    m0, n = 530000, 1200000
+    small, large = _uniform(m0, 1), _uniform(n, 2)
     w = float(large[:, 3].sum())
     conf = P.make_conf(gsize=256, assign=P.TSC, intlace=True, bsize=L, kbin=0.02)
     ds, dl = P.DeviceArray.from_numpy(small), P.DeviceArray.from_numpy(large)
@@ -42,7 +43,7 @@ def test_one_allocation_less_for_a_larger_run(faults, k, graph):
             return ctx.run_device(dev, m, ws)
         return ctx.run_batch(dev, [0, m], [ws], graph=graph)[0]
 
-    run(ds, 1000, float(small[:, 3].sum()))
+    run(ds, m0, float(small[:, 3].sum()))
     P.fault_inject(P.FAULT_ALLOC, k)
     first = run(dl, n, w)
     P.fault_inject(P.FAULT_ALLOC, 0)
