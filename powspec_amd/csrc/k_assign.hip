@@ -375,8 +375,8 @@ __host__ __device__ inline uint32_t window_tiles(uint32_t tpm, size_t ntotal) {
 // 256 CUs, between 256 and kChunkMax, and at least half of the window
 // (whose clearing and flushing a chunk pays for).
 inline size_t bucket_chunk(const PshAssignGeom &g, size_t ntotal) {
-  if (g.lean) return kChunkMax;
   const uint32_t win = window_tiles((uint32_t)g.ntile[0] * g.ntile[1] * g.ntile[2], ntotal);
+  if (g.lean && win) return kChunkMax;   // few workgroups' ranges to keep
   size_t c = 256;
   while (c < (size_t)kChunkMax && (2 * c * 512 <= ntotal || c * 2 < win)) c *= 2;
   return c;
@@ -1338,14 +1338,20 @@ hipError_t launch_deposit(const PshAssignGeom &g, size_t ntiles,
                                          : assign_deposit<SCHEME, false, false, false>));
   raise((const void *)k);
   // one thread per 16 cells (per 8 of 64 bits, whose LDS admits half the
-  // workgroups: survey, N = 512, 1.89 -> 1.64 ms), 256..1024
+  // workgroups: survey, N = 512, 1.89 -> 1.64 ms), 256..1024.  Two waves for
+  // tiles of less than 2048 cells when there are so many of them that starting
+  // the waves takes the time, twice what fills the chip: interlaced, both
+  // grids in a workgroup of 256 / 256 for each / 128 for each: N = 256 CIC,
+  // 2e4 particles, 4x4x4 0.24 / 0.43 / 0.24 ms; N = 512 in 4x4x64
+  // 0.20 / 0.29 / 0.19, PCS 2e6 0.38 / 0.41 / 0.27; few tiles with many
+  // records each want the waves: N = 64 in 4x4x64 PCS 2e6 0.41 / 0.23 / 0.44.
   const size_t tcells = (size_t)g.tile[0] * g.tile[1] * g.tile[2];
+  const size_t blocks = ntiles * (g.intlace ? 2 : 1);
   const size_t per = g.wide ? 8 : 16;
-  unsigned threads = 256;
+  unsigned threads = tcells < 2048 && blocks >= 8192 ? 128 : 256;
   while (threads < 1024 && threads * per < tcells) threads *= 2;
   // one launch, unless its threads pass the 32 bits that a launch counts them
-  // in (both grids of N = 1024 in 4x4x8 tiles: 2^32)
-  const size_t blocks = ntiles * (g.intlace ? 2 : 1);
+  // in (both grids of N = 1024 in 4x4x4 tiles: 2^32)
   const size_t most = (0xffffffffu / threads) & ~15u;   // whole rounds of the XCDs
   for (size_t b0 = 0; b0 < blocks; b0 += most)
     hipLaunchKernelGGL(k, dim3((unsigned)std::min(most, blocks - b0)), dim3(threads), lds, s, g,
