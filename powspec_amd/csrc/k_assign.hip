@@ -969,16 +969,18 @@ __device__ __forceinline__ void clear_cells(AT *lds, int cells) {
 //    gcd(S, ngroups) = 1 (a permutation): a wave's groups lie far apart in
 //    fill order, i.e. far apart in a space-ordered catalogue, so
 //    its lanes' windows rarely meet in one cell (record_group).
-//  - PCS, whose 64 cells leave no room for neighbours in a wave: a stretch of
-//    consecutive records per thread, the stretches of a wave's lanes far
-//    apart; a line's records are then read one after another by one lane.
-//    (Random order: whole waves of consecutive records, as above.)  Dense
-//    ordered catalogues, interlaced deposit of 3e7 particles at N = 256: pairs
-//    in the permuted order 2.27 ms, single records in it 1.84, stretches
-//    1.53; 8e6 at N = 128: 0.77, 0.46, 0.48.  For TSC the stretches gain at
-//    N = 128 (1.31 -> 1.20) and lose without interlacing (N = 256 0.59 ->
-//    0.71); NGP and CIC lose up to a factor of two.
-template <int SCHEME, class F>
+//  - More, with STRETCH (PCS, whose 64 cells leave no room for neighbours in a
+//    wave, and TSC in tiles of whole z rows): a stretch of consecutive records
+//    per thread, the stretches of a wave's lanes far apart; a line's records
+//    are then read one after another by one lane.  (Random order: whole waves
+//    of consecutive records, as above.)  Dense ordered catalogues, interlaced:
+//    PCS, 3e7 particles at N = 256, pairs in the permuted order 2.27 ms, single
+//    records in it 1.84, stretches 1.53; 8e6 at N = 128 0.77, 0.46, 0.48; TSC
+//    in whole z rows, with their transform, 1e8 at N = 256 pairs 7.8 ms,
+//    stretches 5.6.  In the default tiles TSC gains at N = 128 (3e7 particles
+//    1.31 -> 1.20) and loses without interlacing (N = 256 0.59 -> 0.71); NGP
+//    and CIC lose up to a factor of two.
+template <bool STRETCH, class F>
 __device__ __forceinline__ void for_records(const Rec *__restrict__ recs, uint32_t cnt, uint32_t gs,
                                             F visit) {
   const uint32_t t = threadIdx.x, B = blockDim.x;
@@ -992,7 +994,7 @@ __device__ __forceinline__ void for_records(const Rec *__restrict__ recs, uint32
     if (live) visit(r);
     return;
   }
-  if constexpr (SCHEME == 3) {
+  if constexpr (STRETCH) {
     // n records per thread, one more for the first `rest` threads (whole
     // waves); stretch l nw + w belongs to lane l of wave w
     const uint32_t q = cnt / B, rest = cnt - q * B, n = q + (t < rest);
@@ -1058,17 +1060,17 @@ __device__ __forceinline__ void for_records(const Rec *__restrict__ recs, uint32
 // log2 of the records a wave reads from consecutive places of a bucket:
 // larger groups use more of the 128-byte lines they touch, smaller ones keep
 // the windows of a space-ordered catalogue's neighbours apart.  Ordered:
-// 1 for PCS (for_records), 2 records for TSC (N = 256, 32 mocks: 1.71, 1.69,
+// 1 with stretches (for_records), 2 records for TSC (N = 256, 32 mocks: 1.71, 1.69,
 // 1.76 ms for 1, 2, 4), 4 for NGP and CIC (N = 512, 2e7 particles: 301, 269, 247 us).
 // A bucket filled in ranges of a few records (fewer than 16 on average, from
 // the count pass's number of ranges) is in random order, where neighbours are
 // no closer than others: a whole wave's (survey, N = 512, 1e8 randoms:
 // 2.12 ms with 4, 1.82 with 64).
-template <int SCHEME>
+template <int SCHEME, bool STRETCH>
 __device__ __forceinline__ uint32_t record_group(const uint32_t *starts, uint32_t ntiles,
                                                  const int *flags) {
   const bool random = starts[ntiles] / 16 < (uint32_t)flags[2];
-  return random ? 6u : SCHEME == 3 ? 0u : SCHEME == 2 ? 1u : 2u;
+  return random ? 6u : STRETCH ? 0u : SCHEME >= 2 ? 1u : 2u;
 }
 
 // One record's window on the plain or the shifted grid of a tile.
@@ -1154,7 +1156,9 @@ assign_deposit(PshAssignGeom g, const uint32_t *__restrict__ starts,
   const DepTile d = dep_tile(g, tile);
   const bool wrap = d.T[0] == g.Ng || d.T[1] == g.Ng || d.T[2] == g.Ng;
   clear_cells(lds - lead, cells);
-  for_records<SCHEME>(recs + k.s0, k.cnt, record_group<SCHEME>(starts, ntiles, flags), [&](const Rec &r) {
+  constexpr bool STRETCH = SCHEME == 3;
+  for_records<STRETCH>(recs + k.s0, k.cnt, record_group<SCHEME, STRETCH>(starts, ntiles, flags),
+                       [&](const Rec &r) {
     deposit_rec<SCHEME, WIDE>(lds, d, g, P2, wrap, shifted, r, k.scale);
   });
   __syncthreads();
@@ -1206,7 +1210,9 @@ assign_deposit_z(PshAssignGeom g, const uint32_t *__restrict__ starts,
   const int mock = d.mock;
   const float inv = k.inv;
   clear_cells(ldsq, gcells * (INTLACE ? 2 : 1));
-  for_records<SCHEME>(recs + k.s0, k.cnt, record_group<SCHEME>(starts, gridDim.x, flags), [&](const Rec &r) {
+  constexpr bool STRETCH = SCHEME >= 2;
+  for_records<STRETCH>(recs + k.s0, k.cnt, record_group<SCHEME, STRETCH>(starts, gridDim.x, flags),
+                       [&](const Rec &r) {
     deposit_rec<SCHEME, WIDE>(ldsA, d, g, P2, wrap, false, r, k.scale);
     if (INTLACE) deposit_rec<SCHEME, WIDE>(ldsB, d, g, P2, wrap, true, r, k.scale);
   });
