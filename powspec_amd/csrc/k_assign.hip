@@ -970,7 +970,7 @@ __device__ __forceinline__ void clear_cells(AT *lds, int cells) {
 //    fill order, i.e. far apart in a space-ordered catalogue, so
 //    its lanes' windows rarely meet in one cell (record_group).
 //  - More, with STRETCH (PCS, whose 64 cells leave no room for neighbours in a
-//    wave, and TSC in tiles of whole z rows): a stretch of consecutive records
+//    wave, and TSC with both grids in a workgroup): a stretch of consecutive records
 //    per thread, the stretches of a wave's lanes far apart; a line's records
 //    are then read one after another by one lane.  (Random order: whole waves
 //    of consecutive records, as above.)  Dense ordered catalogues, interlaced:
@@ -1117,57 +1117,13 @@ __device__ __forceinline__ DepBucket dep_bucket(const uint32_t *starts, uint32_t
   return k;
 }
 
-// Deposit of one grid (plain, or with INTLACE every second group of 8
-// workgroups the shifted one) of one tile per workgroup.  Bound: the LDS
-// atomics of the windows and the stores of the mesh; their phases alternate
-// within a workgroup, so it is other workgroups of the CU that overlap them.
-// One grid per workgroup halves the LDS tile: 4 workgroups of 512 threads per
-// CU instead of 2 for 32-bit cells, 2 instead of 1 for the survey's 64-bit
-// cells, for a second read of the records (the two grids of a tile follow
-// one another on one XCD: workgroups are dealt to the XCDs in turn).
-// Measured on MI355X (with the records' local cells, the next record in
-// flight and 16-byte LDS reads): N = 1024 PCS, 2e7 particles 2.72 -> 2.34 ms,
-// 8.6 GB of mesh at 3.7 TB/s; the survey's 64-bit CIC, N = 512, 1.5e8 records
-// 2.81 -> 1.64 ms; N = 512 CIC, 2e7 particles 0.31 -> 0.25 ms.
-template <int SCHEME, bool INTLACE, bool WIDE, bool NT>
-__global__ void __launch_bounds__(1024)
-assign_deposit(PshAssignGeom g, const uint32_t *__restrict__ starts,
-               const Rec *__restrict__ recs, size_t rec_cap,
-               float *__restrict__ meshA, float *__restrict__ meshB,
-               size_t mstride, const int *__restrict__ flags, int P2, int lead, int cells,
-               uint32_t ntiles, uint32_t b0) {
-  using AT = typename Acc<WIDE>::T;
-  extern __shared__ __align__(16) long long ldsraw[];
-  AT *lds = reinterpret_cast<AT *>(ldsraw) + lead;
-  const uint32_t b = blockIdx.x + b0;
-  uint32_t tile = b;
-  bool shifted = false;
-  if (INTLACE) {
-    // blocks 16 n + (0..7) and 16 n + 8 + (0..7): the grids of tiles 8 n + (0..7)
-    if (ntiles & 7) {
-      shifted = b & 1;
-      tile = b >> 1;
-    } else {
-      shifted = (b >> 3) & 1;
-      tile = (b >> 4) * 8 + (b & 7);
-    }
-  }
-  const DepBucket k = dep_bucket<Acc<WIDE>::TOP>(starts, tile, rec_cap, flags);
-  const DepTile d = dep_tile(g, tile);
-  const bool wrap = d.T[0] == g.Ng || d.T[1] == g.Ng || d.T[2] == g.Ng;
-  clear_cells(lds - lead, cells);
-  constexpr bool STRETCH = SCHEME == 3;
-  for_records<STRETCH>(recs + k.s0, k.cnt, record_group<SCHEME, STRETCH>(starts, ntiles, flags),
-                       [&](const Rec &r) {
-    deposit_rec<SCHEME, WIDE>(lds, d, g, P2, wrap, shifted, r, k.scale);
-  });
-  __syncthreads();
-
-  // write the tile: rows of T[2] floats along z, 4 cells per thread
+// A grid's tile to its mesh: rows of T[2] floats along z, 4 cells per thread.
+template <int SCHEME, bool NT, class AT>
+__device__ __forceinline__ void write_tile(const AT *lds, const DepTile &d, const PshAssignGeom &g,
+                                           int P2, int lead, float inv, float *out) {
   const int nrow = d.T[0] * d.T[1];
   const int q4s = g.tile_shift[2] - 2;   // T[2] = 4 * 2^q4s (T[2] >= 4)
   const int q4 = 1 << q4s;
-  float *out = (shifted ? meshB : meshA) + (size_t)d.mock * mstride;
   for (int i = threadIdx.x; i < nrow * q4; i += blockDim.x) {
     const int row = i >> q4s, q = i & (q4 - 1);
     const int lx = row >> g.tile_shift[1], ly = row & (d.T[1] - 1);
@@ -1183,10 +1139,65 @@ assign_deposit(PshAssignGeom g, const uint32_t *__restrict__ starts,
 #pragma unroll
       for (int h = 0; h < 4; h++) c[h] = lds[li + h];
     }
-    const float4 v = make_float4((float)c[0] * k.inv, (float)c[1] * k.inv, (float)c[2] * k.inv,
-                                 (float)c[3] * k.inv);
+    const float4 v = make_float4((float)c[0] * inv, (float)c[1] * inv, (float)c[2] * inv,
+                                 (float)c[3] * inv);
     store4<NT>(out + gidx, v);
   }
+}
+
+// Deposit of one grid (plain, or with INTLACE every second group of 8
+// workgroups the shifted one) of one tile per workgroup.  Bound: the LDS
+// atomics of the windows and the stores of the mesh; their phases alternate
+// within a workgroup, so it is other workgroups of the CU that overlap them.
+// One grid per workgroup halves the LDS tile: 4 workgroups of 512 threads per
+// CU instead of 2 for 32-bit cells, 2 instead of 1 for the survey's 64-bit
+// cells, for a second read of the records (the two grids of a tile follow
+// one another on one XCD: workgroups are dealt to the XCDs in turn).
+// Measured on MI355X (with the records' local cells, the next record in
+// flight and 16-byte LDS reads): N = 1024 PCS, 2e7 particles 2.72 -> 2.34 ms,
+// 8.6 GB of mesh at 3.7 TB/s; the survey's 64-bit CIC, N = 512, 1.5e8 records
+// 2.81 -> 1.64 ms; N = 512 CIC, 2e7 particles 0.31 -> 0.25 ms.
+// BOTH: both grids of the tile in one workgroup, for catalogues whose second
+// read costs more than that (launch_deposit).
+template <int SCHEME, bool INTLACE, bool WIDE, bool NT, bool BOTH = false>
+__global__ void __launch_bounds__(1024)
+assign_deposit(PshAssignGeom g, const uint32_t *__restrict__ starts,
+               const Rec *__restrict__ recs, size_t rec_cap,
+               float *__restrict__ meshA, float *__restrict__ meshB,
+               size_t mstride, const int *__restrict__ flags, int P2, int lead, int cells,
+               uint32_t ntiles, uint32_t b0) {
+  using AT = typename Acc<WIDE>::T;
+  extern __shared__ __align__(16) long long ldsraw[];
+  AT *lds = reinterpret_cast<AT *>(ldsraw) + lead;
+  const uint32_t b = blockIdx.x + b0;
+  uint32_t tile = b;
+  bool shifted = false;
+  if (INTLACE && !BOTH) {
+    // blocks 16 n + (0..7) and 16 n + 8 + (0..7): the grids of tiles 8 n + (0..7)
+    if (ntiles & 7) {
+      shifted = b & 1;
+      tile = b >> 1;
+    } else {
+      shifted = (b >> 3) & 1;
+      tile = (b >> 4) * 8 + (b & 7);
+    }
+  }
+  const DepBucket k = dep_bucket<Acc<WIDE>::TOP>(starts, tile, rec_cap, flags);
+  const DepTile d = dep_tile(g, tile);
+  const bool wrap = d.T[0] == g.Ng || d.T[1] == g.Ng || d.T[2] == g.Ng;
+  clear_cells(lds - lead, BOTH ? 2 * cells : cells);
+  constexpr bool STRETCH = SCHEME == 3 || BOTH;
+  for_records<STRETCH>(recs + k.s0, k.cnt, record_group<SCHEME, STRETCH>(starts, ntiles, flags),
+                       [&](const Rec &r) {
+    deposit_rec<SCHEME, WIDE>(lds, d, g, P2, wrap, shifted, r, k.scale);
+    if (BOTH) deposit_rec<SCHEME, WIDE>(lds + cells, d, g, P2, wrap, true, r, k.scale);
+  });
+  __syncthreads();
+
+  write_tile<SCHEME, NT>(lds, d, g, P2, lead, k.inv,
+                         (shifted ? meshB : meshA) + (size_t)d.mock * mstride);
+  if (BOTH)
+    write_tile<SCHEME, NT>(lds + cells, d, g, P2, lead, k.inv, meshB + (size_t)d.mock * mstride);
 }
 
 // Deposit of both grids of a tile of whole z rows, transformed along z.
@@ -1277,7 +1288,7 @@ assign_deposit_z(PshAssignGeom g, const uint32_t *__restrict__ starts,
 }
 
 template <int SCHEME>
-hipError_t launch_deposit(const PshAssignGeom &g, size_t ntiles,
+hipError_t launch_deposit(const PshAssignGeom &g, size_t ntiles, size_t ntotal,
                           const uint32_t *starts, const Rec *recs,
                           size_t rec_cap, float *meshA, float *meshB,
                           size_t mstride, const int *flags, hipStream_t s) {
@@ -1296,7 +1307,7 @@ hipError_t launch_deposit(const PshAssignGeom &g, size_t ntiles,
     lead = (4 - W % 4) % 4;
     cells = quads;
   }
-  const size_t lds = cell * cells;
+  size_t lds = cell * cells;
   // non-temporal mesh stores when the launch's meshes outgrow the 256 MB
   // Infinity Cache (every cell is written once and read by the next pass
   // only after the whole launch)
@@ -1342,6 +1353,22 @@ hipError_t launch_deposit(const PshAssignGeom &g, size_t ntiles,
                                          : assign_deposit<SCHEME, false, true, false>)
                             : (g.intlace ? assign_deposit<SCHEME, true, false, false>
                                          : assign_deposit<SCHEME, false, false, false>));
+  // TSC in a launch of many tiles with 0.3 particles per cell and more: records
+  // read once for both grids (deposit, one / both: N = 512, 1e8 particles in
+  // space order 3.25 / 2.57 ms, shuffled 2.26 / 2.39; N = 640 2.84 / 2.65,
+  // 2.24 / 2.39).  Fewer tiles leave the chip idle (N = 64 1.06 / 1.57) or
+  // keep more of the second read in the caches (N = 256, 8e6 shuffled
+  // 0.19 / 0.21); the other schemes are faster with one grid, or equal.
+  bool both = false;
+  if constexpr (SCHEME == 2) {
+    both = g.intlace && !g.wide && ntiles >= 8192 && 2 * lds <= 160 * 1024 &&
+           10 * ntotal >= 3 * ntiles * g.tile[0] * g.tile[1] * g.tile[2];
+    if (both) {
+      k = stream ? assign_deposit<2, true, false, true, true>
+                 : assign_deposit<2, true, false, false, true>;
+      lds *= 2;
+    }
+  }
   raise((const void *)k);
   // one thread per 16 cells (per 8 of 64 bits, whose LDS admits half the
   // workgroups: survey, N = 512, 1.89 -> 1.64 ms), 256..1024.  Two waves for
@@ -1352,7 +1379,7 @@ hipError_t launch_deposit(const PshAssignGeom &g, size_t ntiles,
   // 0.20 / 0.29 / 0.19, PCS 2e6 0.38 / 0.41 / 0.27; few tiles with many
   // records each want the waves: N = 64 in 4x4x64 PCS 2e6 0.41 / 0.23 / 0.44.
   const size_t tcells = (size_t)g.tile[0] * g.tile[1] * g.tile[2];
-  const size_t blocks = ntiles * (g.intlace ? 2 : 1);
+  const size_t blocks = ntiles * (g.intlace && !both ? 2 : 1);
   const size_t per = g.wide ? 8 : 16;
   unsigned threads = tcells < 2048 && blocks >= 8192 ? 128 : 256;
   while (threads < 1024 && threads * per < tcells) threads *= 2;
@@ -1484,9 +1511,9 @@ hipError_t psh_assign_run(const PshAssignGeom &g, PshDevPart *d_parts, const Psh
   if ((e = bucket(true)) != hipSuccess) return e;
   if (ev_deposit) (void)hipEventRecord(ev_deposit, s);
   switch (g.scheme) {
-    case 0: return launch_deposit<0>(g, ntiles, starts, recs, rec_cap, meshA, meshB, mstride, d_flags, s);
-    case 1: return launch_deposit<1>(g, ntiles, starts, recs, rec_cap, meshA, meshB, mstride, d_flags, s);
-    case 2: return launch_deposit<2>(g, ntiles, starts, recs, rec_cap, meshA, meshB, mstride, d_flags, s);
-    default: return launch_deposit<3>(g, ntiles, starts, recs, rec_cap, meshA, meshB, mstride, d_flags, s);
+    case 0: return launch_deposit<0>(g, ntiles, ntotal, starts, recs, rec_cap, meshA, meshB, mstride, d_flags, s);
+    case 1: return launch_deposit<1>(g, ntiles, ntotal, starts, recs, rec_cap, meshA, meshB, mstride, d_flags, s);
+    case 2: return launch_deposit<2>(g, ntiles, ntotal, starts, recs, rec_cap, meshA, meshB, mstride, d_flags, s);
+    default: return launch_deposit<3>(g, ntiles, ntotal, starts, recs, rec_cap, meshA, meshB, mstride, d_flags, s);
   }
 }
