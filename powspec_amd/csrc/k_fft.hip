@@ -571,8 +571,9 @@ struct XCfg {
   static constexpr int WAVES = SMALL ? 2 : 4;
   // the next tile's rows loaded during phase 2 (see x_bin_kernel).  Where the
   // interlaced kernel holds 16 values per thread and field (N = 1024,
-  // 2048) the rows in flight spill; measured on MI355X with / without:
-  // N = 1024 3.14 / 3.02 ms, N = 768 1.46 / 1.56 ms, N = 640 1.33 / 1.47 ms.
+  // 2048) the rows in flight spill and nothing is gained; measured on MI355X,
+  // poles 0, 2, 4, with / without: N = 1024 2.97 / 3.02 ms, N = 768
+  // 1.43 / 1.62, N = 640 0.88 / 0.98, with log bins and poles 0..4 1.02 / 1.23.
   static constexpr bool PREFETCH = !(IL && !SMALL && C * N >= 16 * T);
   static_assert(T % C == 0, "a thread keeps one column");
 };
@@ -642,14 +643,15 @@ __device__ __forceinline__ int bin_exact(const PshBins &b, double ksqx, double k
 }
 
 // What bounds it: up to N = 640 the row reads, from N = 768 on the transforms'
-// LDS exchanges and instructions as well (N = 1024, interlaced, 5.2 GB of live
+// LDS exchanges and instructions as well (N = 1024, interlaced, 6.9 GB of live
 // rows: 1.4 ms without the transforms and the binning, the transforms add
 // 1.2 ms, the binning 0.4).  Rows prefetched through the whole of phase 2
 // (nothing in it waits on memory: tables from LDS or scalar loads, no select
-// on a loaded value) and binning without address arithmetic or FP64 took,
-// on MI355X, start of the tuning -> now: plain 256^3 47 -> 33 us, interlaced
-// 640^3 log bins 1.72 -> 1.20 ms, 1024^3 3.40 -> 3.02 ms, 32 interlaced 256^3
-// 1.31 -> 1.14 ms, alias-corrected 512^3 with |mu| cells 343 -> 257 us.
+// on a loaded value), binning without address arithmetic or FP64 and, for log
+// bins, tiles past the last edge left out took, on MI355X, before -> now: plain
+// 256^3 51 -> 36 us, interlaced 640^3 log bins, poles 0..4, 1.72 -> 1.02 ms,
+// 1024^3 3.38 -> 3.02 ms, 32 interlaced 256^3 1.33 -> 1.17 ms, alias-corrected
+// 512^3 with |mu| cells 348 -> 249 us.
 //
 // Forward x transform of one (y, kz-tile) column tile fused with the
 // interlace combine and the binning of its modes.  Two phases per tile:
@@ -1109,8 +1111,8 @@ x_bin_kernel(XBinDev a, int ntz, int H, const float2 *__restrict__ tw) {
           }
           return;
         }
-        // poles above 4: a rolled loop (for any poles, as it was before, the
-        // interlaced 640^3 pass with poles 0..4 took 1.33 ms, now 1.20)
+        // poles above 4: a rolled loop (for any poles, the interlaced 640^3 pass
+        // with poles 0..4 over every tile took 1.33 ms, with the above 1.20)
         const int lmask = single ? ~0 : ~a.oddmask;
 #pragma unroll 1
         for (int l = 0; l < b.nl; l++) {
