@@ -142,26 +142,18 @@ def measured_traffic(kernel):
 
 
 def roofline(stages, Ng, nmesh, npart, x_live=1.0):
+    """Every stage is one launch for both meshes (plain and shifted grid)."""
     b = stage_bytes(Ng, nmesh, npart, x_live)
     cands = {k: stages[k] for k in ("deposit", "z_r2c", "y_fft", "x_fft_bin")}
     dom = max(cands, key=lambda k: cands[k])
-    per_launch = b[dom]
-    # z and y cover both meshes (plain and shifted grid) in one launch, like the
-    # deposit and the fused x pass; their figures are given per mesh
-    launches = nmesh if dom in ("z_r2c", "y_fft") else 1
-    t = stages[dom] / launches
-    ach = per_launch / launches / (t * 1e-3) / 1e9
-    table = {}
-    for k in cands:
-        nl = nmesh if k in ("z_r2c", "y_fft") else 1
-        if stages[k] > 0:
-            table[k] = {"ms": round(stages[k], 4),
-                        "GBps": round(b[k] / (stages[k] * 1e-3) / 1e9, 1),
-                        "launches": nl}
+    ach = b[dom] / (stages[dom] * 1e-3) / 1e9
+    table = {k: {"ms": round(stages[k], 4),
+                 "GBps": round(b[k] / (stages[k] * 1e-3) / 1e9, 1), "launches": 1}
+             for k in cands if stages[k] > 0}
     return {"kernel": KERNELS[dom], "bound": "hbm", "achieved": round(ach, 1),
             "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(ach / HBM_PEAK_GBS, 4),
             "traffic": measured_traffic(KERNELS[dom]),
-            "bytes_per_launch": per_launch / launches, "ms_per_launch": round(t, 4),
+            "bytes_per_launch": b[dom], "ms_per_launch": round(stages[dom], 4),
             "stages": table}
 
 
